@@ -114,7 +114,7 @@ __device__ __forceinline__ StageArgs<R> slot_args(const SlotDesc<R>* sd) {
     StageArgs<R> a;
     Ctrl* ctrl = uni(sd->ctrl);
     a.ctrl = ctrl;
-    a.lam_bits = &ctrl->lam_bits;
+    a.lam_bits = lam_slots(ctrl);
     a.geo_e = uni(sd->geo_e);
     a.geo_f = uni(sd->geo_f);
     a.nbr = uni(sd->nbr);
@@ -334,7 +334,7 @@ const void* batch_stage_fn(int kind, int mask) {
 
 template <typename R>
 __global__ void k_batch_dt(const SlotDesc<R>* __restrict__ slots, const int* __restrict__ nslots) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    const int s = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);  // one wavefront per slot
     if (s < *nslots) dt_update(slots[s].ctrl);
 }
 
@@ -470,7 +470,7 @@ class EngineT : public BatchEngine {
             HIPST(hipMalloc((void**)&d_slots, cap_slots * sizeof(SlotDesc<R>)));
             HIPST(hipMalloc((void**)&d_status, cap_slots * 3 * sizeof(double)));
             HIPST(hipMalloc((void**)&d_ctrls, cap_slots * sizeof(Ctrl)));
-            dt_grid = (cap_slots + 63) / 64;
+            dt_grid = (cap_slots + 3) / 4;
             drop_graph();
         }
         if (ni > cap_items) {
@@ -655,7 +655,7 @@ class EngineT : public BatchEngine {
     }
 
     Status step_direct() {
-        hipLaunchKernelGGL((k_batch_dt<R>), dim3(dt_grid), dim3(64), 0, st, d_slots, d_xcd + BATCH_NSLOT_AT);
+        hipLaunchKernelGGL((k_batch_dt<R>), dim3(dt_grid), dim3(256), 0, st, d_slots, d_xcd + BATCH_NSLOT_AT);
         HIPST(hipGetLastError());
         Status s0;
         for (int k : {ST_RK4_1, ST_RK4_2, ST_RK4_3, ST_RK4_4}) {

@@ -82,40 +82,69 @@ struct Ctrl {
     double min_r;    // minimum inscribed-circle diameter of the mesh
     double two_p1;   // 2p + 1
     int64_t steps;   // steps taken
-    // maximum cell wave speed of the current state, as the bit pattern of a
-    // non-negative double (ordered like the value), accumulated with one
-    // atomic max per workgroup; reset by the dt kernel after it is read
-    unsigned long long lam_bits;
+    unsigned long long lam_bits;  // maximum cell wave speed the current step's dt was taken from
     int active;      // the stages of the current step run
     int done;        // t reached t_end
     int has_end;     // clamp to t_end
     int pad;
 };
 
-__device__ __forceinline__ void lam_commit(double mx, unsigned long long* bits) {
-    if (mx > 0.0) atomicMax(bits, (unsigned long long)__double_as_longlong(mx));
+// Maximum cell wave speed of the current state: LAM_SLOTS partial maxima
+// behind the control block, each the bit pattern of a non-negative double
+// (ordered like the value) on a line of its own.  A workgroup commits with
+// one atomic max to the slot of its number; the dt kernel reduces the slots
+// and clears them.  One address for all workgroups made the last stage wait
+// for its atomics, which the memory takes one after another (about 35 ns
+// each: 4,096 workgroups of the lane kernel, Euler p = 1 at 524,288
+// triangles, a step of 4 stages 167 us; with 64 slots 133 us).
+constexpr int LAM_SLOTS = 64;
+constexpr int LAM_STRIDE = 8;     // 64 bytes apart
+constexpr size_t CTRL_LAM_AT = 256;  // byte offset of the slots behind a solve's control block
+constexpr size_t CTRL_BYTES = CTRL_LAM_AT + LAM_SLOTS * LAM_STRIDE * sizeof(unsigned long long);
+static_assert(sizeof(Ctrl) <= CTRL_LAM_AT, "the wave-speed slots follow the control block");
+
+__host__ __device__ inline unsigned long long* lam_slots(Ctrl* ctrl) {
+    return reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(ctrl) + CTRL_LAM_AT);
+}
+
+__device__ __forceinline__ void lam_commit(double mx, unsigned long long* slots) {
+    if (mx > 0.0)
+        atomicMax(slots + (blockIdx.x & (LAM_SLOTS - 1)) * LAM_STRIDE, (unsigned long long)__double_as_longlong(mx));
+}
+
+// The maximum over the slots (every lane of one wavefront calls it).
+__device__ __forceinline__ double lam_reduce(const unsigned long long* slots) {
+    double v = __longlong_as_double((long long)slots[(threadIdx.x & (LAM_SLOTS - 1)) * LAM_STRIDE]);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
+    return v;
 }
 
 // Start of a step on the device: dt = cfl * min_r / max lambda / (2p+1),
 // clamped to t_end, t advanced before the stages (time_integrator.cu:254-270);
-// reads the accumulated maximum wave speed and clears it for the step's last
-// stage to fill.  A step not taken (t_end reached) leaves it: it still holds
-// the wave speed of the current state, which a later run starts from.  One
-// thread.
+// reduces the accumulated wave speeds and clears them for the step's last
+// stage to fill.  A step not taken (t_end reached) leaves them: they still
+// hold the wave speed of the current state, which a later run starts from.
+// One wavefront.
 __device__ __forceinline__ void dt_update(Ctrl* ctrl) {
+    const bool first = (threadIdx.x & 63) == 0;
     if (ctrl->done) {
-        ctrl->active = 0;
+        if (first) ctrl->active = 0;
         return;
     }
     double t = ctrl->t;
     if (ctrl->has_end && !(t < ctrl->t_end)) {
-        ctrl->active = 0;
-        ctrl->done = 1;
-        ctrl->dt = 0.0;
+        if (first) {
+            ctrl->active = 0;
+            ctrl->done = 1;
+            ctrl->dt = 0.0;
+        }
         return;
     }
-    const double mx = __longlong_as_double((long long)ctrl->lam_bits);
-    ctrl->lam_bits = 0ull;
+    unsigned long long* slots = lam_slots(ctrl);
+    const double mx = lam_reduce(slots);
+    slots[(threadIdx.x & (LAM_SLOTS - 1)) * LAM_STRIDE] = 0ull;
+    if (!first) return;
     double dt = ctrl->cfl * ctrl->min_r / mx / ctrl->two_p1;
     if (ctrl->has_end && t + dt > ctrl->t_end) {
         dt = ctrl->t_end - t;
@@ -123,6 +152,7 @@ __device__ __forceinline__ void dt_update(Ctrl* ctrl) {
     } else {
         t += dt;
     }
+    ctrl->lam_bits = (unsigned long long)__double_as_longlong(mx);
     ctrl->dt = dt;
     ctrl->t = t;
     ctrl->steps += 1;
@@ -266,7 +296,7 @@ struct StageArgs {
     const R* geo_f;   // [9][Kp]: (nx, ny, len) for faces 0..2
     const int* nbr;   // [3][Kp]
     const Ctrl* ctrl;
-    unsigned long long* lam_bits; // &ctrl->lam_bits (last stage)
+    unsigned long long* lam_bits; // lam_slots(ctrl) (last stage)
     int K, Kp;        // elements, and the padded count (multiple of 64) of every [..][Kp] array
     int kind;
     int ntiles;       // tiles (workgroups) that carry elements

@@ -134,7 +134,7 @@ hipError_t mfma_layout_probe(float* host_out);
 hipError_t mfma_layout_probe_f64(double* host_out);
 constexpr int VALU_TILE_ELEMS = 128;
 
-// resets ctrl->lam_bits and accumulates the state's maximum cell wave speed into it
+// resets the solve's wave-speed slots and accumulates the state's maximum cell wave speed into them
 template <typename R>
 hipError_t launch_lambda(const R* u, const StateIx& ix, int K, double b0, const PhysP& ph, Ctrl* ctrl,
                          hipStream_t st);

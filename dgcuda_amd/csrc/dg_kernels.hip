@@ -54,21 +54,21 @@ __global__ void __launch_bounds__(256) k_lambda(const R* u, StateIx ix, int K, d
 }
 
 __global__ void k_reset_lam(Ctrl* ctrl) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) ctrl->lam_bits = 0ull;
+    lam_slots(ctrl)[threadIdx.x * LAM_STRIDE] = 0ull;  // LAM_SLOTS threads
 }
 
 // dt = cfl * min_r / max lambda / (2p+1), clamped to t_end
 // (time_integrator.cu:254-270); reads and clears the accumulated maximum.
 __global__ void k_dt(Ctrl* ctrl) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) dt_update(ctrl);
+    dt_update(ctrl);  // one wavefront
 }
 
 // host-chosen step: activate the stages with the given dt
 __global__ void k_set_dt(Ctrl* ctrl, double dt, int advance) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
+    lam_slots(ctrl)[threadIdx.x * LAM_STRIDE] = 0ull;  // LAM_SLOTS threads
+    if (threadIdx.x == 0) {
         ctrl->dt = dt;
         ctrl->active = 1;
-        ctrl->lam_bits = 0ull;
         if (advance) {
             ctrl->t += dt;
             ctrl->steps += 1;
@@ -195,9 +195,9 @@ template hipError_t launch_stage_valu<double>(int, int, const StageArgs<double>&
 template <typename R>
 hipError_t launch_lambda(const R* u, const StateIx& ix, int K, double b0, const PhysP& ph, Ctrl* ctrl,
                          hipStream_t st) {
-    hipLaunchKernelGGL(k_reset_lam, dim3(1), dim3(64), 0, st, ctrl);
+    hipLaunchKernelGGL(k_reset_lam, dim3(1), dim3(LAM_SLOTS), 0, st, ctrl);
     const dim3 grid(std::min((K + 255) / 256, 2048));
-    unsigned long long* bits = &ctrl->lam_bits;
+    unsigned long long* bits = lam_slots(ctrl);
     if (ix.N == 1)
         hipLaunchKernelGGL((k_lambda<1, R>), grid, dim3(256), 0, st, u, ix, K, b0, ph, bits);
     else
@@ -215,7 +215,7 @@ hipError_t launch_dt(Ctrl* ctrl, hipStream_t st) {
 }
 
 hipError_t launch_set_dt(Ctrl* ctrl, double dt, int advance, hipStream_t st) {
-    hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(64), 0, st, ctrl, dt, advance);
+    hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(LAM_SLOTS), 0, st, ctrl, dt, advance);
     return hipGetLastError();
 }
 

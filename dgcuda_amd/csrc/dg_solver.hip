@@ -390,7 +390,8 @@ class SolverT : public Solver {
         if (!(st = alloc((void**)&Jd, (size_t)Kp * sizeof(double)))) return st;
         audit_blocks = (K + 255) / 256;
         if (!(st = alloc((void**)&audit_part, (size_t)audit_blocks * 8 * sizeof(double)))) return st;
-        if (!(st = alloc((void**)&ctrl, sizeof(Ctrl)))) return st;
+        if (!(st = alloc((void**)&ctrl, CTRL_BYTES))) return st;
+        HIPST(hipMemsetAsync(ctrl, 0, CTRL_BYTES, stream));
         HIPST(hipMemsetAsync(c, 0, M * sizeof(R), stream));
         HIPST(hipMemsetAsync(acc, 0, M * sizeof(R), stream));
         HIPST(hipMemsetAsync(ua, 0, M * sizeof(R), stream));
@@ -670,7 +671,7 @@ class SolverT : public Solver {
         a.geo_f = geo_f;
         a.nbr = nbr;
         a.ctrl = ctrl;
-        a.lam_bits = &ctrl->lam_bits;
+        a.lam_bits = lam_slots(ctrl);
         a.K = K;
         a.Kp = Kp;
         a.kind = kind;
@@ -859,9 +860,10 @@ class SolverT : public Solver {
     Status cfl_dt(double cfl, double* dt) override {
         Status st = ensure_lambda();
         if (!st) return st;
-        unsigned long long bits = 0;
-        HIPST(hipMemcpyAsync(&bits, &ctrl->lam_bits, sizeof(bits), hipMemcpyDeviceToHost, stream));
+        unsigned long long slots[LAM_SLOTS * LAM_STRIDE], bits = 0;
+        HIPST(hipMemcpyAsync(slots, lam_slots(ctrl), sizeof(slots), hipMemcpyDeviceToHost, stream));
         HIPST(hipStreamSynchronize(stream));
+        for (int i = 0; i < LAM_SLOTS; i++) bits = std::max(bits, slots[i * LAM_STRIDE]);
         double mx;
         std::memcpy(&mx, &bits, sizeof(mx));
         *dt = cfl * min_r / mx / (2. * p + 1.);
