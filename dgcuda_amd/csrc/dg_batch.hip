@@ -22,6 +22,7 @@
 
 #include "dg_batch.h"
 #include "dg_worklist.h"
+#include "dg_lane_body.h"
 #include "dg_mfma_body.h"
 #include "dg_valu_body.h"
 
@@ -38,6 +39,8 @@ struct SlotDesc {
     const int* halo;
     const void* face4;
     const void* metric4;
+    const void* lface;
+    const void* lmetric;
     Ctrl* ctrl;
     int K, Kp, N, p, hcap, path;  // path 1 = lane per element, 2 = matrix-core tiles
     PhysP phys;
@@ -118,12 +121,14 @@ __device__ __forceinline__ StageArgs<R> slot_args(const SlotDesc<R>* sd) {
     a.geo_e = uni(sd->geo_e);
     a.geo_f = uni(sd->geo_f);
     a.nbr = uni(sd->nbr);
+    a.lface = uni(sd->lface);
+    a.lmetric = uni(sd->lmetric);
     a.K = uni(sd->K);
     a.Kp = uni(sd->Kp);
     a.kind = KIND;
     a.ntiles = 0;
     a.xcd_remap = 0;
-    a.pad = 0;
+    a.stream = 0;
     a.bnd = nullptr;  // batched solves have no boundary sides
     a.phys.gamma = uni(sd->phys.gamma);
     a.phys.ax = uni(sd->phys.ax);
@@ -192,6 +197,12 @@ __device__ __forceinline__ void batch_lane_items(const SlotDesc<R>* __restrict__
                                                  const int2* __restrict__ items, int it, int i1, int G8,
                                                  double* sh) {
     constexpr bool LAST = (KIND == ST_RK4_4 || KIND == ST_RK2_2);
+    __shared__ __align__(16) R lt1[EUL ? LaneTab<1>::SIZE : 4], lt2[EUL ? LaneTab<2>::SIZE : 4];
+    if constexpr (EUL) {
+        LaneTab<1>::fill(lt1, threadIdx.x, blockDim.x);
+        LaneTab<2>::fill(lt2, threadIdx.x, blockDim.x);
+        __syncthreads();
+    }
     for (; it < i1; it += G8) {
         const int2 item = items[it];
         const SlotDesc<R>* sd = slots + uni(item.x);
@@ -201,8 +212,10 @@ __device__ __forceinline__ void batch_lane_items(const SlotDesc<R>* __restrict__
         const int e = uni(item.y) * BATCH_VALU_TILE + threadIdx.x;
         double lam = 0.0;
         if constexpr (EUL) {
-            if (N == 4 && p == 2) lam = valu_process<4, 2, R>(a, e, KIND);
-            else if (N == 4 && p == 1) lam = valu_process<4, 1, R>(a, e, KIND);
+            // with the non-temporal hint: 1-2% faster per step than without
+            // on ragged batches of 24, 32 and 64 solves
+            if (N == 4 && p == 2) lam = lane_process<2, KIND, R, false, true>(a, e, lt2);
+            else if (N == 4 && p == 1) lam = lane_process<1, KIND, R, false, true>(a, e, lt1);
         }
         if constexpr (ADV) {
             if (N == 1 && p == 2) lam = valu_process<1, 2, R>(a, e, KIND);
@@ -580,6 +593,8 @@ class EngineT : public BatchEngine {
             d.halo = si.halo;
             d.face4 = si.face4;
             d.metric4 = si.metric4;
+            d.lface = si.lface;
+            d.lmetric = si.lmetric;
             d.ctrl = si.ctrl;
             d.K = si.K;
             d.Kp = si.Kp;

@@ -269,19 +269,31 @@ __device__ __forceinline__ R rk_update(R c, R aa, R k, R* acc_out) {
 //      ((e/16)*N + v)*256 + (m%4)*64 + (e%16)*4 + m/4.
 //    The wavefront's 64 lanes cover the block's variable contiguously.
 //    Modes >= NP are padding and hold zeros.
+//  * Vector layout of the Euler lane kernels up to p = 3: per mode, rows of
+//    16-byte pieces of one element's variables, so a lane moves its element's
+//    mode in one (FP32, tiled = 3: all 4 variables) or two (FP64, tiled = 4:
+//    2 variables each) accesses:
+//      FP32 (m*Kp + e)*4 + v;  FP64 ((m*2 + v/2)*Kp + e)*2 + v%2.
 constexpr int tile_groups(int NP) { return (NP + 3) / 4; }
+enum { LAYOUT_MODES = 0, LAYOUT_TILE32 = 1, LAYOUT_TILE64 = 2, LAYOUT_VEC32 = 3, LAYOUT_VEC64 = 4 };
 
 struct StateIx {
     int N, NP, Kp, tiled;
+    // mode slots stored per (variable, element): NP, or the tile layout's
+    __host__ __device__ int slots() const {
+        return tiled == LAYOUT_TILE32 ? 4 * tile_groups(NP) : tiled == LAYOUT_TILE64 ? 16 : NP;
+    }
     __host__ __device__ size_t at(int v, int m, int e) const {
         if (!tiled) return ((size_t)v * NP + m) * Kp + e;
+        if (tiled == LAYOUT_VEC32) return (((size_t)m * Kp + e) << 2) + v;
+        if (tiled == LAYOUT_VEC64) return ((((size_t)m * 2 + (v >> 1)) * Kp + e) << 1) + (v & 1);
         if (tiled == 2) return (((size_t)(e >> 4) * N + v) << 8) + (size_t)(((m & 3) << 6) + ((e & 15) << 2) + (m >> 2));
         const int G = tile_groups(NP);
         return ((((size_t)(e >> 4) * N + v) * G + (m >> 2)) << 6) + (size_t)((e & 15) << 2) + (m & 3);
     }
     // entries of one array: N*NP*Kp, or the tile layout's padded count
     __host__ __device__ size_t elems() const {
-        if (!tiled) return (size_t)N * NP * Kp;
+        if (!tiled || tiled >= LAYOUT_VEC32) return (size_t)N * NP * Kp;
         return (size_t)N * (tiled == 2 ? 16 : 4 * tile_groups(NP)) * Kp;
     }
 };
@@ -301,8 +313,13 @@ struct StageArgs {
     int kind;
     int ntiles;       // tiles (workgroups) that carry elements
     int xcd_remap;    // map consecutive tiles to one XCD
-    int pad;
+    int stream;       // vector layout: the solve's arrays exceed the memory-side cache
     PhysP phys;
+    // lane kernels in the vector layout: packed geometry, per face 4 values
+    // (nx, ny, len, neighbour word: FP32 its bits, FP64 its value) [3][Kp],
+    // per element 4 values (xr, yr, xs, ys) [Kp]
+    const void* lface;
+    const void* lmetric;
     // boundary sides, [side][point][4] FP64 (lane kernel only): the ghost
     // state of inflow / outflow points, the wall normal (Nx, Ny, 0, 0) of
     // reflecting points; null for a mesh without boundary sides

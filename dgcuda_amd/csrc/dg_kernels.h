@@ -91,6 +91,12 @@ hipError_t launch_stream_copy(const void* src, void* dst, int64_t bytes, hipStre
 
 template <typename R>
 hipError_t launch_stage_valu(int N, int p, const StageArgs<R>& a, dim3 grid, hipStream_t st);
+// packed geometry of the vector layout (StageArgs::lface, lmetric)
+template <typename R>
+hipError_t launch_lane_pack(const R* geo_e, const R* geo_f, const int* nbr, int Kp, void* lface, void* lmetric,
+                            hipStream_t st);
+// orders and physics whose lane kernel keeps its state in the vector layout
+__host__ __device__ constexpr bool lane_vec(int N, int p) { return N == 4 && p <= 3; }
 
 // Extra per-solve data of the matrix-core kernel: per (element, face) a
 // 32-bit word {bits 0..11 LDS slot of the neighbour (own tile element or

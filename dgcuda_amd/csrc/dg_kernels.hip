@@ -15,6 +15,7 @@
 //                      reduced per workgroup with wavefront shuffles.
 #include <algorithm>
 
+#include "dg_lane_body.h"
 #include "dg_valu_body.h"
 
 namespace dgmi {
@@ -35,6 +36,64 @@ __global__ void __launch_bounds__(128) k_stage_valu(StageArgs<R> a) {
         if (threadIdx.x == 0) lam_commit(mx, a.lam_bits);
     }
 }
+
+// Euler, p <= 3: the lane body on the vector layout, one instance per stage
+// kind (the RK operands' loads and the update are fixed at compile time)
+// Wavefronts per SIMD the registers are held to: the most that fit without
+// spills (FP32 p = 1, 2: 5 and 4; FP64 p = 1, 2: 2).
+template <int P, typename R>
+constexpr int lane_minw() {
+    if (sizeof(R) == 4) return P <= 1 ? 5 : P == 2 ? 4 : 2;
+    return P <= 2 ? 2 : 1;
+}
+template <int P, int KIND, typename R, bool BND, bool NT>
+__global__ void __launch_bounds__(128, (lane_minw<P, R>())) k_stage_lane(StageArgs<R> a) {
+    __shared__ double sh[8];
+    if (!a.ctrl->active) return;
+    const int tile = tile_of_block(blockIdx.x, gridDim.x, a.xcd_remap);
+    if (tile >= a.ntiles) return;
+    __shared__ __align__(16) R ltab[LaneTab<P>::SIZE];
+    LaneTab<P>::fill(ltab, threadIdx.x, blockDim.x);
+    __syncthreads();
+    const double lam = lane_process<P, KIND, R, BND, NT>(a, tile * blockDim.x + threadIdx.x, ltab);
+    if constexpr (KIND == ST_RK4_4 || KIND == ST_RK2_2) {
+        const double mx = block_max(lam, sh);
+        if (threadIdx.x == 0) lam_commit(mx, a.lam_bits);
+    }
+}
+
+// Packs the geometry of the vector layout (one thread per element).
+template <typename R>
+__global__ void __launch_bounds__(256) k_lane_pack(const R* __restrict__ geo_e, const R* __restrict__ geo_f,
+                                                  const int* __restrict__ nbr, int Kp,
+                                                  typename LaneV<R>::G* __restrict__ lface,
+                                                  typename LaneV<R>::G* __restrict__ lmetric) {
+    using G4 = typename LaneV<R>::G;
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= Kp) return;
+    const size_t kp = (size_t)Kp;
+    for (int f = 0; f < 3; f++) {
+        const int wd = nbr[f * kp + e];
+        R wv;
+        if constexpr (sizeof(R) == 4)
+            wv = __int_as_float(wd);
+        else
+            wv = (R)wd;
+        lface[f * kp + e] = G4{geo_f[3 * f * kp + e], geo_f[(3 * f + 1) * kp + e], geo_f[(3 * f + 2) * kp + e], wv};
+    }
+    lmetric[e] = G4{geo_e[e], geo_e[kp + e], geo_e[2 * kp + e], geo_e[3 * kp + e]};
+}
+
+template <typename R>
+hipError_t launch_lane_pack(const R* geo_e, const R* geo_f, const int* nbr, int Kp, void* lface, void* lmetric,
+                            hipStream_t st) {
+    using G4 = typename LaneV<R>::G;
+    hipLaunchKernelGGL((k_lane_pack<R>), dim3((Kp + 255) / 256), dim3(256), 0, st, geo_e, geo_f, nbr, Kp, (G4*)lface,
+                       (G4*)lmetric);
+    return hipGetLastError();
+}
+template hipError_t launch_lane_pack<float>(const float*, const float*, const int*, int, void*, void*, hipStream_t);
+template hipError_t launch_lane_pack<double>(const double*, const double*, const int*, int, void*, void*, hipStream_t);
 
 // Maximum cell wave speed of a state without stepping it (first step of a
 // run, dg_cfl_dt): grid-stride over elements, workgroup max, one atomic max.
@@ -105,9 +164,8 @@ __global__ void __launch_bounds__(128) k_project_ic(R* c, StateIx ix, const doub
             for (int n = 0; n < N; n++) U[n] += T.W[j] * u0[j][n] * T.B[i][j];
         for (int n = 0; n < N; n++) c[ix.at(n, i, e)] = (R)U[n];
     }
-    if (ix.tiled)  // padding modes of the last group
-        for (int i = NP; i < 4 * tile_groups(NP); i++)
-            for (int n = 0; n < N; n++) c[ix.at(n, i, e)] = R(0);
+    for (int i = NP; i < ix.slots(); i++)  // padding modes of the tile layouts
+        for (int n = 0; n < N; n++) c[ix.at(n, i, e)] = R(0);
 }
 
 // ---------------------------------------------------------------------------
@@ -158,35 +216,71 @@ __global__ void __launch_bounds__(256) k_audit(const R* c, StateIx ix, const dou
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-template <int N, typename R>
-static hipError_t launch_stage_valu_np(int p, const StageArgs<R>& a, dim3 grid, hipStream_t st) {
-    if (a.bnd) {
-        static_assert(VALU_BOUNDARY_MAX_P == 3, "boundary instantiations below are p = 0..3");
-        switch (p) {
-            case 0: hipLaunchKernelGGL((k_stage_valu<N, 0, R, true>), grid, dim3(128), 0, st, a); break;
-            case 1: hipLaunchKernelGGL((k_stage_valu<N, 1, R, true>), grid, dim3(128), 0, st, a); break;
-            case 2: hipLaunchKernelGGL((k_stage_valu<N, 2, R, true>), grid, dim3(128), 0, st, a); break;
-            case 3: hipLaunchKernelGGL((k_stage_valu<N, 3, R, true>), grid, dim3(128), 0, st, a); break;
-            default: return hipErrorInvalidValue;  // refused on the host before this
-        }
-        return hipGetLastError();
-    }
-    switch (p) {
-        case 0: hipLaunchKernelGGL((k_stage_valu<N, 0, R>), grid, dim3(128), 0, st, a); break;
-        case 1: hipLaunchKernelGGL((k_stage_valu<N, 1, R>), grid, dim3(128), 0, st, a); break;
-        case 2: hipLaunchKernelGGL((k_stage_valu<N, 2, R>), grid, dim3(128), 0, st, a); break;
-        case 3: hipLaunchKernelGGL((k_stage_valu<N, 3, R>), grid, dim3(128), 0, st, a); break;
-        case 4: hipLaunchKernelGGL((k_stage_valu<N, 4, R>), grid, dim3(128), 0, st, a); break;
-        case 5: hipLaunchKernelGGL((k_stage_valu<N, 5, R>), grid, dim3(128), 0, st, a); break;
+template <int P, typename R, bool BND, bool NT>
+static hipError_t launch_stage_lane(const StageArgs<R>& a, dim3 grid, hipStream_t st) {
+    switch (a.kind) {
+        case ST_RHS: hipLaunchKernelGGL((k_stage_lane<P, ST_RHS, R, BND, NT>), grid, dim3(128), 0, st, a); break;
+        case ST_RK4_1: hipLaunchKernelGGL((k_stage_lane<P, ST_RK4_1, R, BND, NT>), grid, dim3(128), 0, st, a); break;
+        case ST_RK4_2: hipLaunchKernelGGL((k_stage_lane<P, ST_RK4_2, R, BND, NT>), grid, dim3(128), 0, st, a); break;
+        case ST_RK4_3: hipLaunchKernelGGL((k_stage_lane<P, ST_RK4_3, R, BND, NT>), grid, dim3(128), 0, st, a); break;
+        case ST_RK4_4: hipLaunchKernelGGL((k_stage_lane<P, ST_RK4_4, R, BND, NT>), grid, dim3(128), 0, st, a); break;
+        case ST_RK2_1: hipLaunchKernelGGL((k_stage_lane<P, ST_RK2_1, R, BND, NT>), grid, dim3(128), 0, st, a); break;
+        case ST_RK2_2: hipLaunchKernelGGL((k_stage_lane<P, ST_RK2_2, R, BND, NT>), grid, dim3(128), 0, st, a); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
 
+// advection at every order (boundary sides up to p = 3), Euler at p = 4, 5
+template <int N, int P, typename R>
+static hipError_t launch_stage_valu_np(const StageArgs<R>& a, dim3 grid, hipStream_t st) {
+    if (a.bnd) {
+        if constexpr (P <= VALU_BOUNDARY_MAX_P)
+            hipLaunchKernelGGL((k_stage_valu<N, P, R, true>), grid, dim3(128), 0, st, a);
+        else
+            return hipErrorInvalidValue;  // refused on the host before this
+    } else {
+        hipLaunchKernelGGL((k_stage_valu<N, P, R>), grid, dim3(128), 0, st, a);
+    }
+    return hipGetLastError();
+}
+
+template <int P, typename R>
+static hipError_t launch_euler(const StageArgs<R>& a, dim3 grid, hipStream_t st) {
+    if constexpr (lane_vec(4, P)) {
+        static_assert(P <= VALU_BOUNDARY_MAX_P, "the vector layout's kernels carry boundary sides");
+        if constexpr (sizeof(R) == 4)
+            if (!a.stream)
+                return a.bnd ? launch_stage_lane<P, R, true, false>(a, grid, st)
+                             : launch_stage_lane<P, R, false, false>(a, grid, st);
+        return a.bnd ? launch_stage_lane<P, R, true, true>(a, grid, st)
+                     : launch_stage_lane<P, R, false, true>(a, grid, st);
+    } else {
+        return launch_stage_valu_np<4, P, R>(a, grid, st);
+    }
+}
+
 template <typename R>
 hipError_t launch_stage_valu(int N, int p, const StageArgs<R>& a, dim3 grid, hipStream_t st) {
-    if (N == 1) return launch_stage_valu_np<1, R>(p, a, grid, st);
-    if (N == 4) return launch_stage_valu_np<4, R>(p, a, grid, st);
+    if (N == 1) {
+        switch (p) {
+            case 0: return launch_stage_valu_np<1, 0, R>(a, grid, st);
+            case 1: return launch_stage_valu_np<1, 1, R>(a, grid, st);
+            case 2: return launch_stage_valu_np<1, 2, R>(a, grid, st);
+            case 3: return launch_stage_valu_np<1, 3, R>(a, grid, st);
+            case 4: return launch_stage_valu_np<1, 4, R>(a, grid, st);
+            case 5: return launch_stage_valu_np<1, 5, R>(a, grid, st);
+        }
+    } else if (N == 4) {
+        switch (p) {
+            case 0: return launch_euler<0, R>(a, grid, st);
+            case 1: return launch_euler<1, R>(a, grid, st);
+            case 2: return launch_euler<2, R>(a, grid, st);
+            case 3: return launch_euler<3, R>(a, grid, st);
+            case 4: return launch_euler<4, R>(a, grid, st);
+            case 5: return launch_euler<5, R>(a, grid, st);
+        }
+    }
     return hipErrorInvalidValue;
 }
 template hipError_t launch_stage_valu<float>(int, int, const StageArgs<float>&, dim3, hipStream_t);
@@ -274,8 +368,7 @@ __global__ void __launch_bounds__(256) k_ref_to_state(const double* __restrict__
     const int v = t / ix.Kp, i = t - v * ix.Kp;
     const size_t src = (size_t)perm[i];
     // every slot of the layout is written: padding modes hold zeros
-    const int mp = ix.tiled == 0 ? ix.NP : ix.tiled == 2 ? 16 : 4 * tile_groups(ix.NP);
-    for (int m = 0; m < mp; m++)
+    for (int m = 0; m < ix.slots(); m++)
         dst[ix.at(v, m, i)] = m < ix.NP ? (R)ref[((size_t)v * ix.NP + m) * K + src] : R(0);
 }
 

@@ -70,6 +70,8 @@ struct SlotInfo {
     const int* halo;
     const void* face4;      // packed geometry of the matrix-core kernels
     const void* metric4;
+    const void* lface;      // packed geometry of the lane kernels' vector layout
+    const void* lmetric;
     Ctrl* ctrl;
     int K, Kp, N, p, hcap, kind;
     int boundary;           // the mesh has boundary sides (batched as a solo solve)

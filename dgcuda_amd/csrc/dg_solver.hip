@@ -294,6 +294,7 @@ class SolverT : public Solver {
     uint32_t* fword = nullptr;
     int* halo = nullptr;
     void *face4 = nullptr, *metric4 = nullptr;
+    void *lface = nullptr, *lmetric = nullptr;  // packed geometry of the lane kernel's vector layout
     int64_t tile_bytes = 0;  // fword, halo and packed geometry
     MfmaArgs mx{};
     double *V = nullptr, *Jd = nullptr, *audit_part = nullptr;
@@ -321,13 +322,24 @@ class SolverT : public Solver {
         if (stream) (void)hipStreamSynchronize(stream);  // nothing queued may use the buffers
         if (gexec) (void)hipGraphExecDestroy(gexec);
         void* bufs[] = {c,  acc,        ua,   ub,    geo_e, geo_f, nbr,     V,      Jd,
-                        audit_part, ctrl, fword, halo,  face4, metric4, bnd, perm_d};
+                        audit_part, ctrl, fword, halo,  face4, metric4, bnd, perm_d, lface, lmetric};
         for (void* b : bufs) pool_free(b);
         pool_release_stream(stream);
     }
 
     // StateIx::tiled of this precision's tile layout
-    static constexpr int tile_kind() { return sizeof(R) == 4 ? 1 : 2; }
+    static constexpr int tile_kind() { return sizeof(R) == 4 ? LAYOUT_TILE32 : LAYOUT_TILE64; }
+    // of the lane kernel
+    int lane_kind() const {
+        if (!lane_vec(N, p)) return LAYOUT_MODES;
+        return sizeof(R) == 4 ? LAYOUT_VEC32 : LAYOUT_VEC64;
+    }
+
+    // the four state arrays and the geometry do not fit the 256 MB
+    // memory-side cache
+    int stream_hint() const {
+        return (4 * six.elems() + 17 * (size_t)Kp) * sizeof(R) > (size_t(256) << 20) ? 1 : 0;
+    }
 
     // entries allocated per state array: room for either layout
     size_t state_alloc() const {
@@ -377,7 +389,7 @@ class SolverT : public Solver {
         if (!st) return st;
         HIPST(hipGetDevice(&device));
         if (!(st = pool_stream(&stream))) return st;
-        six = StateIx{N, NP, Kp, 0};
+        six = StateIx{N, NP, Kp, lane_kind()};
         const size_t M = state_alloc();
         if (!(st = alloc((void**)&c, M * sizeof(R)))) return st;
         if (!(st = alloc((void**)&acc, M * sizeof(R)))) return st;
@@ -547,6 +559,12 @@ class SolverT : public Solver {
                 if (res >= 8) s.grid = std::min(s.grid, res / 8 * 8);
                 if (max_groups >= 8) s.grid = std::min(s.grid, max_groups / 8 * 8);
             }
+        } else if (lane_vec(N, p) && !lface) {
+            Status st = alloc(&lface, 12 * (size_t)Kp * sizeof(R));
+            if (st) st = alloc(&lmetric, 4 * (size_t)Kp * sizeof(R));
+            if (!st) return st;
+            HIPST(launch_lane_pack<R>(geo_e, geo_f, nbr, Kp, lface, lmetric, stream));
+            HIPST(hipStreamSynchronize(stream));  // stages may run on other streams
         }
         return Status::ok();
     }
@@ -627,7 +645,7 @@ class SolverT : public Solver {
             // automatic choice falls back to the lane kernel
             if (!(st = make_shape(1, s))) return st;
         }
-        const StateIx nix{N, NP, Kp, s.kind >= 2 ? tile_kind() : 0};
+        const StateIx nix{N, NP, Kp, s.kind >= 2 ? tile_kind() : lane_kind()};
         if (nix.tiled != six.tiled) {
             // acc, ua and ub are written in full (padding included) by a
             // stage before any stage reads them; c is carried over
@@ -677,7 +695,10 @@ class SolverT : public Solver {
         a.kind = kind;
         a.ntiles = shape.ntiles;
         a.xcd_remap = shape.xcd_remap;
+        a.stream = stream_hint();
         a.phys = phys;
+        a.lface = lface;
+        a.lmetric = lmetric;
         a.bnd = bnd;
         hipError_t e;
         hipStream_t sx = on ? on : stream;
@@ -1031,6 +1052,8 @@ class SolverT : public Solver {
         o->halo = halo;
         o->face4 = face4;
         o->metric4 = metric4;
+        o->lface = lface;
+        o->lmetric = lmetric;
         o->ctrl = ctrl;
         o->K = K;
         o->Kp = Kp;

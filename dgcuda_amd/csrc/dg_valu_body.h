@@ -14,9 +14,8 @@
 //   RK stage update    (time_integrator.cu:194-218, 445-464; RK4 in stage
 //                      states, rk_update)
 //   CFL wave speed     (euler.cu:252-278) of the new state on the last stage.
-// Euler up to p = 3 uses the normal-flux forms of the matrix-core kernels
-// (fewer operations and registers); otherwise the reference's operation
-// order is kept.
+// The reference's operation order is kept.  Advection at every order and
+// Euler at p = 4, 5; Euler up to p = 3 runs in dg_lane_body.h.
 #pragma once
 #include "dg_kernels.h"
 
@@ -39,9 +38,6 @@ template <int N, int P, typename R, bool BND = false>
 __device__ __forceinline__ double valu_process(const StageArgs<R>& a, int e, int kind) {
     static_assert(!BND || P <= VALU_BOUNDARY_MAX_P, "boundary sides are compiled for p <= VALU_BOUNDARY_MAX_P");
     constexpr int NP = n_modes(P), NQ = n_quad_vol(P), NQ1 = P + 1;
-    // Euler up to p = 3 uses the normal-flux forms of the matrix-core
-    // kernels (fewer operations and registers; p >= 4 keeps its allocation)
-    constexpr bool NF_FORM = N == 4 && P <= 3;
     const TabP<R, P>& T = tab<R, P>();
     const bool valid = e < a.K;
     const int ee = valid ? e : a.K - 1;
@@ -88,25 +84,13 @@ __device__ __forceinline__ double valu_process(const StageArgs<R>& a, int e, int
 #pragma unroll
                 for (int v = 0; v < N; v++) U[v] += u[v][m] * T.B[m][q];
             R fx[N], fy[N];
-            if constexpr (NF_FORM) {
-                // Euler: fluxes contracted with the inverse map first
-                // (metric_flux), then with the weighted basis gradients
-                metric_flux<R>(a.phys, U, xr, yr, xs, ys, fx, fy);
+            flux<N, R>(a.phys, U, fx, fy);
 #pragma unroll
-                for (int m = 0; m < NP; m++) {
-                    const R bgx = T.Gx[m][q], bgy = T.Gy[m][q];
+            for (int m = 0; m < NP; m++) {
+                const R bgx = T.Gx[m][q], bgy = T.Gy[m][q];
 #pragma unroll
-                    for (int v = 0; v < N; v++) tot[v][m] += fx[v] * bgx + fy[v] * bgy;
-                }
-            } else {
-                flux<N, R>(a.phys, U, fx, fy);
-#pragma unroll
-                for (int m = 0; m < NP; m++) {
-                    const R bgx = T.Gx[m][q], bgy = T.Gy[m][q];
-#pragma unroll
-                    for (int v = 0; v < N; v++)
-                        tot[v][m] += fx[v] * (bgx * ys - bgy * yr) + fy[v] * (-bgx * xs + bgy * xr);
-                }
+                for (int v = 0; v < N; v++)
+                    tot[v][m] += fx[v] * (bgx * ys - bgy * yr) + fy[v] * (-bgx * xs + bgy * xr);
             }
         }
     }
@@ -168,33 +152,20 @@ __device__ __forceinline__ double valu_process(const StageArgs<R>& a, int e, int
             }
             if constexpr (BND)
                 if (bnd) boundary_ghost<N, NQ1, R>(a.bnd, w, j, Uo, Un);
-            if constexpr (NF_FORM) {
-                // Euler: normal fluxes of both sides, the side's sign in
-                // the speed (the matrix-core kernel's form; both elements of
-                // the side still get bit-identical values)
-                R Fo[N], Fb[N], so, sb;
-                normal_flux_speed<R>(a.phys, Uo, nx, ny, Fo, so);
-                normal_flux_speed<R>(a.phys, Un, nx, ny, Fb, sb);
-                const R lm = fmax(so, sb);
-                const R lms = left ? lm : -lm;
+            R UL[N], UR[N];
 #pragma unroll
-                for (int v = 0; v < N; v++) FS[j][v] = T.W1[j] * (R(0.5) * fma(lms, Uo[v] - Un[v], Fo[v] + Fb[v]));
-            } else {
-                R UL[N], UR[N];
-#pragma unroll
-                for (int v = 0; v < N; v++) {
-                    UL[v] = left ? Uo[v] : Un[v];
-                    UR[v] = left ? Un[v] : Uo[v];
-                }
-                R fxl[N], fyl[N], fxr[N], fyr[N];
-                flux<N, R>(a.phys, UL, fxl, fyl);
-                flux<N, R>(a.phys, UR, fxr, fyr);
-                const R lam = llf_speed<N, R>(a.phys, UL, UR, nx, ny);
-#pragma unroll
-                for (int v = 0; v < N; v++)
-                    FS[j][v] = T.W1[j] *
-                               (R(0.5) * ((fxl[v] + fxr[v]) * nx + (fyl[v] + fyr[v]) * ny + lam * (UL[v] - UR[v])));
+            for (int v = 0; v < N; v++) {
+                UL[v] = left ? Uo[v] : Un[v];
+                UR[v] = left ? Un[v] : Uo[v];
             }
+            R fxl[N], fyl[N], fxr[N], fyr[N];
+            flux<N, R>(a.phys, UL, fxl, fyl);
+            flux<N, R>(a.phys, UR, fxr, fyr);
+            const R lam = llf_speed<N, R>(a.phys, UL, UR, nx, ny);
+#pragma unroll
+            for (int v = 0; v < N; v++)
+                FS[j][v] = T.W1[j] *
+                           (R(0.5) * ((fxl[v] + fxr[v]) * nx + (fyl[v] + fyr[v]) * ny + lam * (UL[v] - UR[v])));
         }
         const R coef = left ? -len / R(2) : len / R(2);
 #pragma unroll
