@@ -199,6 +199,7 @@ enum StageKind {
     ST_RK4_4 = 4, // u = u4: c = acc + u4/3 + k/6; wave-speed partials
     ST_RK2_1 = 5, // out = c + k/2
     ST_RK2_2 = 6, // c = c + k; wave-speed partials
+    ST_RHS_REF = 7, // k = dt M^-1 R(u) on FP64 arrays in the reference layout (StageArgs::ref_u, ref_k, ref_dt)
 };
 
 // Classical RK4 (time_integrator.cu:221) on every stage kernel, written
@@ -240,7 +241,7 @@ __device__ __forceinline__ R div3(R x) {
 
 template <int KIND, typename R>
 __device__ __forceinline__ R rk_update(R c, R aa, R k, R* acc_out) {
-    if constexpr (KIND == ST_RHS) {
+    if constexpr (KIND == ST_RHS || KIND == ST_RHS_REF) {
         return k;
     } else if constexpr (KIND == ST_RK4_1 || KIND == ST_RK2_1) {
         return c + R(0.5) * k;
@@ -254,6 +255,18 @@ __device__ __forceinline__ R rk_update(R c, R aa, R k, R* acc_out) {
     } else {
         return c + k;
     }
+}
+
+// Pointers that arrive through memory (the batch slot table) are generic
+// to the compiler, which then issues FLAT accesses with 64-bit per-lane
+// addresses.  Reading and writing through a global-address-space view
+// gives scalar-base global loads whatever the pointer's origin.
+#ifndef DG_GLOBAL  // a host build of these headers (tests/host_check) defines it empty
+#define DG_GLOBAL __attribute__((address_space(1)))
+#endif
+template <typename T>
+__device__ __forceinline__ DG_GLOBAL T* gp(T* p) {
+    return (DG_GLOBAL T*)p;
 }
 
 // Placement of entry (variable v, mode m, element e) of a state array in HBM.
@@ -315,6 +328,14 @@ struct StageArgs {
     int xcd_remap;    // map consecutive tiles to one XCD
     int stream;       // vector layout: the solve's arrays exceed the memory-side cache
     PhysP phys;
+    // ST_RHS_REF: input and output [N][n_p][K] in the caller's element order,
+    // the caller's element of each element (null: the same order), and dt.
+    // The kernel reads and writes the caller's arrays itself, so neither the
+    // control block nor a copy of the state in the solve's layout is needed.
+    const double* ref_u;
+    double* ref_k;
+    const int* ref_perm;
+    double ref_dt;
     // lane kernels in the vector layout: packed geometry, per face 4 values
     // (nx, ny, len, neighbour word: FP32 its bits, FP64 its value) [3][Kp],
     // per element 4 values (xr, yr, xs, ys) [Kp]
@@ -325,6 +346,23 @@ struct StageArgs {
     // reflecting points; null for a mesh without boundary sides
     const double* bnd;
 };
+
+// caller's element of element e
+template <typename R>
+__device__ __forceinline__ int ref_elem(const StageArgs<R>& a, int e) {
+    return a.ref_perm ? a.ref_perm[e] : e;
+}
+// entry (row = v*n_p + m, uniform; caller's element o) of an array in the
+// reference layout: a scalar row base and a 32-bit byte offset per lane
+// (o < 2^28)
+__device__ __forceinline__ const DG_GLOBAL double* ref_at(const double* x, int row, int K, int o) {
+    const char DG_GLOBAL* b = (const char DG_GLOBAL*)(const DG_GLOBAL double*)x + (size_t)row * K * 8;
+    return (const DG_GLOBAL double*)(b + (unsigned)o * 8u);
+}
+__device__ __forceinline__ DG_GLOBAL double* ref_at(double* x, int row, int K, int o) {
+    char DG_GLOBAL* b = (char DG_GLOBAL*)(DG_GLOBAL double*)x + (size_t)row * K * 8;
+    return (DG_GLOBAL double*)(b + (unsigned)o * 8u);
+}
 
 // Workgroup -> tile mapping.  The dispatcher places workgroup b on XCD b % 8;
 // with remapping, XCD x receives the contiguous tile range
@@ -341,18 +379,6 @@ __device__ __forceinline__ int tile_of_block(int b, int nblocks, int remap) {
 // reference's euler.cu:61-168 (pressure, eval_c, eval_flux, eval_lambda) and
 // of the advection flux F = (ax u, ay u) with the LLF speed |a.n|.
 // ---------------------------------------------------------------------------
-// Pointers that arrive through memory (the batch slot table) are generic
-// to the compiler, which then issues FLAT accesses with 64-bit per-lane
-// addresses.  Reading and writing through a global-address-space view
-// gives scalar-base global loads whatever the pointer's origin.
-#ifndef DG_GLOBAL  // a host build of these headers (tests/host_check) defines it empty
-#define DG_GLOBAL __attribute__((address_space(1)))
-#endif
-template <typename T>
-__device__ __forceinline__ DG_GLOBAL T* gp(T* p) {
-    return (DG_GLOBAL T*)p;
-}
-
 template <typename R>
 __device__ __forceinline__ R rdiv(R a, R b);
 template <>

@@ -97,6 +97,12 @@ hipError_t launch_lane_pack(const R* geo_e, const R* geo_f, const int* nbr, int 
                             hipStream_t st);
 // orders and physics whose lane kernel keeps its state in the vector layout
 __host__ __device__ constexpr bool lane_vec(int N, int p) { return N == 4 && p <= 3; }
+// Whether kernel kind `kind` has an instance on the caller's arrays
+// (ST_RHS_REF): all but the Euler lane kernel at p = 4, 5, whose arithmetic
+// and spills (0.4 ms at 131,072 triangles) leave the conversions no weight.
+__host__ __device__ constexpr bool ref_rhs_supported(int N, int p, int kind) {
+    return kind >= 2 || N == 1 || lane_vec(N, p);
+}
 
 // Extra per-solve data of the matrix-core kernel: per (element, face) a
 // 32-bit word {bits 0..11 LDS slot of the neighbour (own tile element or

@@ -23,9 +23,15 @@ namespace dgmi {
 DGMI_TABLE_UPLOADER(upload_tables_kernels)
 
 // BND: the variant for meshes with boundary sides (p <= VALU_BOUNDARY_MAX_P)
-template <int N, int P, typename R, bool BND = false>
+// REF: the right-hand side on the caller's arrays
+template <int N, int P, typename R, bool BND = false, bool REF = false>
 __global__ void __launch_bounds__(128) k_stage_valu(StageArgs<R> a) {
     __shared__ double sh[8];
+    if constexpr (REF) {
+        const int t = tile_of_block(blockIdx.x, gridDim.x, a.xcd_remap);
+        if (t < a.ntiles) valu_process<N, P, R, BND, true>(a, t * blockDim.x + threadIdx.x, ST_RHS);
+        return;
+    }
     if (!a.ctrl->active) return;
     const int tile = tile_of_block(blockIdx.x, gridDim.x, a.xcd_remap);
     if (tile >= a.ntiles) return;
@@ -49,7 +55,8 @@ constexpr int lane_minw() {
 template <int P, int KIND, typename R, bool BND, bool NT>
 __global__ void __launch_bounds__(128, (lane_minw<P, R>())) k_stage_lane(StageArgs<R> a) {
     __shared__ double sh[8];
-    if (!a.ctrl->active) return;
+    if constexpr (KIND != ST_RHS_REF)
+        if (!a.ctrl->active) return;
     const int tile = tile_of_block(blockIdx.x, gridDim.x, a.xcd_remap);
     if (tile >= a.ntiles) return;
     __shared__ __align__(16) R ltab[LaneTab<P>::SIZE];
@@ -226,6 +233,13 @@ static hipError_t launch_stage_lane(const StageArgs<R>& a, dim3 grid, hipStream_
         case ST_RK4_4: hipLaunchKernelGGL((k_stage_lane<P, ST_RK4_4, R, BND, NT>), grid, dim3(128), 0, st, a); break;
         case ST_RK2_1: hipLaunchKernelGGL((k_stage_lane<P, ST_RK2_1, R, BND, NT>), grid, dim3(128), 0, st, a); break;
         case ST_RK2_2: hipLaunchKernelGGL((k_stage_lane<P, ST_RK2_2, R, BND, NT>), grid, dim3(128), 0, st, a); break;
+        case ST_RHS_REF:
+            if constexpr (NT) {  // (its streams are the caller's arrays)
+                hipLaunchKernelGGL((k_stage_lane<P, ST_RHS_REF, R, BND, NT>), grid, dim3(128), 0, st, a);
+                break;
+            } else {
+                return hipErrorInvalidValue;
+            }
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -234,6 +248,20 @@ static hipError_t launch_stage_lane(const StageArgs<R>& a, dim3 grid, hipStream_
 // advection at every order (boundary sides up to p = 3), Euler at p = 4, 5
 template <int N, int P, typename R>
 static hipError_t launch_stage_valu_np(const StageArgs<R>& a, dim3 grid, hipStream_t st) {
+    if (a.kind == ST_RHS_REF) {
+        if constexpr (ref_rhs_supported(N, P, 1)) {
+            if constexpr (P <= VALU_BOUNDARY_MAX_P)
+                if (a.bnd) {
+                    hipLaunchKernelGGL((k_stage_valu<N, P, R, true, true>), grid, dim3(128), 0, st, a);
+                    return hipGetLastError();
+                }
+            if (a.bnd) return hipErrorInvalidValue;  // refused on the host before this
+            hipLaunchKernelGGL((k_stage_valu<N, P, R, false, true>), grid, dim3(128), 0, st, a);
+            return hipGetLastError();
+        } else {
+            return hipErrorInvalidValue;
+        }
+    }
     if (a.bnd) {
         if constexpr (P <= VALU_BOUNDARY_MAX_P)
             hipLaunchKernelGGL((k_stage_valu<N, P, R, true>), grid, dim3(128), 0, st, a);
@@ -250,7 +278,7 @@ static hipError_t launch_euler(const StageArgs<R>& a, dim3 grid, hipStream_t st)
     if constexpr (lane_vec(4, P)) {
         static_assert(P <= VALU_BOUNDARY_MAX_P, "the vector layout's kernels carry boundary sides");
         if constexpr (sizeof(R) == 4)
-            if (!a.stream)
+            if (!a.stream && a.kind != ST_RHS_REF)
                 return a.bnd ? launch_stage_lane<P, R, true, false>(a, grid, st)
                              : launch_stage_lane<P, R, false, false>(a, grid, st);
         return a.bnd ? launch_stage_lane<P, R, true, true>(a, grid, st)

@@ -128,6 +128,15 @@ __device__ __forceinline__ void lane_load(const R* __restrict__ x, int Kp, int e
         }
 }
 
+// all modes of caller's element o of an FP64 array in the reference layout
+template <int NP, typename R>
+__device__ __forceinline__ void lane_load_ref(const double* __restrict__ x, int K, int o, R (&u)[4][NP]) {
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+#pragma unroll
+        for (int m = 0; m < NP; m++) u[v][m] = (R)*ref_at(x, v * NP + m, K, o);
+}
+
 // Neighbour-side trace table of order P in LDS: row (face, own point j)
 // holds phi_m at the neighbour's point NQ1-1-j, the modes of a row
 // contiguous (16-byte reads).  The neighbour's face differs from lane to lane; reading the
@@ -163,12 +172,21 @@ __device__ __forceinline__ double lane_process(const StageArgs<R>& a, int e, con
     const bool valid = e < a.K;
     const int ee = valid ? e : a.K - 1;
     const int Kp = a.Kp;
+    constexpr bool REF = KIND == ST_RHS_REF;
+    // (element e of the kernel's order: from the stage's input in the vector
+    // layout, or from the caller's array)
+    const auto load = [&](int x, R (&o)[N][NP]) {
+        if constexpr (REF)
+            lane_load_ref<NP, R>(a.ref_u, a.K, ref_elem(a, x), o);
+        else
+            lane_load<NP, R>(a.u, Kp, x, o);
+    };
 
     G4 rec[3];
 #pragma unroll
     for (int f = 0; f < 3; f++) rec[f] = ((const DG_GLOBAL G4*)a.lface)[(size_t)f * Kp + ee];
     R u[N][NP];
-    lane_load<NP, R>(a.u, Kp, ee, u);
+    load(ee, u);
     const G4 me = ((const DG_GLOBAL G4*)a.lmetric)[ee];
     const R ij = gp(a.geo_e)[4 * (size_t)Kp + ee];
 
@@ -184,7 +202,7 @@ __device__ __forceinline__ double lane_process(const StageArgs<R>& a, int e, con
     // one face ahead of its use
     constexpr bool AHEAD = sizeof(R) == 4 ? P <= 2 : P <= 1;
     R nu[AHEAD ? 2 : 1][N][NP];
-    if constexpr (AHEAD) lane_load<NP, R>(a.u, Kp, nb[0], nu[0]);
+    if constexpr (AHEAD) load(nb[0], nu[0]);
 
     R tot[N][NP];
 #pragma unroll
@@ -227,9 +245,9 @@ __device__ __forceinline__ double lane_process(const StageArgs<R>& a, int e, con
             for (int m = 0; m < NP; m++) LANE_KEEP(tot[v][m]);
         LANE_FENCE();
         if constexpr (AHEAD) {
-            if (f < 2) lane_load<NP, R>(a.u, Kp, nb[f + 1], nu[(f + 1) & 1]);
+            if (f < 2) load(nb[f + 1], nu[(f + 1) & 1]);
         } else {
-            lane_load<NP, R>(a.u, Kp, nb[f], nu[0]);
+            load(nb[f], nu[0]);
         }
         if (f == 2) {
             // the stage update's operands, under the last face's arithmetic
@@ -282,6 +300,17 @@ __device__ __forceinline__ double lane_process(const StageArgs<R>& a, int e, con
     }
 
     // ---- inverse mass (M = J*I; 1/J precomputed in FP64) and the RK stage update ----
+    if constexpr (REF) {
+        const R cj = ij * (R)a.ref_dt;
+        if (valid) {
+            const int o = ref_elem(a, e);
+#pragma unroll
+            for (int v = 0; v < N; v++)
+#pragma unroll
+                for (int m = 0; m < NP; m++) *ref_at(a.ref_k, v * NP + m, a.K, o) = (double)(cj * tot[v][m]);
+        }
+        return 0.0;
+    }
     const R cj = ij * (R)a.ctrl->dt;
     double lam = 0.0;
     V o[NP][NG], w[NP][NG];

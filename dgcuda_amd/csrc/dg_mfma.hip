@@ -68,12 +68,14 @@ hipError_t mfma_layout_probe_f64(double* host_out) {
 #ifndef DGMI_MFMA_MINW
 #define DGMI_MFMA_MINW 3
 #endif
-template <typename R>
-constexpr int mfma_minw() { return sizeof(R) == 4 ? DGMI_MFMA_MINW : 2; }
+// The instance on the caller's FP64 arrays (ST_RHS_REF) holds its state as
+// read: 2 in both precisions (3 in FP32 spills and is no faster).
+template <typename R, int KIND>
+constexpr int mfma_minw() { return sizeof(R) == 4 && KIND != ST_RHS_REF ? DGMI_MFMA_MINW : 2; }
 
 // BND: the variant for meshes with boundary sides (Euler only)
 template <int N, int P, int KIND, typename R, bool BND = false>
-__global__ void __launch_bounds__(256, mfma_minw<R>()) k_stage_mfma(StageArgs<R> a, MfmaArgs mx) {
+__global__ void __launch_bounds__(256, (mfma_minw<R, KIND>())) k_stage_mfma(StageArgs<R> a, MfmaArgs mx) {
     using V = typename MfmaT<R>::V;
     constexpr bool LAST = (KIND == ST_RK4_4 || KIND == ST_RK2_2);
     extern __shared__ float4 lds4[];
@@ -81,7 +83,9 @@ __global__ void __launch_bounds__(256, mfma_minw<R>()) k_stage_mfma(StageArgs<R>
     R* ts = tile_traces<V, R>(fd);
     __shared__ double shmax[8];
 
-    if (!a.ctrl->active) return;
+    constexpr bool REF = KIND == ST_RHS_REF;
+    if constexpr (!REF)
+        if (!a.ctrl->active) return;
     const int ntiles = a.ntiles;
     int t, tend, stride;
     if (a.xcd_remap) {
@@ -98,8 +102,12 @@ __global__ void __launch_bounds__(256, mfma_minw<R>()) k_stage_mfma(StageArgs<R>
     const int g = lane >> 4, j = lane & 15;
     double lam = 0.0;
     __shared__ V tabA[MFMA_A_SLOTS * 64];
-    const R dt = (R)a.ctrl->dt;
-    MfmaTileState<N, P, R> st;
+    R dt;
+    if constexpr (REF)
+        dt = (R)a.ref_dt;
+    else
+        dt = (R)a.ctrl->dt;
+    MfmaTileState<N, P, R, REF> st;
     int hid[MfmaTileState<N, P, R>::HPW];
     TileGeo<R> gc;
     // tiles past the end of the walk read tile tend-1 instead (the loads
@@ -108,7 +116,7 @@ __global__ void __launch_bounds__(256, mfma_minw<R>()) k_stage_mfma(StageArgs<R>
     if (t < tend) {
         MfmaTileState<N, P, R>::load_ids(mx.halo, mx.hcap, t, w, j, hid);
         gc.load(a, mx, t, w * 16 + j);
-        st.load_data(a.u, a.K, t, w, g, j, hid);
+        st.load_next(a, t, w, g, j, hid);
         MfmaTileState<N, P, R>::load_ids(mx.halo, mx.hcap, walk(t + stride), w, j, hid);
     }
     if (w == 0) mfma_a_to_lds<N, P, R>(tabA, lane);
@@ -221,6 +229,7 @@ static hipError_t prepare_lds() {
             if (e == hipSuccess) e = allow_large_lds(&k_stage_mfma<N, P, ST_RK4_4, R, BND>);
             if (e == hipSuccess) e = allow_large_lds(&k_stage_mfma<N, P, ST_RK2_1, R, BND>);
             if (e == hipSuccess) e = allow_large_lds(&k_stage_mfma<N, P, ST_RK2_2, R, BND>);
+            if (e == hipSuccess) e = allow_large_lds(&k_stage_mfma<N, P, ST_RHS_REF, R, BND>);
             return e;
         }();
         return once;
@@ -240,6 +249,7 @@ static hipError_t launch_np(const StageArgs<R>& a, const MfmaArgs& mx, dim3 grid
         case ST_RK4_4: hipLaunchKernelGGL((k_stage_mfma<N, P, ST_RK4_4, R, BND>), grid, dim3(256), lds, st, a, mx); break;
         case ST_RK2_1: hipLaunchKernelGGL((k_stage_mfma<N, P, ST_RK2_1, R, BND>), grid, dim3(256), lds, st, a, mx); break;
         case ST_RK2_2: hipLaunchKernelGGL((k_stage_mfma<N, P, ST_RK2_2, R, BND>), grid, dim3(256), lds, st, a, mx); break;
+        case ST_RHS_REF: hipLaunchKernelGGL((k_stage_mfma<N, P, ST_RHS_REF, R, BND>), grid, dim3(256), lds, st, a, mx); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

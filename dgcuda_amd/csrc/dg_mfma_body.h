@@ -27,6 +27,8 @@
 // atomics, no face buffers in HBM.
 #pragma once
 
+#include <type_traits>
+
 #include "dg_kernels.h"
 
 namespace dgmi {
@@ -184,13 +186,47 @@ __device__ __forceinline__ void mfma_a_to_lds(typename MfmaT<R>::V* tabA, int la
 // State operands of one tile held by one wavefront: its own sub-tile, and
 // its share of the halo, dealt as (halo sub-tile, variable) pairs
 // round-robin to the 4 wavefronts.
-template <int N, int P, typename R = float>
+// REF: the state comes from the caller's FP64 array in the reference layout
+// (ST_RHS_REF) and is held as read; `own` and `halo` give the operands in
+// the bulk precision.
+template <int N, int P, typename R = float, bool REF = false>
 struct MfmaTileState {
     using V = typename MfmaT<R>::V;
+    using VM = typename MfmaT<typename std::conditional<REF, double, R>::type>::V;
     static constexpr int HPW = (4 * N + 3) / 4;  // most halo pairs per wave (hcap <= 64)
     static constexpr int VS = tile_var_stride<P, R>();
-    V ub[N];
-    V hb[HPW];
+    VM ub[N];
+    VM hb[HPW];
+    __device__ __forceinline__ static V bulk(const VM& x) {
+        if constexpr (REF)
+            return V{(R)x[0], (R)x[1], (R)x[2], (R)x[3]};
+        else
+            return x;
+    }
+    __device__ __forceinline__ V own(int v) const { return bulk(ub[v]); }
+    __device__ __forceinline__ V halo(int q) const { return bulk(hb[q]); }
+    // variable v, modes pos(g, 0..3) (padding modes read the last mode: they
+    // meet zero matrix entries) of caller's element o
+    __device__ __forceinline__ static VM load_ref(const double* __restrict__ x, int v, int K, int g, int o) {
+        constexpr int NP = n_modes(P);
+        VM r;
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+            r[s] = *(const DG_GLOBAL double*)((const char DG_GLOBAL*)(const DG_GLOBAL double*)x +
+                                              ((size_t)(v * NP + min(MfmaT<R>::pos(g, s), NP - 1)) * K + o) * 8);
+        return r;
+    }
+    __device__ __forceinline__ void load_ref_data(const StageArgs<R>& a, int tile, int w, int g, int j,
+                                                  const int (&hid)[HPW]) {
+        const int o = ref_elem(a, min(tile * MFMA_TILE + w * 16 + j, a.K - 1));
+        int oh[HPW];
+#pragma unroll
+        for (int q = 0; q < HPW; q++) oh[q] = ref_elem(a, hid[q]);
+#pragma unroll
+        for (int v = 0; v < N; v++) ub[v] = load_ref(a.ref_u, v, a.K, g, o);
+#pragma unroll
+        for (int q = 0; q < HPW; q++) hb[q] = load_ref(a.ref_u, (w + 4 * q) % N, a.K, g, oh[q]);
+    }
     // Halo element ids of this wave's pairs.  A halo state load depends on
     // its id, and waiting for an id waits for every load issued before it,
     // so the ids are requested ahead of the state loads that use them.
@@ -215,11 +251,12 @@ struct MfmaTileState {
 #pragma unroll
         for (int q = 0; q < HPW; q++) hb[q] = gp4(u)[((w + 4 * q) % N) * VS + tile_lane4<N, P, R>(hid[q], g)];
     }
-    __device__ __forceinline__ void load(const R* __restrict__ u, int K, const int* __restrict__ halo, int hcap,
-                                         int tile, int w, int g, int j) {
-        int hid[HPW];
-        load_ids(halo, hcap, tile, w, j, hid);
-        load_data(u, K, tile, w, g, j, hid);
+    __device__ __forceinline__ void load_next(const StageArgs<R>& a, int tile, int w, int g, int j,
+                                              const int (&hid)[HPW]) {
+        if constexpr (REF)
+            load_ref_data(a, tile, w, g, j, hid);
+        else
+            load_data(a.u, a.K, tile, w, g, j, hid);
     }
 };
 
@@ -352,7 +389,8 @@ __device__ __forceinline__ void side_flux(const StageArgs<R>& a, const typename 
 // LDS table `tabA`.
 template <int N, int P, int KIND, typename R, bool BND = false>
 __device__ __forceinline__ double mfma_process_tile_pipe(const StageArgs<R>& a, const MfmaArgs& mx,
-                                                         const typename MfmaT<R>::V* tabA, MfmaTileState<N, P, R>& st,
+                                                         const typename MfmaT<R>::V* tabA,
+                                                         MfmaTileState<N, P, R, KIND == ST_RHS_REF>& st,
                                                          int (&hid)[MfmaTileState<N, P, R>::HPW], TileGeo<R>& gc,
                                                          R dt, int tile, int next, int next2,
                                                          typename MfmaT<R>::V* fd, R* ts) {
@@ -382,6 +420,10 @@ __device__ __forceinline__ double mfma_process_tile_pipe(const StageArgs<R>& a, 
     // plus a padding row; points >= 3(p+1) are read by the surface
     // projection only to be replaced by zero)
     const V Atr = tabA[MFMA_A_TR * 64 + lane];
+    constexpr bool REF = KIND == ST_RHS_REF;
+    V ub[N];
+#pragma unroll
+    for (int v = 0; v < N; v++) ub[v] = st.own(v);
     {
         V T[N];
 #pragma unroll
@@ -389,7 +431,7 @@ __device__ __forceinline__ double mfma_process_tile_pipe(const StageArgs<R>& a, 
             T[v] = V{0, 0, 0, 0};
 #pragma unroll
             for (int s = 0; s < 4; s++)
-                if (mode_step_used<R, NP>(s)) T[v] = M::mma(Atr[s], st.ub[v][s], T[v]);
+                if (mode_step_used<R, NP>(s)) T[v] = M::mma(Atr[s], ub[v][s], T[v]);
         }
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -406,9 +448,10 @@ __device__ __forceinline__ double mfma_process_tile_pipe(const StageArgs<R>& a, 
         if (pr < npairs) {
             const int slot = TILE + (pr / N) * 16 + j, v = pr % N;
             V acc = {0, 0, 0, 0};
+            const V hb = st.halo(q);
 #pragma unroll
             for (int s = 0; s < 4; s++)
-                if (mode_step_used<R, NP>(s)) acc = M::mma(Atr[s], st.hb[q][s], acc);
+                if (mode_step_used<R, NP>(s)) acc = M::mma(Atr[s], hb[s], acc);
 #pragma unroll
             for (int i = 0; i < 4; i++) ts[slot * TS + M::qpos(g, i) * N + v] = acc[i];
         }
@@ -443,7 +486,7 @@ __device__ __forceinline__ double mfma_process_tile_pipe(const StageArgs<R>& a, 
         V acc = {0, 0, 0, 0};
 #pragma unroll
         for (int s = 0; s < 4; s++)
-            if (mode_step_used<R, NP>(s)) acc = M::mma(Avol[s], st.ub[v][s], acc);
+            if (mode_step_used<R, NP>(s)) acc = M::mma(Avol[s], ub[v][s], acc);
         U[v] = acc;
     }
     // RK registers of this tile, then the next tile's state (st is dead
@@ -465,15 +508,15 @@ __device__ __forceinline__ double mfma_process_tile_pipe(const StageArgs<R>& a, 
     for (int v = 0; v < N; v++) {
         cr[v] = V{0, 0, 0, 0};
         ar[v] = V{0, 0, 0, 0};
-        if constexpr (RK::C_FROM_INPUT) cr[v] = st.ub[v];
-        if constexpr (RK::ACC_FROM_INPUT) ar[v] = st.ub[v];
+        if constexpr (RK::C_FROM_INPUT) cr[v] = ub[v];
+        if constexpr (RK::ACC_FROM_INPUT) ar[v] = ub[v];
         if constexpr (sizeof(R) == 4) {
             if constexpr (RK::LOAD_C) cr[v] = __builtin_nontemporal_load(&gp4(a.c)[v * VS + l4]);
             if constexpr (RK::LOAD_ACC) ar[v] = __builtin_nontemporal_load(&gp4(a.acc)[v * VS + l4]);
         }
     }
     __builtin_amdgcn_sched_barrier(0);
-    st.load_data(a.u, K, next, w, g, j, hid);
+    st.load_next(a, next, w, g, j, hid);
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(0);
     V Rv[N];
@@ -585,6 +628,22 @@ __device__ __forceinline__ double mfma_process_tile_pipe(const StageArgs<R>& a, 
     MfmaTileState<N, P>::load_ids(mx.halo, mx.hcap, next2, w, j, hid);
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(0);
+
+    if constexpr (REF) {
+        // k into the caller's array; lane holds modes m = pos(g, i)
+        if (valid) {
+            const int o = ref_elem(a, e);
+#pragma unroll
+            for (int v = 0; v < N; v++)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (M::pos(g, i) < NP)
+                        *(DG_GLOBAL double*)((char DG_GLOBAL*)(DG_GLOBAL double*)a.ref_k +
+                                             ((size_t)(v * NP + M::pos(g, i)) * K + o) * 8) = (double)(cj * Rv[v][i]);
+        }
+        __syncthreads();  // the next tile reuses the LDS
+        return 0.0;
+    }
 
     // inverse mass and the RK stage update; lane holds modes m = pos(g, i)
     const unsigned s4 = tile_lane4<N, P, R>(e, g);

@@ -34,7 +34,8 @@ __device__ __forceinline__ R face_phi(const TabP<R, P>& T, int f, int m, int j, 
 // BND: the variant for meshes with boundary sides (p <= VALU_BOUNDARY_MAX_P);
 // without it the face loop carries no branch and the loads of the three
 // faces can be scheduled together.
-template <int N, int P, typename R, bool BND = false>
+// REF: the right-hand side on the caller's arrays (ST_RHS_REF).
+template <int N, int P, typename R, bool BND = false, bool REF = false>
 __device__ __forceinline__ double valu_process(const StageArgs<R>& a, int e, int kind) {
     static_assert(!BND || P <= VALU_BOUNDARY_MAX_P, "boundary sides are compiled for p <= VALU_BOUNDARY_MAX_P");
     constexpr int NP = n_modes(P), NQ = n_quad_vol(P), NQ1 = P + 1;
@@ -42,12 +43,25 @@ __device__ __forceinline__ double valu_process(const StageArgs<R>& a, int e, int
     const bool valid = e < a.K;
     const int ee = valid ? e : a.K - 1;
     const int Kp = a.Kp;
-    const R dt = (R)a.ctrl->dt;
+    R dt;
+    if constexpr (REF)
+        dt = (R)a.ref_dt;
+    else
+        dt = (R)a.ctrl->dt;
+    // mode (v, m) of element x, at `o` in the caller's order
+    const auto at = [&](int v, int m, int x, int o) -> R {
+        if constexpr (REF)
+            return (R)*ref_at(a.ref_u, v * NP + m, a.K, o);
+        else
+            return gp(a.u)[(size_t)(v * NP + m) * Kp + x];
+    };
+    const auto caller = [&](int x) { return REF ? ref_elem(a, x) : 0; };
+    const int oe = caller(ee);
     R u[N][NP];
 #pragma unroll
     for (int v = 0; v < N; v++)
 #pragma unroll
-        for (int m = 0; m < NP; m++) u[v][m] = gp(a.u)[(size_t)(v * NP + m) * Kp + ee];
+        for (int m = 0; m < NP; m++) u[v][m] = at(v, m, ee, oe);
 
     R tot[N][NP];
 #pragma unroll
@@ -64,11 +78,11 @@ __device__ __forceinline__ double valu_process(const StageArgs<R>& a, int e, int
     if constexpr (!BND) {
 #pragma unroll
         for (int f = 0; f < 3; f++) wf[f] = gp(a.nbr)[f * Kp + ee];
-        const int nb0 = wf[0] & NB_ELEM_MASK;
+        const int nb0 = wf[0] & NB_ELEM_MASK, ob0 = caller(nb0);
 #pragma unroll
         for (int v = 0; v < N; v++)
 #pragma unroll
-            for (int m = 0; m < NP; m++) nu[v][m] = gp(a.u)[(size_t)(v * NP + m) * Kp + nb0];
+            for (int m = 0; m < NP; m++) nu[v][m] = at(v, m, nb0, ob0);
     }
 
     // ---- volume: sum_q F(U_q) . (metric * grad phi_m) ----
@@ -104,11 +118,11 @@ __device__ __forceinline__ double valu_process(const StageArgs<R>& a, int e, int
         } else {
             w = wf[f];
             if (f > 0) {
-                const int nbf = w & NB_ELEM_MASK;
+                const int nbf = w & NB_ELEM_MASK, obf = caller(nbf);
 #pragma unroll
                 for (int v = 0; v < N; v++)
 #pragma unroll
-                    for (int m = 0; m < NP; m++) nu[v][m] = gp(a.u)[(size_t)(v * NP + m) * Kp + nbf];
+                    for (int m = 0; m < NP; m++) nu[v][m] = at(v, m, nbf, obf);
             }
         }
         // boundary side (BND variant): no neighbour, a ghost state
@@ -118,6 +132,7 @@ __device__ __forceinline__ double valu_process(const StageArgs<R>& a, int e, int
             bnd = w < 0;
             if (bnd) nb = ee;
         }
+        const int ob = BND ? caller(nb) : 0;
         const int fn = (w >> 28) & 3;
         const bool left = (w >> 30) & 1;
         const R nx = gp(a.geo_f)[(3 * f + 0) * Kp + ee];
@@ -145,7 +160,7 @@ __device__ __forceinline__ double valu_process(const StageArgs<R>& a, int e, int
                 for (int v = 0; v < N; v++) {
                     Uo[v] += u[v][m] * so;
                     if constexpr (BND)
-                        Un[v] += gp(a.u)[(size_t)(v * NP + m) * Kp + nb] * sn;
+                        Un[v] += at(v, m, nb, ob) * sn;
                     else
                         Un[v] += nu[v][m] * sn;
                 }
@@ -182,6 +197,14 @@ __device__ __forceinline__ double valu_process(const StageArgs<R>& a, int e, int
     // ---- inverse mass (M = J*I; 1/J precomputed in FP64) and the RK stage update ----
     const R cj = gp(a.geo_e)[4 * Kp + ee] * dt;
     double lam = 0.0;
+    if constexpr (REF) {
+        if (valid)
+#pragma unroll
+            for (int v = 0; v < N; v++)
+#pragma unroll
+                for (int m = 0; m < NP; m++) *ref_at(a.ref_k, v * NP + m, a.K, oe) = (double)(cj * tot[v][m]);
+        return 0.0;
+    }
     if (kind == ST_RHS) {
         if (valid)
 #pragma unroll
