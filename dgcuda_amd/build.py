@@ -21,7 +21,8 @@ HIPCC = os.path.join(ROCM, "bin", "hipcc")
 ARCH = "gfx950"
 
 GXX_SOURCES = ["dg_mesh.cpp", "dg_geometry.cpp", "dg_tables.cpp"]
-HIP_SOURCES = ["dg_kernels.hip", "dg_mfma.hip", "dg_solver.hip", "dg_batch.hip", "dg_capi.cpp", "dg_server.cpp"]
+HIP_SOURCES = ["dg_kernels.hip", "dg_mfma.hip", "dg_solver.hip", "dg_batch.hip", "dg_capi.cpp", "dg_server.cpp",
+               "dg_hostcopy.cpp"]
 
 GXX_FLAGS = ["-O2", "-fPIC", "-std=c++17", "-ffp-contract=off", "-fno-fast-math", "-Wall"]
 HIP_FLAGS = [

@@ -1,0 +1,13 @@
+// Copies between the caller's pageable host arrays and device memory through
+// pinned blocks.
+#pragma once
+#include "dg_solver.h"
+
+namespace dgmi {
+
+// Both wait for the copy.  The device side is ready (copy_to_host) or free to
+// be overwritten (copy_to_device) once the work queued on `st` has finished.
+Status copy_to_host(void* dst, const void* src_dev, size_t bytes, hipStream_t st);
+Status copy_to_device(void* dst_dev, const void* src, size_t bytes, hipStream_t st);
+
+}  // namespace dgmi

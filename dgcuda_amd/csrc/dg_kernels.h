@@ -151,11 +151,21 @@ template <typename R>
 hipError_t launch_lambda(const R* u, const StateIx& ix, int K, double b0, const PhysP& ph, Ctrl* ctrl,
                          hipStream_t st);
 hipError_t launch_dt(Ctrl* ctrl, hipStream_t st);
+// An FP64 array in the reference layout on the device, held in one or two
+// pieces: rows (v*n_p + m) below `split` at lo, the others at hi.
+struct RefRows {
+    double *lo, *hi;
+    int split;
+    __device__ double* row(int r, int K) const {
+        return r < split ? lo + (size_t)r * K : hi + (size_t)(r - split) * K;
+    }
+};
 // reference layout (FP64, caller's order) <-> state array in layout ix
 template <typename R>
-hipError_t launch_ref_to_state(const double* ref, R* dst, const int* perm, const StateIx& ix, int K, hipStream_t st);
+hipError_t launch_ref_to_state(const RefRows& ref, R* dst, const int* perm, const StateIx& ix, int K, hipStream_t st);
 template <typename R>
-hipError_t launch_state_to_ref(const R* src, double* ref, const int* perm, const StateIx& ix, int K, hipStream_t st);
+hipError_t launch_state_to_ref(const R* src, const RefRows& ref, const int* perm, const StateIx& ix, int K,
+                               hipStream_t st);
 hipError_t launch_set_dt(Ctrl* ctrl, double dt, int advance, hipStream_t st);
 template <typename R>
 hipError_t launch_project_ic(int p, R* c, const StateIx& ix, const double* V, int K, const IcP& ic, hipStream_t st);

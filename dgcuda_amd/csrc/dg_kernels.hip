@@ -389,7 +389,7 @@ template hipError_t launch_audit<double>(const double*, const StateIx&, const do
 // K-1's id.  One thread per (variable, internal element).
 // ---------------------------------------------------------------------------
 template <typename R>
-__global__ void __launch_bounds__(256) k_ref_to_state(const double* __restrict__ ref, R* __restrict__ dst,
+__global__ void __launch_bounds__(256) k_ref_to_state(RefRows ref, R* __restrict__ dst,
                                                      const int* __restrict__ perm, StateIx ix, int K) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= ix.N * ix.Kp) return;
@@ -397,35 +397,38 @@ __global__ void __launch_bounds__(256) k_ref_to_state(const double* __restrict__
     const size_t src = (size_t)perm[i];
     // every slot of the layout is written: padding modes hold zeros
     for (int m = 0; m < ix.slots(); m++)
-        dst[ix.at(v, m, i)] = m < ix.NP ? (R)ref[((size_t)v * ix.NP + m) * K + src] : R(0);
+        dst[ix.at(v, m, i)] = m < ix.NP ? (R)ref.row(v * ix.NP + m, K)[src] : R(0);
 }
 
 template <typename R>
-__global__ void __launch_bounds__(256) k_state_to_ref(const R* __restrict__ src, double* __restrict__ ref,
+__global__ void __launch_bounds__(256) k_state_to_ref(const R* __restrict__ src, RefRows ref,
                                                      const int* __restrict__ perm, StateIx ix, int K) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= ix.N * K) return;
     const int v = t / K, i = t - v * K;
     const size_t dst = (size_t)perm[i];
-    for (int m = 0; m < ix.NP; m++) ref[((size_t)v * ix.NP + m) * K + dst] = (double)src[ix.at(v, m, i)];
+    for (int m = 0; m < ix.NP; m++) ref.row(v * ix.NP + m, K)[dst] = (double)src[ix.at(v, m, i)];
 }
 
 template <typename R>
-hipError_t launch_ref_to_state(const double* ref, R* dst, const int* perm, const StateIx& ix, int K, hipStream_t st) {
+hipError_t launch_ref_to_state(const RefRows& ref, R* dst, const int* perm, const StateIx& ix, int K, hipStream_t st) {
     const int n = ix.N * ix.Kp;
     hipLaunchKernelGGL((k_ref_to_state<R>), dim3((n + 255) / 256), dim3(256), 0, st, ref, dst, perm, ix, K);
     return hipGetLastError();
 }
 template <typename R>
-hipError_t launch_state_to_ref(const R* src, double* ref, const int* perm, const StateIx& ix, int K, hipStream_t st) {
+hipError_t launch_state_to_ref(const R* src, const RefRows& ref, const int* perm, const StateIx& ix, int K,
+                               hipStream_t st) {
     const int n = ix.N * K;
     hipLaunchKernelGGL((k_state_to_ref<R>), dim3((n + 255) / 256), dim3(256), 0, st, src, ref, perm, ix, K);
     return hipGetLastError();
 }
-template hipError_t launch_ref_to_state<float>(const double*, float*, const int*, const StateIx&, int, hipStream_t);
-template hipError_t launch_ref_to_state<double>(const double*, double*, const int*, const StateIx&, int, hipStream_t);
-template hipError_t launch_state_to_ref<float>(const float*, double*, const int*, const StateIx&, int, hipStream_t);
-template hipError_t launch_state_to_ref<double>(const double*, double*, const int*, const StateIx&, int, hipStream_t);
+template hipError_t launch_ref_to_state<float>(const RefRows&, float*, const int*, const StateIx&, int, hipStream_t);
+template hipError_t launch_ref_to_state<double>(const RefRows&, double*, const int*, const StateIx&, int, hipStream_t);
+template hipError_t launch_state_to_ref<float>(const float*, const RefRows&, const int*, const StateIx&, int,
+                                               hipStream_t);
+template hipError_t launch_state_to_ref<double>(const double*, const RefRows&, const int*, const StateIx&, int,
+                                                hipStream_t);
 
 // Fill the constant-memory tables of every order from the FP64 host tables.
 template <typename R, int P>

