@@ -22,8 +22,8 @@ class BatchEngine {
     // persistent launches a stage runs.
     // Takes effect at the next set_slots.
     virtual void set_launch_form(int form) = 0;
-    // enqueues one step (per-solve dt + 4 stages) for every resident solve
-    virtual Status step(bool use_graph) = 0;
+    // enqueues n steps (per-solve dt + 4 stages) for every resident solve
+    virtual Status steps(int n, bool use_graph) = 0;
     // per slot: done flag, steps, t (waits for the engine's stream)
     virtual Status status(std::vector<double>& out) = 0;
     // every slot's control block, in one copy (waits for the engine's stream)

@@ -21,6 +21,7 @@
 #include <numeric>
 
 #include "dg_batch.h"
+#include "dg_step_graph.h"
 #include "dg_worklist.h"
 #include "dg_lane_body.h"
 #include "dg_mfma_body.h"
@@ -415,14 +416,14 @@ class EngineT : public BatchEngine {
     std::vector<double> raw_cost[BATCH_LISTS]; // each item's estimated cost
     std::vector<int2> h_items;       // host copy of the work lists and their XCD bounds
     std::vector<int> h_parts;
-    hipGraphExec_t gexec = nullptr;
+    StepGraph graph;
     int solo_min = 0;             // 0: every solve in the batch launch
     std::vector<Solver*> solo;    // solves launched with their own kernels
     std::vector<uint64_t> solo_uid;  // their ids: the captured step holds their buffers
 
     ~EngineT() override {
         if (st) (void)hipStreamSynchronize(st);
-        if (gexec) hipGraphExecDestroy(gexec);
+        graph.drop();
         void* b[] = {d_slots, d_items, d_xcd, d_status, d_ctrls};
         for (void* q : b)
             if (q) hipFree(q);
@@ -495,12 +496,7 @@ class EngineT : public BatchEngine {
         return Status::ok();
     }
 
-    void drop_graph() {
-        if (gexec) {
-            hipGraphExecDestroy(gexec);
-            gexec = nullptr;
-        }
-    }
+    void drop_graph() { graph.drop(); }
 
     void set_solo_threshold(int min_elems) override {
         if (min_elems != solo_min) drop_graph();
@@ -681,24 +677,11 @@ class EngineT : public BatchEngine {
         return Status::ok();
     }
 
-    Status step(bool use_graph) override {
-        if (!use_graph) return step_direct();
-        if (!gexec) {
-            hipGraph_t gr = nullptr;
-            HIPST(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-            Status s0 = step_direct();
-            hipError_t ee = hipStreamEndCapture(st, &gr);
-            if (!s0) {
-                if (gr) hipGraphDestroy(gr);
-                return s0;
-            }
-            HIPST(ee);
-            hipError_t ei = hipGraphInstantiate(&gexec, gr, nullptr, nullptr, 0);
-            hipGraphDestroy(gr);
-            HIPST(ei);
-        }
-        HIPST(hipGraphLaunch(gexec, st));
-        return Status::ok();
+    Status steps(int n, bool use_graph) override {
+        if (use_graph) return graph.run(st, n, [&] { return step_direct(); });
+        Status s0;
+        for (int i = 0; i < n && s0; i++) s0 = step_direct();
+        return s0;
     }
 
     Status status(std::vector<double>& out) override {
@@ -870,8 +853,7 @@ class BatchImpl : public Batch {
         if (!(cfl > 0) || nsteps < 0) return Status::err(DG_ERR_ARG, "invalid arguments");
         Status st = begin_all(false, cfl);
         if (!st) return st;
-        for (int i = 0; i < nsteps; i++)
-            if (!(st = eng->step(use_graph))) return st;
+        if (!(st = eng->steps(nsteps, use_graph))) return st;
         return finish_all();
     }
 
@@ -884,8 +866,7 @@ class BatchImpl : public Batch {
         int64_t issued = 0;
         int chunk = 8;
         while (true) {
-            for (int i = 0; i < chunk; i++)
-                if (!(st = eng->step(use_graph))) return st;
+            if (!(st = eng->steps(chunk, use_graph))) return st;
             issued += chunk;
             if (!(st = eng->status(h))) return st;
             bool all = true;

@@ -68,8 +68,19 @@ hipError_t copy_part(char* host, char* dev, size_t bytes, bool to_host, hipStrea
     void* blk[2] = {nullptr, nullptr};
     hipEvent_t ev[2] = {nullptr, nullptr};
     const size_t n = (bytes + COPY_BLOCK - 1) / COPY_BLOCK;
-    const int nb = n > 1 ? 2 : 1;
+    constexpr int nb = 2;
     hipError_t e = hipSuccess;
+    if (n == 1) {  // nothing to overlap: no events
+        if ((e = take_block(&blk[0])) != hipSuccess) return e;
+        if (!to_host) std::memcpy(blk[0], host, bytes);
+        e = to_host ? hipMemcpyAsync(blk[0], dev, bytes, hipMemcpyDeviceToHost, st)
+                    : hipMemcpyAsync(dev, blk[0], bytes, hipMemcpyHostToDevice, st);
+        const hipError_t es = hipStreamSynchronize(st);
+        if (e == hipSuccess) e = es;
+        if (to_host && e == hipSuccess) std::memcpy(host, blk[0], bytes);
+        give_block(blk[0]);
+        return e;
+    }
     for (int i = 0; i < nb && e == hipSuccess; i++) {
         e = take_block(&blk[i]);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming);

@@ -305,7 +305,7 @@ class ServerImpl : public Server {
                 }
                 changed = false;
             }
-            for (int i = 0; i < cfg.steps_per_round && st; i++) st = eng->step(cfg.use_graph != 0);
+            st = eng->steps(cfg.steps_per_round, cfg.use_graph != 0);
             if (st) st = eng->status(h);
             if (!st) {
                 fail_all(st.msg);

@@ -18,6 +18,7 @@
 
 #include "dg_hostcopy.h"
 #include "dg_solver.h"
+#include "dg_step_graph.h"
 
 namespace dgmi {
 
@@ -308,7 +309,7 @@ class SolverT : public Solver {
     int kernel_req = 0;
     int max_groups = 0;  // cap of the persistent matrix-core grid (0: every resident workgroup)
     bool lam_valid = false;
-    hipGraphExec_t gexec = nullptr;
+    StepGraph graph;       // the step of scheme graph_scheme
     int graph_scheme = 0;
     int64_t bytes = 0;
     int audit_blocks = 0;
@@ -322,7 +323,7 @@ class SolverT : public Solver {
 
     ~SolverT() override {
         if (stream) (void)hipStreamSynchronize(stream);  // nothing queued may use the buffers
-        if (gexec) (void)hipGraphExecDestroy(gexec);
+        graph.drop();
         void* bufs[] = {c,  acc,        ua,   ub,    geo_e, geo_f, nbr,     V,      Jd,
                         audit_part, ctrl, fword, halo,  face4, metric4, bnd, perm_d, lface, lmetric};
         for (void* b : bufs) pool_free(b);
@@ -664,10 +665,7 @@ class SolverT : public Solver {
         }
         shape = s;
         lam_valid = false;
-        if (gexec) {
-            hipGraphExecDestroy(gexec);
-            gexec = nullptr;
-        }
+        graph.drop();
         return Status::ok();
     }
 
@@ -761,33 +759,21 @@ class SolverT : public Solver {
         return stage(ST_RK4_4, ua, c, c);
     }
 
-    Status enqueue_cfl_step(int scheme, bool use_graph) {
-        if (use_graph) {
-            if (!gexec || graph_scheme != scheme) {
-                if (gexec) {
-                    hipGraphExecDestroy(gexec);
-                    gexec = nullptr;
-                }
-                hipGraph_t g = nullptr;
-                HIPST(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-                Status st = hip_status(launch_dt(ctrl, stream), "dt kernel");
-                if (st) st = enqueue_stages(scheme);
-                hipError_t ee = hipStreamEndCapture(stream, &g);
-                if (!st) {
-                    if (g) hipGraphDestroy(g);
-                    return st;
-                }
-                HIPST(ee);
-                hipError_t ei = hipGraphInstantiate(&gexec, g, nullptr, nullptr, 0);
-                hipGraphDestroy(g);
-                HIPST(ei);
-                graph_scheme = scheme;
-            }
-            HIPST(hipGraphLaunch(gexec, stream));
-            return Status::ok();
-        }
+    // one step: its dt, then its stages
+    Status enqueue_cfl_step(int scheme) {
         HIPST(launch_dt(ctrl, stream));
         return enqueue_stages(scheme);
+    }
+
+    Status enqueue_cfl_steps(int n, int scheme, bool use_graph) {
+        Status st;
+        if (use_graph) {
+            if (graph_scheme != scheme) graph.drop();
+            graph_scheme = scheme;
+            return graph.run(stream, n, [&] { return enqueue_cfl_step(scheme); });
+        }
+        for (int i = 0; i < n && st; i++) st = enqueue_cfl_step(scheme);
+        return st;
     }
 
     Status begin_run(double t_end, bool has_end, double cfl, hipStream_t on = nullptr) {
@@ -960,8 +946,7 @@ class SolverT : public Solver {
         if (!st) return st;
         int chunk = 8;
         while (true) {
-            for (int i = 0; i < chunk; i++)
-                if (!(st = enqueue_cfl_step(scheme, true))) return st;
+            if (!(st = enqueue_cfl_steps(chunk, scheme, true))) return st;
             if (!(st = pull_ctrl())) return st;
             if (hctrl.done || !(hctrl.t < t_end)) break;
             chunk = std::min(chunk * 2, 64);
@@ -977,8 +962,7 @@ class SolverT : public Solver {
         if (!(cfl > 0)) return Status::err(DG_ERR_ARG, "cfl must be positive");
         Status st = begin_run(0.0, false, cfl);
         if (!st) return st;
-        for (int i = 0; i < nsteps; i++)
-            if (!(st = enqueue_cfl_step(scheme, use_graph))) return st;
+        if (!(st = enqueue_cfl_steps(nsteps, scheme, use_graph))) return st;
         if (!(st = pull_ctrl())) return st;
         t = hctrl.t;
         steps = hctrl.steps;
@@ -1035,7 +1019,7 @@ class SolverT : public Solver {
         HIPST(hipEventCreate(&e0));
         HIPST(hipEventCreate(&e1));
         HIPST(hipEventRecord(e0, stream));
-        for (int i = 0; i < nsteps && st; i++) st = enqueue_cfl_step(DG_RK4, true);
+        st = enqueue_cfl_steps(nsteps, DG_RK4, true);
         float ms = 0.f;
         hipError_t e = hipEventRecord(e1, stream);
         if (e == hipSuccess) e = hipEventSynchronize(e1);
