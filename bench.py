@@ -324,8 +324,8 @@ def main():
     t_reached = s.audit()["t"]
 
     # dominant kernel: the fused stage kernel.  Its live duration comes from
-    # the timed region's events: ms per replayed step, less the dt kernel
-    # (timed per launch), over the 4 stage launches of a step.  Event pairs
+    # the timed region's events: ms per replayed step over its 4 stage
+    # launches (the first computes dt: no launch of its own).  Event pairs
     # around each directly launched stage (stage_ms_direct) separate the
     # kernels and read longer.
     tk = s.time_stage_kernels(20, 0.3)

@@ -130,6 +130,7 @@ __device__ __forceinline__ StageArgs<R> slot_args(const SlotDesc<R>* sd) {
     a.ntiles = 0;
     a.xcd_remap = 0;
     a.stream = 0;
+    a.in_step = 0;  // k_batch_dt starts the step
     a.bnd = nullptr;  // batched solves have no boundary sides
     a.phys.gamma = uni(sd->phys.gamma);
     a.phys.ax = uni(sd->phys.ax);
@@ -212,11 +213,13 @@ __device__ __forceinline__ void batch_lane_items(const SlotDesc<R>* __restrict__
         const int N = uni(sd->N), p = uni(sd->p);
         const int e = uni(item.y) * BATCH_VALU_TILE + threadIdx.x;
         double lam = 0.0;
+        const auto go = [] { return true; };  // asked above
+        const auto dt = [&] { return (R)a.ctrl->dt; };
         if constexpr (EUL) {
             // with the non-temporal hint: 1-2% faster per step than without
             // on ragged batches of 24, 32 and 64 solves
-            if (N == 4 && p == 2) lam = lane_process<2, KIND, R, false, true>(a, e, lt2);
-            else if (N == 4 && p == 1) lam = lane_process<1, KIND, R, false, true>(a, e, lt1);
+            if (N == 4 && p == 2) lam = lane_process<2, KIND, R, false, true>(a, e, lt2, go, dt);
+            else if (N == 4 && p == 1) lam = lane_process<1, KIND, R, false, true>(a, e, lt1, go, dt);
         }
         if constexpr (ADV) {
             if (N == 1 && p == 2) lam = valu_process<1, 2, R>(a, e, KIND);
@@ -224,7 +227,7 @@ __device__ __forceinline__ void batch_lane_items(const SlotDesc<R>* __restrict__
         }
         if constexpr (LAST) {
             const double m = block_max(lam, sh);
-            if (threadIdx.x == 0) lam_commit(m, a.lam_bits);
+            if (threadIdx.x == 0) lam_commit_step(m, a.ctrl);
             __syncthreads();  // sh is reused by the next item
         }
     }
@@ -267,7 +270,7 @@ __device__ __forceinline__ void batch_tile_items(const SlotDesc<R>* __restrict__
         it = next;
         if constexpr (LAST) {
             const double m = block_max(lam, sh);
-            if (threadIdx.x == 0) lam_commit(m, a.lam_bits);
+            if (threadIdx.x == 0) lam_commit_step(m, a.ctrl);
             __syncthreads();  // sh is reused by the next run
         }
     }

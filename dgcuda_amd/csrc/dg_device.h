@@ -87,6 +87,7 @@ struct Ctrl {
     int done;        // t reached t_end
     int has_end;     // clamp to t_end
     int pad;
+    double t_next;   // time after the step whose first stage computed its dt
 };
 
 // Maximum cell wave speed of the current state: LAM_SLOTS partial maxima
@@ -99,10 +100,33 @@ struct Ctrl {
 // triangles, a step of 4 stages 167 us; with 64 slots 133 us).
 constexpr int LAM_SLOTS = 64;
 constexpr int LAM_STRIDE = 8;     // 64 bytes apart
-constexpr size_t CTRL_LAM_AT = 256;  // byte offset of the slots behind a solve's control block
-constexpr size_t CTRL_BYTES = CTRL_LAM_AT + LAM_SLOTS * LAM_STRIDE * sizeof(unsigned long long);
-static_assert(sizeof(Ctrl) <= CTRL_LAM_AT, "the wave-speed slots follow the control block");
+// Device-only words behind the control block (the host never writes them
+// after set-up): two sides of slots, which of them holds the wave speed of
+// the current state, and which the current step's last stage commits to.
+constexpr size_t CTRL_SIDE_AT = 192;
+constexpr size_t CTRL_LAM_AT = 256;
+constexpr int LAM_SIDE = LAM_SLOTS * LAM_STRIDE;  // words of one side
+constexpr size_t CTRL_BYTES = CTRL_LAM_AT + 2 * LAM_SIDE * sizeof(unsigned long long);
+static_assert(sizeof(Ctrl) <= CTRL_SIDE_AT, "the wave-speed words follow the control block");
 
+// View of the control block for words that no workgroup of the running launch
+// writes (or writes only to what every reader concludes anyway): scalar loads.
+#ifdef __HIP__
+#define DG_CONST_VIEW __attribute__((address_space(4)))
+#else  // a host build of these headers
+#define DG_CONST_VIEW
+#endif
+template <typename T>
+__device__ __forceinline__ const DG_CONST_VIEW T* cview(const T* p) {
+    return (const DG_CONST_VIEW T*)p;
+}
+
+struct LamSide {
+    int current, commit;
+};
+__host__ __device__ inline LamSide* lam_side(Ctrl* ctrl) {
+    return reinterpret_cast<LamSide*>(reinterpret_cast<char*>(ctrl) + CTRL_SIDE_AT);
+}
 __host__ __device__ inline unsigned long long* lam_slots(Ctrl* ctrl) {
     return reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(ctrl) + CTRL_LAM_AT);
 }
@@ -111,52 +135,111 @@ __device__ __forceinline__ void lam_commit(double mx, unsigned long long* slots)
     if (mx > 0.0)
         atomicMax(slots + (blockIdx.x & (LAM_SLOTS - 1)) * LAM_STRIDE, (unsigned long long)__double_as_longlong(mx));
 }
+// last stage: commits to the side its step names
+__device__ __forceinline__ void lam_commit_step(double mx, Ctrl* ctrl) {
+    lam_commit(mx, lam_slots(ctrl) + cview(lam_side(ctrl))->commit * LAM_SIDE);
+}
 
-// The maximum over the slots (every lane of one wavefront calls it).
-__device__ __forceinline__ double lam_reduce(const unsigned long long* slots) {
-    double v = __longlong_as_double((long long)slots[(threadIdx.x & (LAM_SLOTS - 1)) * LAM_STRIDE]);
+// this lane's slot of a side, and the maximum over a wavefront's slots
+__device__ __forceinline__ double lam_slot(const unsigned long long* side) {
+    return __longlong_as_double((long long)side[(threadIdx.x & (LAM_SLOTS - 1)) * LAM_STRIDE]);
+}
+__device__ __forceinline__ double lam_reduce(double v) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
     return v;
 }
+__device__ __forceinline__ void lam_clear(unsigned long long* side) {
+    side[(threadIdx.x & (LAM_SLOTS - 1)) * LAM_STRIDE] = 0ull;
+}
 
 // Start of a step on the device: dt = cfl * min_r / max lambda / (2p+1),
-// clamped to t_end, t advanced before the stages (time_integrator.cu:254-270);
-// reduces the accumulated wave speeds and clears them for the step's last
-// stage to fill.  A step not taken (t_end reached) leaves them: they still
-// hold the wave speed of the current state, which a later run starts from.
-// One wavefront.
+// clamped to t_end, t advanced before the stages (time_integrator.cu:254-270).
+// A step not taken (t_end reached) leaves the wave speeds: they still hold
+// the current state's, which a later run starts from.
+__device__ __forceinline__ bool step_not_taken(Ctrl* c) {
+    const auto* ctrl = cview(c);
+    return ctrl->done || (ctrl->has_end && !(ctrl->t < ctrl->t_end));
+}
+__device__ __forceinline__ void step_stop(Ctrl* ctrl) {  // one thread
+    ctrl->active = 0;
+    if (!ctrl->done) {
+        ctrl->done = 1;
+        ctrl->dt = 0.0;
+    }
+}
+__device__ __forceinline__ double step_size(Ctrl* c, double mx, double* t_next) {
+    const auto* ctrl = cview(c);
+    const double t = ctrl->t, dt = ctrl->cfl * ctrl->min_r / mx / ctrl->two_p1;
+    if (ctrl->has_end && t + dt > ctrl->t_end) {
+        *t_next = ctrl->t_end;
+        return ctrl->t_end - t;
+    }
+    *t_next = t + dt;
+    return dt;
+}
+
+// The step's start as a kernel of its own (batches).  One wavefront.
 __device__ __forceinline__ void dt_update(Ctrl* ctrl) {
     const bool first = (threadIdx.x & 63) == 0;
-    if (ctrl->done) {
-        if (first) ctrl->active = 0;
+    if (step_not_taken(ctrl)) {
+        if (first) step_stop(ctrl);
         return;
     }
-    double t = ctrl->t;
-    if (ctrl->has_end && !(t < ctrl->t_end)) {
-        if (first) {
-            ctrl->active = 0;
-            ctrl->done = 1;
-            ctrl->dt = 0.0;
-        }
-        return;
-    }
-    unsigned long long* slots = lam_slots(ctrl);
-    const double mx = lam_reduce(slots);
-    slots[(threadIdx.x & (LAM_SLOTS - 1)) * LAM_STRIDE] = 0ull;
+    const int side = lam_side(ctrl)->current;
+    unsigned long long* slots = lam_slots(ctrl) + side * LAM_SIDE;
+    const double mx = lam_reduce(lam_slot(slots));
+    lam_clear(slots);
     if (!first) return;
-    double dt = ctrl->cfl * ctrl->min_r / mx / ctrl->two_p1;
-    if (ctrl->has_end && t + dt > ctrl->t_end) {
-        dt = ctrl->t_end - t;
-        t = ctrl->t_end;
-    } else {
-        t += dt;
-    }
+    double t;
+    ctrl->dt = step_size(ctrl, mx, &t);
     ctrl->lam_bits = (unsigned long long)__double_as_longlong(mx);
-    ctrl->dt = dt;
     ctrl->t = t;
     ctrl->steps += 1;
     ctrl->active = 1;
+    lam_side(ctrl)->commit = side;
+}
+
+// The step's start inside its first stage (StageArgs::in_step), where a
+// launch of its own and a wait before every stage's loads took 3-5 us of a
+// step: advection p = 1 FP64 on 2,048 triangles 20.2 -> 18.3 us, Euler p = 2
+// FP64 32,768 52.3 -> 50.9, p = 1 FP32 500,000 85.7 -> 82.7, p = 4 FP32
+// 524,288 381 -> 370, p = 3 FP64 131,072 230 -> 226.  Every
+// workgroup computes the same dt from words that no workgroup of this launch
+// writes (t, done, the current side of the wave speeds), and the launch's
+// first wavefront notes it for the later stages and clears the other side,
+// which the last stage commits to; the last stage then moves t, the step
+// count and the current side on (step_finish).  The slot is requested early
+// (`slot`) and reduced where dt is used, so the loads in between are not held up.
+struct StepSlot {
+    double v[2];  // this lane's slot of either side: requested without waiting for which is current
+};
+__device__ __forceinline__ StepSlot step_slot(Ctrl* ctrl) {
+    const unsigned long long* s = lam_slots(ctrl);
+    return StepSlot{{lam_slot(s), lam_slot(s + LAM_SIDE)}};
+}
+__device__ __forceinline__ double step_start(Ctrl* ctrl, const StepSlot& slot) {
+    const int side = cview(lam_side(ctrl))->current;
+    const double mx = lam_reduce(side ? slot.v[1] : slot.v[0]);
+    double t;
+    const double dt = step_size(ctrl, mx, &t);
+    if (blockIdx.x == 0 && threadIdx.x < 64) {
+        lam_clear(lam_slots(ctrl) + (1 - side) * LAM_SIDE);
+        if (threadIdx.x == 0) {
+            ctrl->dt = dt;
+            ctrl->t_next = t;
+            ctrl->lam_bits = (unsigned long long)__double_as_longlong(mx);
+            ctrl->active = 1;
+            lam_side(ctrl)->commit = 1 - side;
+        }
+    }
+    return dt;
+}
+// last stage, first workgroup: one thread
+__device__ __forceinline__ void step_finish(Ctrl* ctrl) {
+    ctrl->t = ctrl->t_next;
+    ctrl->steps += 1;
+    lam_side(ctrl)->current = lam_side(ctrl)->commit;
 }
 
 struct PhysP {
@@ -320,12 +403,13 @@ struct StageArgs {
     const R* geo_e;   // [5][Kp]: xr, yr, xs, ys, J
     const R* geo_f;   // [9][Kp]: (nx, ny, len) for faces 0..2
     const int* nbr;   // [3][Kp]
-    const Ctrl* ctrl;
-    unsigned long long* lam_bits; // lam_slots(ctrl) (last stage)
+    Ctrl* ctrl;
+    unsigned long long* lam_bits; // lam_slots(ctrl)
     int K, Kp;        // elements, and the padded count (multiple of 64) of every [..][Kp] array
     int kind;
     int ntiles;       // tiles (workgroups) that carry elements
     int xcd_remap;    // map consecutive tiles to one XCD
+    int in_step;      // the step's first stage computes its dt (step_start), the last ends it (step_finish)
     int stream;       // vector layout: the solve's arrays exceed the memory-side cache
     PhysP phys;
     // ST_RHS_REF: input and output [N][n_p][K] in the caller's element order,
@@ -346,6 +430,40 @@ struct StageArgs {
     // reflecting points; null for a mesh without boundary sides
     const double* bnd;
 };
+
+__host__ __device__ constexpr bool first_stage(int kind) { return kind == ST_RK4_1 || kind == ST_RK2_1; }
+__host__ __device__ constexpr bool last_stage(int kind) { return kind == ST_RK4_4 || kind == ST_RK2_2; }
+
+// A stage launch's view of its step.  Constructed before the stage's first
+// loads and asked (active) behind them, so that neither waits for the other.
+template <typename R>
+struct StageStep {
+    const StageArgs<R>& a;
+    const bool start;  // this launch starts the step
+    StepSlot slot;
+    __device__ __forceinline__ StageStep(const StageArgs<R>& args, int kind)
+        : a(args), start(first_stage(kind) && args.in_step), slot{} {
+        if (start) slot = step_slot(a.ctrl);
+    }
+    // whether the launch has work (uniform); notes a step not taken
+    __device__ __forceinline__ bool active() const {
+        if (!start) return cview(a.ctrl)->active != 0;
+        if (!step_not_taken(a.ctrl)) return true;
+        if (blockIdx.x == 0 && threadIdx.x == 0) step_stop(a.ctrl);
+        return false;
+    }
+    // the stage's dt (every lane of a wavefront calls it)
+    __device__ __forceinline__ R dt() const { return (R)(start ? step_start(a.ctrl, slot) : cview(a.ctrl)->dt); }
+};
+// keeps loads that come before it before it
+#define DG_LOADS_FIRST() asm volatile("" ::: "memory")
+
+// End of the last stage's launch: the wave speeds, and the step's end.
+template <typename R>
+__device__ __forceinline__ void stage_commit(const StageArgs<R>& a, double mx) {  // one thread per workgroup
+    lam_commit_step(mx, a.ctrl);
+    if (a.in_step && blockIdx.x == 0) step_finish(a.ctrl);
+}
 
 // caller's element of element e
 template <typename R>

@@ -150,7 +150,6 @@ constexpr int VALU_TILE_ELEMS = 128;
 template <typename R>
 hipError_t launch_lambda(const R* u, const StateIx& ix, int K, double b0, const PhysP& ph, Ctrl* ctrl,
                          hipStream_t st);
-hipError_t launch_dt(Ctrl* ctrl, hipStream_t st);
 // An FP64 array in the reference layout on the device, held in one or two
 // pieces: rows (v*n_p + m) below `split` at lo, the others at hi.
 struct RefRows {

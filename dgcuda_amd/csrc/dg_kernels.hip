@@ -32,14 +32,16 @@ __global__ void __launch_bounds__(128) k_stage_valu(StageArgs<R> a) {
         if (t < a.ntiles) valu_process<N, P, R, BND, true>(a, t * blockDim.x + threadIdx.x, ST_RHS);
         return;
     }
-    if (!a.ctrl->active) return;
+    const int kind = a.kind;
+    const StageStep<R> step(a, kind);
+    if (!step.active()) return;
     const int tile = tile_of_block(blockIdx.x, gridDim.x, a.xcd_remap);
     if (tile >= a.ntiles) return;
-    const int kind = a.kind;
-    const double lam = valu_process<N, P, R, BND>(a, tile * blockDim.x + threadIdx.x, kind);
-    if (kind == ST_RK4_4 || kind == ST_RK2_2) {
+    const double lam =
+        valu_process<N, P, R, BND, false>(a, tile * blockDim.x + threadIdx.x, kind, [&] { return step.dt(); });
+    if (last_stage(kind)) {
         const double mx = block_max(lam, sh);
-        if (threadIdx.x == 0) lam_commit(mx, a.lam_bits);
+        if (threadIdx.x == 0) stage_commit(a, mx);
     }
 }
 
@@ -55,17 +57,21 @@ constexpr int lane_minw() {
 template <int P, int KIND, typename R, bool BND, bool NT>
 __global__ void __launch_bounds__(128, (lane_minw<P, R>())) k_stage_lane(StageArgs<R> a) {
     __shared__ double sh[8];
-    if constexpr (KIND != ST_RHS_REF)
-        if (!a.ctrl->active) return;
+    __shared__ __align__(16) R ltab[LaneTab<P>::SIZE];
     const int tile = tile_of_block(blockIdx.x, gridDim.x, a.xcd_remap);
     if (tile >= a.ntiles) return;
-    __shared__ __align__(16) R ltab[LaneTab<P>::SIZE];
-    LaneTab<P>::fill(ltab, threadIdx.x, blockDim.x);
-    __syncthreads();
-    const double lam = lane_process<P, KIND, R, BND, NT>(a, tile * blockDim.x + threadIdx.x, ltab);
-    if constexpr (KIND == ST_RK4_4 || KIND == ST_RK2_2) {
+    const StageStep<R> step(a, KIND);
+    const auto gate = [&] {
+        LaneTab<P>::fill(ltab, threadIdx.x, blockDim.x);
+        __syncthreads();
+        return KIND == ST_RHS_REF || step.active();
+    };
+    const double lam = lane_process<P, KIND, R, BND, NT>(a, tile * blockDim.x + threadIdx.x, ltab, gate,
+                                                         [&] { return step.dt(); });
+    if (lam < 0.0) return;  // inactive: every lane of the launch
+    if constexpr (last_stage(KIND)) {
         const double mx = block_max(lam, sh);
-        if (threadIdx.x == 0) lam_commit(mx, a.lam_bits);
+        if (threadIdx.x == 0) stage_commit(a, mx);
     }
 }
 
@@ -105,8 +111,7 @@ template hipError_t launch_lane_pack<double>(const double*, const double*, const
 // Maximum cell wave speed of a state without stepping it (first step of a
 // run, dg_cfl_dt): grid-stride over elements, workgroup max, one atomic max.
 template <int N, typename R>
-__global__ void __launch_bounds__(256) k_lambda(const R* u, StateIx ix, int K, double b0, PhysP ph,
-                                               unsigned long long* lam_bits) {
+__global__ void __launch_bounds__(256) k_lambda(const R* u, StateIx ix, int K, double b0, PhysP ph, Ctrl* ctrl) {
     __shared__ double sh[8];
     double mx = 0.0;
     for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < K; e += gridDim.x * blockDim.x) {
@@ -116,25 +121,21 @@ __global__ void __launch_bounds__(256) k_lambda(const R* u, StateIx ix, int K, d
         mx = fmax(mx, cell_speed<N>(ph, U));
     }
     mx = block_max(mx, sh);
-    if (threadIdx.x == 0) lam_commit(mx, lam_bits);
+    if (threadIdx.x == 0) lam_commit(mx, lam_slots(ctrl) + lam_side(ctrl)->current * LAM_SIDE);
 }
 
 __global__ void k_reset_lam(Ctrl* ctrl) {
-    lam_slots(ctrl)[threadIdx.x * LAM_STRIDE] = 0ull;  // LAM_SLOTS threads
-}
-
-// dt = cfl * min_r / max lambda / (2p+1), clamped to t_end
-// (time_integrator.cu:254-270); reads and clears the accumulated maximum.
-__global__ void k_dt(Ctrl* ctrl) {
-    dt_update(ctrl);  // one wavefront
+    lam_clear(lam_slots(ctrl) + lam_side(ctrl)->current * LAM_SIDE);  // LAM_SLOTS threads
 }
 
 // host-chosen step: activate the stages with the given dt
 __global__ void k_set_dt(Ctrl* ctrl, double dt, int advance) {
-    lam_slots(ctrl)[threadIdx.x * LAM_STRIDE] = 0ull;  // LAM_SLOTS threads
+    const int side = lam_side(ctrl)->current;
+    lam_clear(lam_slots(ctrl) + side * LAM_SIDE);  // LAM_SLOTS threads
     if (threadIdx.x == 0) {
         ctrl->dt = dt;
         ctrl->active = 1;
+        lam_side(ctrl)->commit = side;
         if (advance) {
             ctrl->t += dt;
             ctrl->steps += 1;
@@ -319,22 +320,16 @@ hipError_t launch_lambda(const R* u, const StateIx& ix, int K, double b0, const 
                          hipStream_t st) {
     hipLaunchKernelGGL(k_reset_lam, dim3(1), dim3(LAM_SLOTS), 0, st, ctrl);
     const dim3 grid(std::min((K + 255) / 256, 2048));
-    unsigned long long* bits = lam_slots(ctrl);
     if (ix.N == 1)
-        hipLaunchKernelGGL((k_lambda<1, R>), grid, dim3(256), 0, st, u, ix, K, b0, ph, bits);
+        hipLaunchKernelGGL((k_lambda<1, R>), grid, dim3(256), 0, st, u, ix, K, b0, ph, ctrl);
     else
-        hipLaunchKernelGGL((k_lambda<4, R>), grid, dim3(256), 0, st, u, ix, K, b0, ph, bits);
+        hipLaunchKernelGGL((k_lambda<4, R>), grid, dim3(256), 0, st, u, ix, K, b0, ph, ctrl);
     return hipGetLastError();
 }
 template hipError_t launch_lambda<float>(const float*, const StateIx&, int, double, const PhysP&, Ctrl*,
                                          hipStream_t);
 template hipError_t launch_lambda<double>(const double*, const StateIx&, int, double, const PhysP&, Ctrl*,
                                           hipStream_t);
-
-hipError_t launch_dt(Ctrl* ctrl, hipStream_t st) {
-    hipLaunchKernelGGL(k_dt, dim3(1), dim3(64), 0, st, ctrl);
-    return hipGetLastError();
-}
 
 hipError_t launch_set_dt(Ctrl* ctrl, double dt, int advance, hipStream_t st) {
     hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(LAM_SLOTS), 0, st, ctrl, dt, advance);

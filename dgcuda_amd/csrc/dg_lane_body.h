@@ -158,10 +158,13 @@ struct LaneTab {
 
 // Processes element e (clamped for loads when past the mesh, no stores
 // then) of RK stage KIND; returns its cell wave speed after the last stage
-// of a step, else 0.  BND: the variant for meshes with boundary sides;
+// of a step, else 0, or -1 if `gate` (asked once the element's own loads are
+// requested; it also makes `ltab` ready) finds the stage inactive.  stage_dt
+// gives the stage's dt where it is used.  BND: the variant for meshes with boundary sides;
 // without it the face loop carries no branch.
-template <int P, int KIND, typename R, bool BND, bool NT>
-__device__ __forceinline__ double lane_process(const StageArgs<R>& a, int e, const R* ltab) {
+template <int P, int KIND, typename R, bool BND, bool NT, typename GATE, typename DT>
+__device__ __forceinline__ double lane_process(const StageArgs<R>& a, int e, const R* ltab, const GATE& gate,
+                                               const DT& stage_dt) {
     using L = LaneV<R>;
     using V = typename L::V;
     using G4 = typename L::G;
@@ -189,6 +192,8 @@ __device__ __forceinline__ double lane_process(const StageArgs<R>& a, int e, con
     load(ee, u);
     const G4 me = ((const DG_GLOBAL G4*)a.lmetric)[ee];
     const R ij = gp(a.geo_e)[4 * (size_t)Kp + ee];
+    DG_LOADS_FIRST();
+    if (!gate()) return -1.0;
 
     int wd[3], nb[3];
 #pragma unroll
@@ -311,7 +316,7 @@ __device__ __forceinline__ double lane_process(const StageArgs<R>& a, int e, con
         }
         return 0.0;
     }
-    const R cj = ij * (R)a.ctrl->dt;
+    const R cj = ij * stage_dt();
     double lam = 0.0;
     V o[NP][NG], w[NP][NG];
 #pragma unroll

@@ -84,8 +84,7 @@ __global__ void __launch_bounds__(256, (mfma_minw<R, KIND>())) k_stage_mfma(Stag
     __shared__ double shmax[8];
 
     constexpr bool REF = KIND == ST_RHS_REF;
-    if constexpr (!REF)
-        if (!a.ctrl->active) return;
+    const StageStep<R> step(a, KIND);
     const int ntiles = a.ntiles;
     int t, tend, stride;
     if (a.xcd_remap) {
@@ -102,11 +101,6 @@ __global__ void __launch_bounds__(256, (mfma_minw<R, KIND>())) k_stage_mfma(Stag
     const int g = lane >> 4, j = lane & 15;
     double lam = 0.0;
     __shared__ V tabA[MFMA_A_SLOTS * 64];
-    R dt;
-    if constexpr (REF)
-        dt = (R)a.ref_dt;
-    else
-        dt = (R)a.ctrl->dt;
     MfmaTileState<N, P, R, REF> st;
     int hid[MfmaTileState<N, P, R>::HPW];
     TileGeo<R> gc;
@@ -120,6 +114,14 @@ __global__ void __launch_bounds__(256, (mfma_minw<R, KIND>())) k_stage_mfma(Stag
         MfmaTileState<N, P, R>::load_ids(mx.halo, mx.hcap, walk(t + stride), w, j, hid);
     }
     if (w == 0) mfma_a_to_lds<N, P, R>(tabA, lane);
+    DG_LOADS_FIRST();
+    R dt;
+    if constexpr (REF) {
+        dt = (R)a.ref_dt;
+    } else {
+        if (!step.active()) return;
+        dt = step.dt();
+    }
     // The first tile needs these loads at once.  Waiting for them here also
     // keeps the compiler's count of loads in flight at the loop head to the
     // steady state (loop back edge), where the next tile's operands were
@@ -132,7 +134,7 @@ __global__ void __launch_bounds__(256, (mfma_minw<R, KIND>())) k_stage_mfma(Stag
 
     if constexpr (LAST) {
         const double m2 = block_max(lam, shmax);
-        if (threadIdx.x == 0) lam_commit(m2, a.lam_bits);
+        if (threadIdx.x == 0) stage_commit(a, m2);
     }
 }
 

@@ -681,7 +681,7 @@ class SolverT : public Solver {
     }
 
     // arguments of every stage launch
-    StageArgs<R> stage_args(int kind) {
+    StageArgs<R> stage_args(int kind, bool in_step = false) {
         StageArgs<R> a{};
         a.acc = acc;
         a.geo_e = geo_e;
@@ -694,6 +694,7 @@ class SolverT : public Solver {
         a.kind = kind;
         a.ntiles = shape.ntiles;
         a.xcd_remap = shape.xcd_remap;
+        a.in_step = in_step ? 1 : 0;
         a.stream = stream_hint();
         a.phys = phys;
         a.lface = lface;
@@ -711,8 +712,8 @@ class SolverT : public Solver {
         return hip_status(e, "stage kernel launch");
     }
 
-    Status stage(int kind, const R* u, const R* cc, R* out, hipStream_t on = nullptr) {
-        StageArgs<R> a = stage_args(kind);
+    Status stage(int kind, const R* u, const R* cc, R* out, hipStream_t on = nullptr, bool in_step = false) {
+        StageArgs<R> a = stage_args(kind, in_step);
         a.u = u;
         a.c = cc;
         a.out = out;
@@ -746,23 +747,18 @@ class SolverT : public Solver {
         return Status::ok();
     }
 
-    // the stages of one step; the step's dt is already in ctrl
-    Status enqueue_stages(int scheme) {
+    // The stages of one step.  in_step: the first computes the step's dt and
+    // the last ends it (step_start, step_finish), else both are done already.
+    Status enqueue_stages(int scheme, bool in_step) {
         Status st;
         if (scheme == DG_RK2) {
-            if (!(st = stage(ST_RK2_1, c, c, ua))) return st;
-            return stage(ST_RK2_2, ua, c, c);
+            if (!(st = stage(ST_RK2_1, c, c, ua, nullptr, in_step))) return st;
+            return stage(ST_RK2_2, ua, c, c, nullptr, in_step);
         }
-        if (!(st = stage(ST_RK4_1, c, c, ua))) return st;
+        if (!(st = stage(ST_RK4_1, c, c, ua, nullptr, in_step))) return st;
         if (!(st = stage(ST_RK4_2, ua, c, ub))) return st;
         if (!(st = stage(ST_RK4_3, ub, c, ua))) return st;
-        return stage(ST_RK4_4, ua, c, c);
-    }
-
-    // one step: its dt, then its stages
-    Status enqueue_cfl_step(int scheme) {
-        HIPST(launch_dt(ctrl, stream));
-        return enqueue_stages(scheme);
+        return stage(ST_RK4_4, ua, c, c, nullptr, in_step);
     }
 
     Status enqueue_cfl_steps(int n, int scheme, bool use_graph) {
@@ -770,9 +766,9 @@ class SolverT : public Solver {
         if (use_graph) {
             if (graph_scheme != scheme) graph.drop();
             graph_scheme = scheme;
-            return graph.run(stream, n, [&] { return enqueue_cfl_step(scheme); });
+            return graph.run(stream, n, [&] { return enqueue_stages(scheme, true); });
         }
-        for (int i = 0; i < n && st; i++) st = enqueue_cfl_step(scheme);
+        for (int i = 0; i < n && st; i++) st = enqueue_stages(scheme, true);
         return st;
     }
 
@@ -916,7 +912,7 @@ class SolverT : public Solver {
     Status rk_step(double dt, int scheme) override {
         if (scheme != DG_RK4 && scheme != DG_RK2) return Status::err(DG_ERR_ARG, "scheme must be DG_RK4 or DG_RK2");
         HIPST(launch_set_dt(ctrl, dt, 1, stream));
-        Status st = enqueue_stages(scheme);
+        Status st = enqueue_stages(scheme, false);
         if (!st) return st;
         lam_valid = true;  // the last stage left the new state's wave speeds
         HIPST(hipStreamSynchronize(stream));
@@ -928,9 +924,12 @@ class SolverT : public Solver {
     Status cfl_dt(double cfl, double* dt) override {
         Status st = ensure_lambda();
         if (!st) return st;
-        unsigned long long slots[LAM_SLOTS * LAM_STRIDE], bits = 0;
-        HIPST(hipMemcpyAsync(slots, lam_slots(ctrl), sizeof(slots), hipMemcpyDeviceToHost, stream));
+        std::vector<char> h(CTRL_BYTES);
+        HIPST(hipMemcpyAsync(h.data(), ctrl, h.size(), hipMemcpyDeviceToHost, stream));
         HIPST(hipStreamSynchronize(stream));
+        Ctrl* hc = reinterpret_cast<Ctrl*>(h.data());
+        const unsigned long long* slots = lam_slots(hc) + lam_side(hc)->current * LAM_SIDE;
+        unsigned long long bits = 0;
         for (int i = 0; i < LAM_SLOTS; i++) bits = std::max(bits, slots[i * LAM_STRIDE]);
         double mx;
         std::memcpy(&mx, &bits, sizeof(mx));
@@ -1041,42 +1040,34 @@ class SolverT : public Solver {
         Status st = begin_run(0.0, false, cfl);
         if (!st) return st;
         const int nst = 4 * nsteps;
-        std::vector<hipEvent_t> ev(2 * nst + 2 * nsteps + 2);
+        std::vector<hipEvent_t> ev(2 * nst + 2);
         for (auto& e : ev) HIPST(hipEventCreate(&e));
         int k = 0;
-        HIPST(hipEventRecord(ev[2 * nst + 2 * nsteps], stream));
+        HIPST(hipEventRecord(ev[2 * nst], stream));
         for (int s = 0; s < nsteps; s++) {
-            HIPST(hipEventRecord(ev[2 * nst + 2 * s], stream));
-            HIPST(launch_dt(ctrl, stream));
-            HIPST(hipEventRecord(ev[2 * nst + 2 * s + 1], stream));
             const int kinds[4] = {ST_RK4_1, ST_RK4_2, ST_RK4_3, ST_RK4_4};
             const R* ins[4] = {c, ua, ub, ua};
             R* outs[4] = {ua, ub, ua, c};
             for (int j = 0; j < 4; j++) {
                 HIPST(hipEventRecord(ev[2 * k], stream));
-                if (!(st = stage(kinds[j], ins[j], c, outs[j]))) return st;
+                if (!(st = stage(kinds[j], ins[j], c, outs[j], nullptr, j == 0 || j == 3))) return st;
                 HIPST(hipEventRecord(ev[2 * k + 1], stream));
                 k++;
             }
         }
-        HIPST(hipEventRecord(ev[2 * nst + 2 * nsteps + 1], stream));
+        HIPST(hipEventRecord(ev[2 * nst + 1], stream));
         HIPST(hipStreamSynchronize(stream));
-        double sum = 0, sumdt = 0;
+        double sum = 0;
         for (int i = 0; i < nst; i++) {
             float ms = 0;
             HIPST(hipEventElapsedTime(&ms, ev[2 * i], ev[2 * i + 1]));
             sum += ms;
         }
-        for (int s = 0; s < nsteps; s++) {
-            float ms = 0;
-            HIPST(hipEventElapsedTime(&ms, ev[2 * nst + 2 * s], ev[2 * nst + 2 * s + 1]));
-            sumdt += ms;
-        }
         float tot = 0;
-        HIPST(hipEventElapsedTime(&tot, ev[2 * nst + 2 * nsteps], ev[2 * nst + 2 * nsteps + 1]));
+        HIPST(hipEventElapsedTime(&tot, ev[2 * nst], ev[2 * nst + 1]));
         for (auto& e : ev) hipEventDestroy(e);
         out[0] = sum / nst;
-        out[1] = sumdt / nsteps;
+        out[1] = 0.0;  // dt is computed in the first stage
         out[2] = tot;
         out[3] = nst;
         if (!(st = pull_ctrl())) return st;

@@ -35,19 +35,15 @@ __device__ __forceinline__ R face_phi(const TabP<R, P>& T, int f, int m, int j, 
 // without it the face loop carries no branch and the loads of the three
 // faces can be scheduled together.
 // REF: the right-hand side on the caller's arrays (ST_RHS_REF).
-template <int N, int P, typename R, bool BND = false, bool REF = false>
-__device__ __forceinline__ double valu_process(const StageArgs<R>& a, int e, int kind) {
+// stage_dt gives the stage's dt where it is used.
+template <int N, int P, typename R, bool BND, bool REF, typename DT>
+__device__ __forceinline__ double valu_process(const StageArgs<R>& a, int e, int kind, const DT& stage_dt) {
     static_assert(!BND || P <= VALU_BOUNDARY_MAX_P, "boundary sides are compiled for p <= VALU_BOUNDARY_MAX_P");
     constexpr int NP = n_modes(P), NQ = n_quad_vol(P), NQ1 = P + 1;
     const TabP<R, P>& T = tab<R, P>();
     const bool valid = e < a.K;
     const int ee = valid ? e : a.K - 1;
     const int Kp = a.Kp;
-    R dt;
-    if constexpr (REF)
-        dt = (R)a.ref_dt;
-    else
-        dt = (R)a.ctrl->dt;
     // mode (v, m) of element x, at `o` in the caller's order
     const auto at = [&](int v, int m, int x, int o) -> R {
         if constexpr (REF)
@@ -195,6 +191,11 @@ __device__ __forceinline__ double valu_process(const StageArgs<R>& a, int e, int
     }
 
     // ---- inverse mass (M = J*I; 1/J precomputed in FP64) and the RK stage update ----
+    R dt;
+    if constexpr (REF)
+        dt = (R)a.ref_dt;
+    else
+        dt = stage_dt();
     const R cj = gp(a.geo_e)[4 * Kp + ee] * dt;
     double lam = 0.0;
     if constexpr (REF) {
@@ -261,6 +262,12 @@ __device__ __forceinline__ double valu_process(const StageArgs<R>& a, int e, int
         }
     }
     return lam;
+}
+
+// the same with the dt of the control block
+template <int N, int P, typename R, bool BND = false, bool REF = false>
+__device__ __forceinline__ double valu_process(const StageArgs<R>& a, int e, int kind) {
+    return valu_process<N, P, R, BND, REF>(a, e, kind, [&] { return (R)a.ctrl->dt; });
 }
 
 }  // namespace dgmi

@@ -302,7 +302,7 @@ int dg_solver_set_max_groups(dg_solver* s, int max_groups);
 int dg_solver_launch_info(const dg_solver* s, int* out4);
 /* Times nsteps RK4 steps with HIP events on the solver's stream, one event
  * pair around every stage-kernel launch.  out[0] = mean stage-kernel ms,
- * out[1] = mean dt-kernel ms, out[2] = total ms, out[3] = number of stage
+ * out[1] = 0 (dt is computed in the step's first stage), out[2] = total ms, out[3] = number of stage
  * launches timed. */
 int dg_time_stage_kernels(dg_solver* s, int nsteps, double cfl, double* out);
 /* Runs nsteps RK4 CFL steps replayed from the captured step graph (the

@@ -43,13 +43,15 @@ static bool one(StageArgs<R> a, StageArgs<R> b, const StateIx& im, const StateIx
                 int threads) {
     a.kind = b.kind = KIND;
     double la = 0, lb = 0;
+    const auto go = [] { return true; };
+    const auto dt = [&] { return (R)b.ctrl->dt; };
     for (int e = 0; e < threads; e++) {
         if (a.bnd) {
             la = std::max(la, valu_process<4, P, R, true>(a, e, KIND));
-            lb = std::max(lb, lane_process<P, KIND, R, true, false>(b, e, ltab.data()));
+            lb = std::max(lb, lane_process<P, KIND, R, true, false>(b, e, ltab.data(), go, dt));
         } else {
             la = std::max(la, valu_process<4, P, R, false>(a, e, KIND));
-            lb = std::max(lb, lane_process<P, KIND, R, false, true>(b, e, ltab.data()));
+            lb = std::max(lb, lane_process<P, KIND, R, false, true>(b, e, ltab.data(), go, dt));
         }
     }
     // states of order 1, updates below 1, some hundred roundings each
