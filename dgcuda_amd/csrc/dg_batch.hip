@@ -36,14 +36,14 @@ struct SlotDesc {
     R *c, *acc, *ua, *ub;
     const R *geo_e, *geo_f;
     const int* nbr;
-    const uint32_t* fword;
+    const int* ntask;
     const int* halo;
-    const void* face4;
+    const void* sides;
     const void* metric4;
     const void* lface;
     const void* lmetric;
     Ctrl* ctrl;
-    int K, Kp, N, p, hcap, path;  // path 1 = lane per element, 2 = matrix-core tiles
+    int K, Kp, N, p, hcap, tcap, path;  // path 1 = lane per element, 2 = matrix-core tiles
     PhysP phys;
 };
 
@@ -250,12 +250,12 @@ __device__ __forceinline__ void batch_tile_items(const SlotDesc<R>* __restrict__
         }
         const StageArgs<R> a = slot_args<R, KIND>(sd);
         MfmaArgs mx;
-        mx.fword = uni(sd->fword);
+        mx.ntask = uni(sd->ntask);
         mx.halo = uni(sd->halo);
-        mx.face4 = uni(sd->face4);
+        mx.sides = uni(sd->sides);
         mx.metric4 = uni(sd->metric4);
         mx.hcap = uni(sd->hcap);
-        mx.pad = 0;
+        mx.tcap = uni(sd->tcap);
         const int N = uni(sd->N), p = uni(sd->p);
         double lam = 0.0;
         int next = it + G8;
@@ -588,9 +588,9 @@ class EngineT : public BatchEngine {
             d.geo_e = (const R*)si.geo_e;
             d.geo_f = (const R*)si.geo_f;
             d.nbr = si.nbr;
-            d.fword = si.fword;
+            d.ntask = si.ntask;
             d.halo = si.halo;
-            d.face4 = si.face4;
+            d.sides = si.sides;
             d.metric4 = si.metric4;
             d.lface = si.lface;
             d.lmetric = si.lmetric;
@@ -600,6 +600,7 @@ class EngineT : public BatchEngine {
             d.N = si.N;
             d.p = si.p;
             d.hcap = si.hcap;
+            d.tcap = si.tcap;
             d.path = tiles ? 2 : 1;
             d.phys = si.phys;
             if (solo_here) {

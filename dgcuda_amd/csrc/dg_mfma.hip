@@ -6,6 +6,8 @@
 // that XCD's L2), and the state of its next tile is in flight while it
 // computes the current one.  The per-tile work is mfma_process_tile_pipe
 // (dg_mfma_body.h), shared with the batched kernel.
+#include <algorithm>
+
 #include "dg_mfma_body.h"
 
 namespace dgmi {
@@ -140,43 +142,48 @@ __global__ void __launch_bounds__(256, (mfma_minw<R, KIND>())) k_stage_mfma(Stag
 
 size_t mfma_lds_bytes(int N, int hcap, int rs) { return mfma_tile_lds_bytes(N, hcap, rs); }
 
-// Packs the geometry of the matrix-core kernel (one thread per element):
-// a tile's 192 face records and 64 element maps become contiguous entries
-// of 4 values (FP32: the neighbour word's bits in the 4th value, FP64: its
-// value).
+// Packs the geometry of the matrix-core kernel: one thread per side record
+// (MfmaArgs) and per element map.
 template <typename R>
 __global__ void __launch_bounds__(256) k_mfma_pack(const R* __restrict__ geo_e, const R* __restrict__ geo_f,
-                                                  const uint32_t* __restrict__ fword, int K, int Kp,
-                                                  typename MfmaT<R>::V* __restrict__ face4,
+                                                  const int* __restrict__ nbr, const SideTask* __restrict__ tasks,
+                                                  int ntasks, int K, int Kp, typename MfmaT<R>::V* __restrict__ sides,
                                                   typename MfmaT<R>::V* __restrict__ metric4) {
     using V = typename MfmaT<R>::V;
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= Kp) return;
-    const size_t s = (size_t)min(e, K - 1), kp = (size_t)Kp;
-    for (int f = 0; f < 3; f++) {
-        const int wd = (int)(fword[f * kp + s] & (e < K ? ~0u : ~FW_OWNER));
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t kp = (size_t)Kp;
+    if (i < ntasks) {
+        const SideTask t = tasks[i];
+        const size_t e = (size_t)(t.ef / 3);
+        const int f = t.ef - 3 * (int)e;
+        const R q = R(0.25) * geo_f[(3 * f + 2) * kp + e];
+        const bool left = (nbr[f * kp + e] >> 30) & 1;
         R wv;
         if constexpr (sizeof(R) == 4)
-            wv = __int_as_float(wd);
+            wv = __int_as_float((int)t.word);
         else
-            wv = (R)wd;
-        face4[3 * (size_t)e + f] = V{geo_f[3 * f * kp + s], geo_f[(3 * f + 1) * kp + s], geo_f[(3 * f + 2) * kp + s], wv};
+            wv = (R)t.word;
+        sides[i] = V{geo_f[3 * f * kp + e], geo_f[(3 * f + 1) * kp + e], left ? -q : q, wv};
     }
-    metric4[e] = V{geo_e[s], geo_e[kp + s], geo_e[2 * kp + s], geo_e[3 * kp + s]};
+    if (i < Kp) {
+        const size_t s = (size_t)min(i, K - 1);
+        metric4[i] = V{geo_e[s], geo_e[kp + s], geo_e[2 * kp + s], geo_e[3 * kp + s]};
+    }
 }
 
 template <typename R>
-hipError_t launch_mfma_pack(const R* geo_e, const R* geo_f, const uint32_t* fword, int K, int Kp, void* face4,
-                            void* metric4, hipStream_t st) {
+hipError_t launch_mfma_pack(const R* geo_e, const R* geo_f, const int* nbr, const SideTask* tasks, int ntasks, int K,
+                            int Kp, void* sides, void* metric4, hipStream_t st) {
     using V = typename MfmaT<R>::V;
-    hipLaunchKernelGGL((k_mfma_pack<R>), dim3((Kp + 255) / 256), dim3(256), 0, st, geo_e, geo_f, fword, K, Kp,
-                       (V*)face4, (V*)metric4);
+    const int n = std::max(ntasks, Kp);
+    hipLaunchKernelGGL((k_mfma_pack<R>), dim3((n + 255) / 256), dim3(256), 0, st, geo_e, geo_f, nbr, tasks, ntasks, K,
+                       Kp, (V*)sides, (V*)metric4);
     return hipGetLastError();
 }
-template hipError_t launch_mfma_pack<float>(const float*, const float*, const uint32_t*, int, int, void*, void*,
-                                            hipStream_t);
-template hipError_t launch_mfma_pack<double>(const double*, const double*, const uint32_t*, int, int, void*, void*,
-                                             hipStream_t);
+template hipError_t launch_mfma_pack<float>(const float*, const float*, const int*, const SideTask*, int, int, int,
+                                            void*, void*, hipStream_t);
+template hipError_t launch_mfma_pack<double>(const double*, const double*, const int*, const SideTask*, int, int, int,
+                                             void*, void*, hipStream_t);
 
 // workgroups of the matrix-core kernel that fit on the device at once
 template <typename R, bool BND>

@@ -85,20 +85,19 @@ __host__ __device__ constexpr bool mode_step_used(int s) {
     return NP > 8 || MfmaT<R>::pos(0, s) < NP;
 }
 
-// LDS of a tile: face records [64][3] of 4 values (nx, ny, len, packed
-// word), the tile's side list (MFMA_TASK_BYTES: 192 entries of 8 bytes and
-// 4 per-wavefront counts), then traces [(64 + hcap)][17*N] values (16
-// points + 1 padding row so consecutive slots start in different banks), N
-// variables innermost; `rs` = bytes per value (4 FP32, 8 FP64).
-constexpr int MFMA_TASK_BYTES = 192 * 8 + 32;
+// LDS of a tile: the records of its sides [192] of 4 values (MfmaArgs), then
+// traces [(64 + hcap)][17*N] values (16 points + 1 padding row so consecutive
+// slots start in different banks), N variables innermost; `rs` = bytes per
+// value (4 FP32, 8 FP64).
+constexpr int MFMA_MAX_SIDES = MFMA_TILE * 3;
 __host__ __device__ constexpr size_t mfma_tile_lds_bytes(int N, int hcap, int rs = 4) {
-    return (size_t)MFMA_TILE * 3 * 4 * rs + MFMA_TASK_BYTES + (size_t)(MFMA_TILE + hcap) * 17 * N * rs;
+    return (size_t)MFMA_MAX_SIDES * 4 * rs + (size_t)(MFMA_TILE + hcap) * MFMA_SLOT_POINTS * N * rs;
 }
 
-// the traces of a tile's LDS, after the face records `fd` and the side list
+// the traces of a tile's LDS, after the side records `fd`
 template <typename V, typename R>
 __device__ __forceinline__ R* tile_traces(V* fd) {
-    return reinterpret_cast<R*>(reinterpret_cast<unsigned char*>(fd + MFMA_TILE * 3) + MFMA_TASK_BYTES);
+    return reinterpret_cast<R*>(fd + MFMA_MAX_SIDES);
 }
 
 // State arrays are in the tile layout (StateIx, tiled): lane j + 16g of a
@@ -286,19 +285,20 @@ constexpr bool rk_writes_acc() {
     return KIND == ST_RK4_2;
 }
 
-// Geometry of one tile from the packed arrays: the (face normal, length,
-// packed neighbour word) record this thread stores to LDS (threads 0..191
-// hold one of the 64 x 3 records; the others load record 191 again and
-// store nothing, so the load is not under a branch), the affine map and
-// the Jacobian of the lane's own element.  Padding elements replicate
-// element K-1 in every geometry array.
+// Geometry of one tile from the packed arrays: the side record this thread
+// stores to LDS (threads past tcap hold the tile's last again and store
+// nothing, so the load is not under a branch), the number of sides, the
+// affine map and the inverse mass of the lane's own element.  Padding
+// elements replicate element K-1 in every geometry array.
 template <typename R = float>
 struct TileGeo {
     using V = typename MfmaT<R>::V;
     V f;
+    int ntask;
     R xr, yr, xs, ys, ij;  // ij: the inverse mass 1/J (M = J*I), precomputed in FP64
     __device__ __forceinline__ void load(const StageArgs<R>& a, const MfmaArgs& mx, int tile, int el) {
-        f = ((const DG_GLOBAL V*)mx.face4)[(unsigned)(tile * (MFMA_TILE * 3) + min((int)threadIdx.x, MFMA_TILE * 3 - 1))];
+        f = ((const DG_GLOBAL V*)mx.sides)[(unsigned)(tile * mx.tcap + min((int)threadIdx.x, mx.tcap - 1))];
+        ntask = gp(mx.ntask)[(unsigned)tile];
         const unsigned ue = (unsigned)(tile * MFMA_TILE + el);
         const V m = ((const DG_GLOBAL V*)mx.metric4)[ue];
         xr = m[0];
@@ -309,28 +309,27 @@ struct TileGeo {
     }
 };
 
-// neighbour word of a face record (FP32: the bits of the 4th value, FP64:
+// word of a side record (FP32: the bits of the 4th value, FP64:
 // its value)
 __device__ __forceinline__ int face_word(float x) { return __float_as_int(x); }
 __device__ __forceinline__ int face_word(double x) { return (int)x; }
 
-// LLF flux of one point of one side: face record `r`, the element's trace
-// at the point `own` and the neighbour's `nbt`, in the orientation of the
-// element; written over `own`, and its negation over `nbt` when the
+// LLF flux of one point of one side: record `r` (word `wd`), the element's
+// trace at the point `own` and the neighbour's `nbt`, in the orientation of
+// the element; written over `own`, and its negation over `nbt` when the
 // neighbour is an element of the tile.  For a boundary side, `nw` is the
 // side's neighbour word (the ghost data's index) and jo the point.
 template <int N, int NQ1, typename R, bool BND>
-__device__ __forceinline__ void side_flux(const StageArgs<R>& a, const typename MfmaT<R>::V r, R* own, R* nbt,
+__device__ __forceinline__ void side_flux(const StageArgs<R>& a, const typename MfmaT<R>::V r, int wd, R* own, R* nbt,
                                           int nw, int jo) {
     using V = typename MfmaT<R>::V;
-    const int wd = face_word(r[3]);
-    const bool left = (wd >> 14) & 1;
-    const bool inner = (wd & 0xFFF) < MFMA_TILE;
+    const bool left = r[2] < R(0);
+    const bool inner = wd & SIDE_INNER;
     // boundary side (the element is its left element, the slot its own): the
     // ghost state of the point replaces the neighbour trace, which is not
     // read.  Only the BND instantiation carries this code, so the kernels
     // of meshes without boundary sides keep their register allocation.
-    const bool bside = BND && ((wd >> 15) & 1);
+    const bool bside = BND && (wd & SIDE_BOUNDARY);
     if constexpr (BND)
         if (bside) nbt = own;
     R G[N];
@@ -350,9 +349,8 @@ __device__ __forceinline__ void side_flux(const StageArgs<R>& a, const typename 
         normal_flux_speed<R>(a.phys, un, r[0], r[1], Fb, sb);
         const R lm = fmax(so, sb);
         const R lms = left ? lm : -lm;
-        const R cf = left ? R(-0.25) * r[2] : R(0.25) * r[2];
 #pragma unroll
-        for (int v = 0; v < N; v++) G[v] = cf * fma(lms, uo[v] - un[v], Fo[v] + Fb[v]);
+        for (int v = 0; v < N; v++) G[v] = r[2] * fma(lms, uo[v] - un[v], Fo[v] + Fb[v]);
         *reinterpret_cast<V*>(own) = V{G[0], G[1], G[2], G[3]};
         if (inner && !bside) *reinterpret_cast<V*>(nbt) = V{-G[0], -G[1], -G[2], -G[3]};
     } else {
@@ -368,7 +366,7 @@ __device__ __forceinline__ void side_flux(const StageArgs<R>& a, const typename 
         flux<N, R>(a.phys, UL, fxl, fyl);
         flux<N, R>(a.phys, UR, fxr, fyr);
         const R lm = llf_speed<N, R>(a.phys, UL, UR, r[0], r[1]);
-        const R coef = left ? R(-0.5) * r[2] : R(0.5) * r[2];
+        const R coef = R(2) * r[2];
         G[0] = coef * (R(0.5) * ((fxl[0] + fxr[0]) * r[0] + (fyl[0] + fyr[0]) * r[1] + lm * (UL[0] - UR[0])));
         own[0] = G[0];
         if (inner && !bside) nbt[0] = -G[0];
@@ -398,7 +396,7 @@ __device__ __forceinline__ double mfma_process_tile_pipe(const StageArgs<R>& a, 
     using V = typename M::V;
     constexpr int NP = n_modes(P), NQ = n_quad_vol(P), NQ1 = P + 1, NPT = 3 * NQ1;
     constexpr int TILE = MFMA_TILE;
-    constexpr int TS = 17 * N;
+    constexpr int TS = MFMA_SLOT_POINTS * N;
     constexpr bool LAST = (KIND == ST_RK4_4 || KIND == ST_RK2_2);
     using RK = RkNeeds<KIND>;
     constexpr int HPW = MfmaTileState<N, P, R>::HPW;
@@ -456,27 +454,7 @@ __device__ __forceinline__ double mfma_process_tile_pipe(const StageArgs<R>& a, 
             for (int i = 0; i < 4; i++) ts[slot * TS + M::qpos(g, i) * N + v] = acc[i];
         }
     }
-    // face records, and the side list: the thread of record t = 3 el + f of
-    // a side this tile computes writes entry (word bits 16..23) of the list,
-    // {offset of the element's trace at point 0 of the face | offset of the
-    // neighbour's trace at its last point << 16, t}; per wavefront the count
-    uint2* task = reinterpret_cast<uint2*>(fd + TILE * 3);
-    int* ntask4 = reinterpret_cast<int*>(task + TILE * 3);
-    {
-        const int t = threadIdx.x;
-        const int wd = face_word(gc.f[3]);
-        const bool owner = t < TILE * 3 && (wd & FW_OWNER);
-        if (t < TILE * 3) fd[t] = gc.f;
-        if (owner) {
-            const int eo = t / 3, f = t - 3 * eo;
-            const int slot = wd & 0xFFF, fn = (wd >> 12) & 3;
-            const unsigned oo = (unsigned)(eo * TS + f * NQ1 * N);
-            const unsigned no = (unsigned)(slot * TS + (fn * NQ1 + NQ1 - 1) * N);
-            task[(wd >> FW_TASK_SHIFT) & 0xFF] = make_uint2(oo | (no << 16), (unsigned)t);
-        }
-        const unsigned long long bm = __ballot(owner);
-        if (lane == 0) ntask4[w] = __popcll(bm);
-    }
+    if ((int)threadIdx.x < mx.tcap) fd[threadIdx.x] = gc.f;
 
     // ---- phase 2: volume, side fluxes, surface, inverse mass, RK update ----
     V U[N];
@@ -556,7 +534,7 @@ __device__ __forceinline__ double mfma_process_tile_pipe(const StageArgs<R>& a, 
     // ---- phase 2b: the LLF flux of each side of the tile, once ----
     // (after the volume terms, which use only this wave's registers, so the
     // waves meet at the barrier with the next tile's loads long in flight)
-    // Work item (side k of the list, point jo); the 64-item blocks of a
+    // Work item (side k, point jo); the 64-item blocks of a
     // round go to the wavefronts in an order that rotates with the tile, so
     // the partial last round falls to each wavefront in turn.  The flux is
     // computed in the orientation of the record's element and written over
@@ -567,21 +545,23 @@ __device__ __forceinline__ double mfma_process_tile_pipe(const StageArgs<R>& a, 
     // entry of the tile's elements belongs to one side and one point, so the
     // item that reads it is the only one that writes it.
     {
-        const int nitem = (ntask4[0] + ntask4[1] + ntask4[2]) * NQ1;
+        const int nitem = gc.ntask * NQ1;
         const int wblk = ((w + tile) & 3) * 64;
         for (int r0 = 0; r0 < nitem; r0 += 256) {
             if (r0 + wblk >= nitem) continue;  // uniform over the wavefront
             const int it = r0 + wblk + lane;
             if (it < nitem) {
                 const int k = it / NQ1, jo = it - k * NQ1;
-                const uint2 en = task[k];
+                const V rec = fd[k];
+                const int wd = face_word(rec[3]);
+                const int oo = wd & ((1 << SIDE_OWN_BITS) - 1);
+                const int no = (wd >> SIDE_OWN_BITS) & ((1 << SIDE_NBR_BITS) - 1);
                 int nw = 0;
                 if constexpr (BND) {
-                    const int eo = (int)en.y / 3, f = (int)en.y - 3 * eo;
+                    const int eo = oo / MFMA_SLOT_POINTS, f = (oo - eo * MFMA_SLOT_POINTS) / NQ1;
                     nw = gp(a.nbr)[f * a.Kp + base + eo];
                 }
-                side_flux<N, NQ1, R, BND>(a, fd[en.y], ts + (en.x & 0xFFFF) + jo * N, ts + (en.x >> 16) - jo * N,
-                                          nw, jo);
+                side_flux<N, NQ1, R, BND>(a, rec, wd, ts + (oo + jo) * N, ts + (no - jo) * N, nw, jo);
             }
         }
     }

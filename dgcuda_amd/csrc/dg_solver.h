@@ -66,14 +66,14 @@ struct LaunchShape {
 struct SlotInfo {
     void *c, *acc, *ua, *ub, *geo_e, *geo_f;
     const int* nbr;
-    const uint32_t* fword;
+    const int* ntask;
     const int* halo;
-    const void* face4;      // packed geometry of the matrix-core kernels
+    const void* sides;      // packed geometry of the matrix-core kernels
     const void* metric4;
     const void* lface;      // packed geometry of the lane kernels' vector layout
     const void* lmetric;
     Ctrl* ctrl;
-    int K, Kp, N, p, hcap, kind;
+    int K, Kp, N, p, hcap, tcap, kind;
     int boundary;           // the mesh has boundary sides (batched as a solo solve)
     PhysP phys;
 };

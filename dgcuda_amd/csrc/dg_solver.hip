@@ -294,11 +294,11 @@ class SolverT : public Solver {
     int* perm_d = nullptr;  // [Kp]: caller's element of internal element i (padding: element K-1's)
     int device = -1;
     std::vector<int> h_nbr[3];
-    uint32_t* fword = nullptr;
+    int* ntask = nullptr;
     int* halo = nullptr;
-    void *face4 = nullptr, *metric4 = nullptr;
+    void *sides = nullptr, *metric4 = nullptr;
     void *lface = nullptr, *lmetric = nullptr;  // packed geometry of the lane kernel's vector layout
-    int64_t tile_bytes = 0;  // fword, halo and packed geometry
+    int64_t tile_bytes = 0;  // side counts, halo lists and packed geometry
     MfmaArgs mx{};
     double *V = nullptr, *Jd = nullptr, *audit_part = nullptr;
     double* bnd = nullptr;      // boundary sides' ghost data (boundary_data)
@@ -325,7 +325,7 @@ class SolverT : public Solver {
         if (stream) (void)hipStreamSynchronize(stream);  // nothing queued may use the buffers
         graph.drop();
         void* bufs[] = {c,  acc,        ua,   ub,    geo_e, geo_f, nbr,     V,      Jd,
-                        audit_part, ctrl, fword, halo,  face4, metric4, bnd, perm_d, lface, lmetric};
+                        audit_part, ctrl, ntask, halo,  sides, metric4, bnd, perm_d, lface, lmetric};
         for (void* b : bufs) pool_free(b);
         pool_release_stream(stream);
     }
@@ -458,82 +458,92 @@ class SolverT : public Solver {
         return Status::ok();
     }
 
-    // Matrix-core tiling: per (element, face) the LDS slot of the neighbour
-    // (inside the tile, or in the tile's halo list), the halo lists, and the
-    // tile's side list: the sides the tile computes (boundary and halo sides,
-    // and of each side between two of its elements the left element's
-    // record), numbered in record order.
+    // Matrix-core tiling: the tiles' halo lists (a neighbour's LDS slot is its
+    // place in the tile or, past the tile, in the list) and the sides each
+    // tile computes (MfmaArgs): boundary and halo sides, and of each side
+    // between two of its elements the left element's, in (element, face) order.
     Status build_mfma_tiles(int tile_elems) {
         const int ntiles = (K + tile_elems - 1) / tile_elems;
-        std::vector<uint32_t> words(3 * (size_t)Kp, 0);
         std::vector<std::vector<int>> halos(ntiles);
-        int hmax = 0;
+        std::vector<std::vector<SideTask>> lists(ntiles);
+        size_t hmax = 0, tmax = 0;
         for (int t = 0; t < ntiles; t++) {
             const int b = t * tile_elems, end = std::min(b + tile_elems, K);
             std::vector<int>& h = halos[t];
-            uint32_t ntask = 0;
             for (int e = b; e < end; e++)
                 for (int f = 0; f < 3; f++) {
                     const int wv = h_nbr[f][e];
-                    uint32_t wd;
-                    bool owner;
+                    const uint32_t own = (e - b) * MFMA_SLOT_POINTS + f * NQ1;
                     if (wv < 0) {
-                        // boundary side: own slot and face, left, flag bit 15
-                        // (the kernel reads the ghost data through the
-                        // neighbour word)
-                        wd = (uint32_t)((e - b) | (f << 12) | (1 << 14) | (1 << 15));
-                        owner = true;
-                    } else {
-                        const int nb = wv & NB_ELEM_MASK, fn = (wv >> 28) & 3, left = (wv >> 30) & 1;
-                        int slot;
-                        if (nb >= b && nb < end) {
-                            slot = nb - b;
-                        } else {
-                            auto it = std::find(h.begin(), h.end(), nb);
-                            slot = tile_elems + (int)(it - h.begin());
-                            if (it == h.end()) h.push_back(nb);
-                        }
-                        if (slot >= 4096) return Status::err(DG_ERR_UNSUPPORTED, "tile halo too large");
-                        wd = (uint32_t)(slot | (fn << 12) | (left << 14));
-                        owner = slot >= tile_elems || left;
+                        // boundary side: the kernel reads the ghost data through
+                        // the neighbour word
+                        lists[t].push_back(SideTask{3 * e + f, own | SIDE_BOUNDARY});
+                        continue;
                     }
-                    if (owner) wd |= (ntask++ << FW_TASK_SHIFT) | FW_OWNER;
-                    words[f * (size_t)Kp + e] = wd;
+                    const int nb = wv & NB_ELEM_MASK, fn = (wv >> 28) & 3, left = (wv >> 30) & 1;
+                    const bool inner = nb >= b && nb < end;
+                    if (inner && !left) continue;  // the left element's record computes it
+                    uint32_t slot = nb - b;
+                    if (!inner) {
+                        auto it = std::find(h.begin(), h.end(), nb);
+                        slot = tile_elems + (int)(it - h.begin());
+                        if (it == h.end()) h.push_back(nb);
+                    }
+                    const uint32_t nbr_at = slot * MFMA_SLOT_POINTS + fn * NQ1 + NQ1 - 1;
+                    lists[t].push_back(SideTask{3 * e + f, own | (nbr_at << SIDE_OWN_BITS) | (inner ? SIDE_INNER : 0)});
                 }
-            hmax = std::max(hmax, (int)h.size());
+            hmax = std::max(hmax, h.size());
+            tmax = std::max(tmax, lists[t].size());
         }
-        const int hcap = std::max(16, (hmax + 15) / 16 * 16);
-        // LDS per workgroup: traces and face records, plus the 5-slot operand table
+        const int hcap = std::max(16, (int)(hmax + 15) / 16 * 16);
+        const int tcap = (int)(tmax + 3) / 4 * 4;
+        // LDS per workgroup: traces and side records, plus the 5-slot operand table
         if (hcap > MFMA_MAX_HALO || mfma_lds_bytes(N, hcap, (int)sizeof(R)) + 5 * 64 * 4 * sizeof(R) > 160 * 1024)
             return Status::err(DG_ERR_UNSUPPORTED, "tile halo too large for the matrix-core kernel");
-        std::vector<int> hl((size_t)ntiles * hcap);
-        for (int t = 0; t < ntiles; t++)
+        static_assert(MFMA_TILE_ELEMS * MFMA_SLOT_POINTS <= (1 << SIDE_OWN_BITS) &&
+                          (MFMA_TILE_ELEMS + MFMA_MAX_HALO) * MFMA_SLOT_POINTS <= (1 << SIDE_NBR_BITS),
+                      "trace offsets fit a side's word");
+        std::vector<int> hl((size_t)ntiles * hcap), nt(ntiles);
+        std::vector<SideTask> tl((size_t)ntiles * tcap);  // unused records repeat the tile's last
+        for (int t = 0; t < ntiles; t++) {
             for (int i = 0; i < hcap; i++)
                 hl[(size_t)t * hcap + i] = i < (int)halos[t].size() ? halos[t][i] : t * tile_elems;
+            nt[t] = (int)lists[t].size();
+            for (int i = 0; i < tcap; i++)
+                tl[(size_t)t * tcap + i] = nt[t] ? lists[t][std::min(i, nt[t] - 1)] : SideTask{3 * t * tile_elems, 0};
+        }
         HIPST(hipStreamSynchronize(stream));  // queued launches may still read the old lists
-        for (void* b : {(void*)fword, (void*)halo, (void*)face4, (void*)metric4}) pool_free(b);
-        fword = nullptr;
+        for (void* b : {(void*)ntask, (void*)halo, sides, metric4}) pool_free(b);
+        ntask = nullptr;
         halo = nullptr;
-        face4 = nullptr;
+        sides = nullptr;
         metric4 = nullptr;
         tile_bytes = 0;
-        const size_t bw = words.size() * sizeof(uint32_t), bh = hl.size() * sizeof(int);
-        const size_t bf = (size_t)Kp * 3 * 4 * sizeof(R), bm = (size_t)Kp * 4 * sizeof(R);
-        Status sa = pool_alloc((void**)&fword, bw);
+        const size_t bn = nt.size() * sizeof(int), bh = hl.size() * sizeof(int);
+        const size_t bf = tl.size() * 4 * sizeof(R), bm = (size_t)Kp * 4 * sizeof(R), bt = tl.size() * sizeof(SideTask);
+        struct Temp {
+            void* p = nullptr;
+            ~Temp() { pool_free(p); }
+        } tasks;
+        Status sa = pool_alloc((void**)&ntask, bn);
         if (sa) sa = pool_alloc((void**)&halo, bh);
-        if (sa) sa = pool_alloc((void**)&face4, bf);
-        if (sa) sa = pool_alloc((void**)&metric4, bm);
+        if (sa) sa = pool_alloc(&sides, bf);
+        if (sa) sa = pool_alloc(&metric4, bm);
+        if (sa) sa = pool_alloc(&tasks.p, bt);
         if (!sa) return sa;
-        tile_bytes = (int64_t)(bw + bh + bf + bm);
-        if (!(sa = copy_to_device(fword, words.data(), bw, stream))) return sa;
+        tile_bytes = (int64_t)(bn + bh + bf + bm);
+        if (!(sa = copy_to_device(ntask, nt.data(), bn, stream))) return sa;
         if (!(sa = copy_to_device(halo, hl.data(), bh, stream))) return sa;
-        HIPST(launch_mfma_pack<R>(geo_e, geo_f, fword, K, Kp, face4, metric4, stream));
+        if (!(sa = copy_to_device(tasks.p, tl.data(), bt, stream))) return sa;
+        HIPST(launch_mfma_pack<R>(geo_e, geo_f, nbr, (const SideTask*)tasks.p, (int)tl.size(), K, Kp, sides, metric4,
+                                  stream));
         HIPST(hipStreamSynchronize(stream));
-        mx.fword = fword;
+        mx.ntask = ntask;
         mx.halo = halo;
-        mx.face4 = face4;
+        mx.sides = sides;
         mx.metric4 = metric4;
         mx.hcap = hcap;
+        mx.tcap = tcap;
         return Status::ok();
     }
 
@@ -1084,9 +1094,9 @@ class SolverT : public Solver {
         o->geo_e = geo_e;
         o->geo_f = geo_f;
         o->nbr = nbr;
-        o->fword = fword;
+        o->ntask = ntask;
         o->halo = halo;
-        o->face4 = face4;
+        o->sides = sides;
         o->metric4 = metric4;
         o->lface = lface;
         o->lmetric = lmetric;
@@ -1096,6 +1106,7 @@ class SolverT : public Solver {
         o->N = N;
         o->p = p;
         o->hcap = mx.hcap;
+        o->tcap = mx.tcap;
         o->kind = shape.kind;
         o->boundary = has_boundary ? 1 : 0;
         o->phys = phys;
