@@ -361,8 +361,12 @@ __device__ __forceinline__ DG_GLOBAL T* gp(T* p) {
 //    lane's matrix products leave in its registers):
 //    - FP32 (tiled = 1): G = ceil(NP/4) groups, group g = modes 4g..4g+3,
 //      (((e/16)*N + v)*G + m/4)*64 + (e%16)*4 + m%4;
-//    - FP64 (tiled = 2): 4 groups, group g = modes g, g+4, g+8, g+12,
-//      ((e/16)*N + v)*256 + (m%4)*64 + (e%16)*4 + m/4.
+//    - FP64 (tiled = 2): the lane of group g holds modes g, g+4, g+8, g+12
+//      (r = m/4 = 0..3, g = m%4).  Per block and variable the used modes only
+//      (p = 4: 16 slots for 15), in pieces of one access each: from 9 modes on
+//      [4 groups][16 elements][r = 0, 1], then at p = 4 the same of r = 2, 3
+//      and at p = 3 [2 groups][16 elements] of r = 2; below, per r
+//      [groups][16 elements] (tile64_at).
 //    The wavefront's 64 lanes cover the block's variable contiguously.
 //    Modes >= NP are padding and hold zeros.
 //  * Vector layout of the Euler lane kernels up to p = 3: per mode, rows of
@@ -371,26 +375,35 @@ __device__ __forceinline__ DG_GLOBAL T* gp(T* p) {
 //    2 variables each) accesses:
 //      FP32 (m*Kp + e)*4 + v;  FP64 ((m*2 + v/2)*Kp + e)*2 + v%2.
 constexpr int tile_groups(int NP) { return (NP + 3) / 4; }
+// mode slots per (variable, element) of the FP64 tile layout, and the place
+// of (mode m, element j of 16) in a block's variable
+__host__ __device__ constexpr int tile64_slots(int NP) { return NP > 12 ? 16 : NP; }
+__host__ __device__ constexpr int tile64_at(int NP, int m, int j) {
+    const int g = m & 3, r = m >> 2;
+    if (NP <= 8) return r * 64 + g * 16 + j;
+    if (r < 2) return (g * 16 + j) * 2 + r;
+    return NP > 12 ? 128 + (g * 16 + j) * 2 + (r - 2) : 128 + g * 16 + j;
+}
 enum { LAYOUT_MODES = 0, LAYOUT_TILE32 = 1, LAYOUT_TILE64 = 2, LAYOUT_VEC32 = 3, LAYOUT_VEC64 = 4 };
 
 struct StateIx {
     int N, NP, Kp, tiled;
     // mode slots stored per (variable, element): NP, or the tile layout's
     __host__ __device__ int slots() const {
-        return tiled == LAYOUT_TILE32 ? 4 * tile_groups(NP) : tiled == LAYOUT_TILE64 ? 16 : NP;
+        return tiled == LAYOUT_TILE32 ? 4 * tile_groups(NP) : tiled == LAYOUT_TILE64 ? tile64_slots(NP) : NP;
     }
     __host__ __device__ size_t at(int v, int m, int e) const {
         if (!tiled) return ((size_t)v * NP + m) * Kp + e;
         if (tiled == LAYOUT_VEC32) return (((size_t)m * Kp + e) << 2) + v;
         if (tiled == LAYOUT_VEC64) return ((((size_t)m * 2 + (v >> 1)) * Kp + e) << 1) + (v & 1);
-        if (tiled == 2) return (((size_t)(e >> 4) * N + v) << 8) + (size_t)(((m & 3) << 6) + ((e & 15) << 2) + (m >> 2));
+        if (tiled == LAYOUT_TILE64)
+            return ((size_t)(e >> 4) * N + v) * (16 * tile64_slots(NP)) + tile64_at(NP, m, e & 15);
         const int G = tile_groups(NP);
         return ((((size_t)(e >> 4) * N + v) * G + (m >> 2)) << 6) + (size_t)((e & 15) << 2) + (m & 3);
     }
     // entries of one array: N*NP*Kp, or the tile layout's padded count
     __host__ __device__ size_t elems() const {
-        if (!tiled || tiled >= LAYOUT_VEC32) return (size_t)N * NP * Kp;
-        return (size_t)N * (tiled == 2 ? 16 : 4 * tile_groups(NP)) * Kp;
+        return (size_t)N * slots() * Kp;
     }
 };
 

@@ -46,11 +46,9 @@ __device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c) {
 // The FP32 product leaves D[4g + r][j] in register r of lane j + 16g, the
 // FP64 product D[g + 4r][j]; pos(g, r) names that row.  Every reduction is
 // ordered the same way (product s of lane group g takes index pos(g, s)),
-// so a lane's B operands are the rows it holds in the output.  When at
-// most 8 modes are in use, a mode step s whose modes pos(0..3, s) are all
-// padding (FP64: modes 4s..4s+3) is left out: at p = 2 in FP64 that is
-// two steps of four, 6.7% faster per stage; the one step of p = 3
-// measured 2% slower left out, so p = 3 keeps it.
+// so a lane's B operands are the rows it holds in the output.  A mode
+// step s whose modes pos(0..3, s) are all padding (FP64 up to p = 3: modes
+// 4s..4s+3) is left out: p = 3 at 131,072 triangles 173.5 -> 166.2 us per step.
 // Volume and face points are placed by the A tables of the interpolations:
 // row i holds point qrow(i), so register r of lane group g holds point
 // qpos(g, r) = g + 4r in both precisions.  Product step r of the
@@ -82,7 +80,7 @@ constexpr int MFMA_TILE = 64;
 // whether mode step s of the mode reductions is issued (see above)
 template <typename R, int NP>
 __host__ __device__ constexpr bool mode_step_used(int s) {
-    return NP > 8 || MfmaT<R>::pos(0, s) < NP;
+    return MfmaT<R>::pos(0, s) < NP;
 }
 
 // LDS of a tile: the records of its sides [192] of 4 values (MfmaArgs), then
@@ -100,41 +98,86 @@ __device__ __forceinline__ R* tile_traces(V* fd) {
     return reinterpret_cast<R*>(fd + MFMA_MAX_SIDES);
 }
 
-// State arrays are in the tile layout (StateIx, tiled): lane j + 16g of a
-// wavefront reads the 4 modes pos(g, 0..3) of its element as one access of
-// 4 values (16 bytes FP32, 32 bytes FP64).  Addresses are a wavefront-uniform
-// base (scalar registers) plus one per-lane 32-bit index in units of 4
-// values.
-template <typename R>
-__device__ __forceinline__ const DG_GLOBAL typename MfmaT<R>::V* gp4(const R* p) {
-    return (const DG_GLOBAL typename MfmaT<R>::V*)p;
+// State access in the tile layout (StateIx): lane j + 16g of a wavefront
+// moves the modes pos(g, 0..3) of its element and one variable.  Lanes whose
+// group or register holds no mode read another lane's entry instead (in
+// bounds; their operands meet zero matrix entries) and store nothing.
+template <typename V>
+__device__ __forceinline__ V tile_get(const DG_GLOBAL V* p, bool nt) {
+    return nt ? __builtin_nontemporal_load(p) : *p;
 }
-template <typename R>
-__device__ __forceinline__ DG_GLOBAL typename MfmaT<R>::V* gp4(R* p) {
-    return (DG_GLOBAL typename MfmaT<R>::V*)p;
-}
-
-// mode groups per variable of a 16-element block: ceil(n_p/4) in FP32, 4 in
-// FP64 (a lane's modes g, g+4, g+8, g+12 span all groups)
-template <typename R>
-__host__ __device__ constexpr int tile_groups_of(int NP) {
-    return sizeof(R) == 4 ? tile_groups(NP) : 4;
-}
-
-// stride (in units of 4 values) between the variables of one 16-element block
-template <int P, typename R>
-constexpr int tile_var_stride() { return 16 * tile_groups_of<R>(n_modes(P)); }
-
-// index (in units of 4 values) of (variable 0, lane group g, element e);
-// variable v adds v * tile_var_stride<P, R>().  Lanes of groups past the
-// last (FP32, p <= 3) read the last group again; their operands meet zero
-// matrix entries and they store nothing.
 template <int N, int P, typename R>
-__device__ __forceinline__ unsigned tile_lane4(int e, int g) {
-    constexpr int G = tile_groups_of<R>(n_modes(P));
-    const int gg = (G == 4) ? g : min(g, G - 1);
-    return (unsigned)((e >> 4) * (N * 16 * G) + gg * 16 + (e & 15));
-}
+struct TileIo;
+// FP32: one access of 16 bytes; groups of 4 modes
+template <int N, int P>
+struct TileIo<N, P, float> {
+    using V = floatx4;
+    static constexpr int G = tile_groups(n_modes(P)), VS = 16 * G;
+    unsigned at;  // in units of 4 values: a scalar base and a 32-bit index
+    __device__ __forceinline__ TileIo(int e, int g)
+        : at((unsigned)((e >> 4) * (N * 16 * G) + (G == 4 ? g : min(g, G - 1)) * 16 + (e & 15))) {}
+    __device__ __forceinline__ V load(const float* p, int v, bool nt = false) const {
+        return tile_get((const DG_GLOBAL V*)p + (v * VS + at), nt);
+    }
+    __device__ __forceinline__ void store(float* p, int v, int g, V x) const {
+        if (G == 4 || g < G) __builtin_nontemporal_store(x, (DG_GLOBAL V*)p + (v * VS + at));
+    }
+};
+// FP64: pieces of 16 and 8 bytes (tile64_at).  Storing the used modes only
+// instead of 16 slots cuts the state's bytes by 37% at p = 3 and 62% at p = 2,
+// and 16-byte pieces a wavefront covers without gaps replace two halves of 32:
+// per step p = 3 at 131,072 triangles 225.3 -> 173.5 us (at 524,288 786 -> 624),
+// p = 2 at 32,768 74 -> 45.6, p = 4 at 131,072 243.7 -> 227.0, advection p = 3
+// at 131,072 64.3 -> 54.9 and p = 1 at 2,048 18.0 -> 16.5.
+template <int N, int P>
+struct TileIo<N, P, double> {
+    using V = doublex4;
+    typedef double V2 __attribute__((ext_vector_type(2)));
+    static constexpr int NP = n_modes(P), VS = 16 * tile64_slots(NP);
+    static constexpr bool PAIRS = NP > 8;
+    // lanes per register r whose group holds a mode
+    __host__ __device__ static constexpr int groups(int r) { return NP - 4 * r < 4 ? NP - 4 * r : 4; }
+    size_t block;
+    int a, b;  // places of registers 0 (and 1) and of the next piece
+    __device__ __forceinline__ TileIo(int e, int g) : block((size_t)(e >> 4) * (N * VS)) {
+        const int j = e & 15;
+        if constexpr (PAIRS) {
+            a = (g * 16 + j) * 2;
+            b = NP > 12 ? 128 + a : 128 + min(g, groups(2) - 1) * 16 + j;
+        } else {
+            a = min(g, groups(0) - 1) * 16 + j;
+            b = 64 + min(g, NP > 4 ? groups(1) - 1 : 0) * 16 + j;
+        }
+    }
+    __device__ __forceinline__ V load(const double* p, int v, bool nt = false) const {
+        const DG_GLOBAL double* q = (const DG_GLOBAL double*)p + block + v * VS;
+        if constexpr (PAIRS) {
+            const V2 x = tile_get((const DG_GLOBAL V2*)(q + a), nt);
+            if constexpr (NP > 12) {
+                const V2 y = tile_get((const DG_GLOBAL V2*)(q + b), nt);
+                return V{x[0], x[1], y[0], y[1]};
+            }
+            return V{x[0], x[1], tile_get(q + b, nt), 0.0};
+        }
+        const double x = tile_get(q + a, nt);
+        if constexpr (NP > 4) return V{x, tile_get(q + b, nt), 0.0, 0.0};
+        return V{x, 0.0, 0.0, 0.0};
+    }
+    __device__ __forceinline__ void store(double* p, int v, int g, V x) const {
+        DG_GLOBAL double* q = (DG_GLOBAL double*)p + block + v * VS;
+        if constexpr (PAIRS) {
+            __builtin_nontemporal_store(V2{x[0], x[1]}, (DG_GLOBAL V2*)(q + a));
+            if constexpr (NP > 12)
+                __builtin_nontemporal_store(V2{x[2], x[3]}, (DG_GLOBAL V2*)(q + b));
+            else if (g < groups(2))
+                __builtin_nontemporal_store(x[2], q + b);
+        } else {
+            if (g < groups(0)) __builtin_nontemporal_store(x[0], q + a);
+            if constexpr (NP > 4)
+                if (g < groups(1)) __builtin_nontemporal_store(x[1], q + b);
+        }
+    }
+};
 
 // per-lane A operands of the five products (lane layout: A[i][k] from lane
 // i + 16k, B[k][j] from lane j + 16k, D[4(l/16)+r][l%16] in register r).
@@ -193,7 +236,6 @@ struct MfmaTileState {
     using V = typename MfmaT<R>::V;
     using VM = typename MfmaT<typename std::conditional<REF, double, R>::type>::V;
     static constexpr int HPW = (4 * N + 3) / 4;  // most halo pairs per wave (hcap <= 64)
-    static constexpr int VS = tile_var_stride<P, R>();
     VM ub[N];
     VM hb[HPW];
     __device__ __forceinline__ static V bulk(const VM& x) {
@@ -244,11 +286,11 @@ struct MfmaTileState {
     }
     __device__ __forceinline__ void load_data(const R* __restrict__ u, int K, int tile, int w, int g, int j,
                                               const int (&hid)[HPW]) {
-        const unsigned l4 = tile_lane4<N, P, R>(min(tile * MFMA_TILE + w * 16 + j, K - 1), g);
+        const TileIo<N, P, R> io(min(tile * MFMA_TILE + w * 16 + j, K - 1), g);
 #pragma unroll
-        for (int v = 0; v < N; v++) ub[v] = gp4(u)[v * VS + l4];
+        for (int v = 0; v < N; v++) ub[v] = io.load(u, v);
 #pragma unroll
-        for (int q = 0; q < HPW; q++) hb[q] = gp4(u)[((w + 4 * q) % N) * VS + tile_lane4<N, P, R>(hid[q], g)];
+        for (int q = 0; q < HPW; q++) hb[q] = TileIo<N, P, R>(hid[q], g).load(u, (w + 4 * q) % N);
     }
     __device__ __forceinline__ void load_next(const StageArgs<R>& a, int tile, int w, int g, int j,
                                               const int (&hid)[HPW]) {
@@ -479,8 +521,7 @@ __device__ __forceinline__ double mfma_process_tile_pipe(const StageArgs<R>& a, 
     // with requests to make gets the issue slot before waves computing
     // (measured 1.5% faster per step at 524,288 triangles, p = 4).
     __builtin_amdgcn_s_setprio(2);
-    constexpr int VS = tile_var_stride<P, R>();
-    const unsigned l4 = tile_lane4<N, P, R>(ee, g);
+    const TileIo<N, P, R> io(ee, g);
     V cr[N], ar[N];
 #pragma unroll
     for (int v = 0; v < N; v++) {
@@ -489,8 +530,8 @@ __device__ __forceinline__ double mfma_process_tile_pipe(const StageArgs<R>& a, 
         if constexpr (RK::C_FROM_INPUT) cr[v] = ub[v];
         if constexpr (RK::ACC_FROM_INPUT) ar[v] = ub[v];
         if constexpr (sizeof(R) == 4) {
-            if constexpr (RK::LOAD_C) cr[v] = __builtin_nontemporal_load(&gp4(a.c)[v * VS + l4]);
-            if constexpr (RK::LOAD_ACC) ar[v] = __builtin_nontemporal_load(&gp4(a.acc)[v * VS + l4]);
+            if constexpr (RK::LOAD_C) cr[v] = io.load(a.c, v, true);
+            if constexpr (RK::LOAD_ACC) ar[v] = io.load(a.acc, v, true);
         }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -600,8 +641,8 @@ __device__ __forceinline__ double mfma_process_tile_pipe(const StageArgs<R>& a, 
         // triangles, p = 4); FP32 measured no gain from the same move
 #pragma unroll
         for (int v = 0; v < N; v++) {
-            if constexpr (RK::LOAD_C) cr[v] = __builtin_nontemporal_load(&gp4(a.c)[v * VS + l4]);
-            if constexpr (RK::LOAD_ACC) ar[v] = __builtin_nontemporal_load(&gp4(a.acc)[v * VS + l4]);
+            if constexpr (RK::LOAD_C) cr[v] = io.load(a.c, v, true);
+            if constexpr (RK::LOAD_ACC) ar[v] = io.load(a.acc, v, true);
         }
     }
     gc.load(a, mx, next, el);
@@ -626,7 +667,7 @@ __device__ __forceinline__ double mfma_process_tile_pipe(const StageArgs<R>& a, 
     }
 
     // inverse mass and the RK stage update; lane holds modes m = pos(g, i)
-    const unsigned s4 = tile_lane4<N, P, R>(e, g);
+    const TileIo<N, P, R> so(e, g);
     R c0[N];
     double lam = 0.0;
 #pragma unroll
@@ -639,10 +680,8 @@ __device__ __forceinline__ double mfma_process_tile_pipe(const StageArgs<R>& a, 
             an[i] = t;
         }
         // padding elements (e >= K) compute a copy of element K-1 into their own slots
-        if (tile_groups_of<R>(NP) == 4 || g < tile_groups_of<R>(NP)) {
-            if constexpr (rk_writes_acc<KIND>()) __builtin_nontemporal_store(an, &gp4(a.acc)[v * VS + s4]);
-            __builtin_nontemporal_store(o, &gp4(a.out)[v * VS + s4]);
-        }
+        if constexpr (rk_writes_acc<KIND>()) so.store(a.acc, v, g, an);
+        so.store(a.out, v, g, o);
         c0[v] = o[0];
     }
     if constexpr (LAST) {

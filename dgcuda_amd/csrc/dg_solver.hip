@@ -896,7 +896,9 @@ class SolverT : public Solver {
         if (cur != device) return Status::err(DG_ERR_STATE, "the solver's device is not the current device");
         char* base = static_cast<char*>(noalloc_scratch(device));
         if (!base) return Status::err(DG_ERR_STATE, "the device's scratch is not set up");
-        const size_t one = (six.elems() * sizeof(R) + 255) / 256 * 256;
+        // (the limit counts 16 mode slots in the FP64 tile layout, as stated in the interface)
+        const size_t slots = six.tiled == LAYOUT_TILE64 ? 16 : six.slots();
+        const size_t one = ((size_t)N * slots * Kp * sizeof(R) + 255) / 256 * 256;
         if (2 * one > NOALLOC_SCRATCH_BYTES)
             return Status::err(DG_ERR_BUDGET, "this solve needs " + std::to_string(2 * one) +
                                                   " bytes of scratch; the allocation-free entry point has " +
