@@ -43,7 +43,7 @@ struct SlotDesc {
     const void* lface;
     const void* lmetric;
     Ctrl* ctrl;
-    int K, Kp, N, p, hcap, tcap, path;  // path 1 = lane per element, 2 = matrix-core tiles
+    int K, Kp, N, p, hcap, tcap, cls;  // cls: the solve's class (BM_* bit)
     PhysP phys;
 };
 
@@ -164,10 +164,10 @@ __device__ __forceinline__ StageArgs<R> slot_args(const SlotDesc<R>* sd) {
 // Work-item classes, as bits of a launch's mask: the bodies a stage kernel
 // carries.  A batch runs each stage as one or more persistent launches whose
 // masks cover the classes present:
-//   one launch (the default): BM_ALL, so light (advection) and heavy (Euler)
-//     items share the CUs;
+//   one launch: BM_ALL, so light (advection) and heavy (Euler) items share
+//     the CUs;
 //   per class: one launch per class, each with the register budget of its
-//     own bodies.
+//     own bodies and on a stream of its own (enqueue_steps).
 // A kernel's register allocation, and with it the wavefronts a SIMD holds,
 // is that of the bodies it carries (FP64: Euler tiles alone 2 wavefronts per
 // SIMD, every body together 1).
@@ -178,7 +178,8 @@ enum : int {
     BM_TILE_EUL = 8,
     BM_LANES = BM_LANE_ADV | BM_LANE_EUL,
     BM_TILES = BM_TILE_ADV | BM_TILE_EUL,
-    BM_ALL = BM_LANES | BM_TILES
+    BM_ALL = BM_LANES | BM_TILES,
+    BM_SOLO = 16  // class of the solves that run their own kernels
 };
 
 // Work lists in `parts` (XCD x = blockIdx % 8), 9 bounds per list:
@@ -355,10 +356,11 @@ const void* batch_stage_fn(int kind, int mask) {
     }
 }
 
+// starts a step of the solves of `classes`
 template <typename R>
-__global__ void k_batch_dt(const SlotDesc<R>* __restrict__ slots, const int* __restrict__ nslots) {
+__global__ void k_batch_dt(const SlotDesc<R>* __restrict__ slots, const int* __restrict__ nslots, int classes) {
     const int s = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);  // one wavefront per slot
-    if (s < *nslots) dt_update(slots[s].ctrl);
+    if (s < *nslots && (slots[s].cls & classes)) dt_update(slots[s].ctrl);
 }
 
 // every slot's control block into one array (one host copy)
@@ -416,16 +418,23 @@ class EngineT : public BatchEngine {
     int cap_slots = 0, cap_items = 0;
     int nslots = 0, nitems = 0, dt_grid = 0, cus = 0;
     int max_groups_req = 0;          // set_max_groups (0: no cap)
-    // set_launch_form; the default is the form measured faster on the
-    // 64-solve ragged mix in each precision (FP32 one launch: 1.15x the
-    // per-class form; FP64 per class: 1.12x the one launch)
-    int form = sizeof(R) == 8 ? DG_BATCH_PER_CLASS : DG_BATCH_ONE_LAUNCH;
+    // set_launch_form (-1: automatic, per_class_form).  Several launches run
+    // side by side, so a CU's registers are shared: capped at two workgroups
+    // per CU each (PER_CLASS_GROUPS), 1-5% faster per step than every workgroup
+    // that fits alone, one per CU 3-10% slower (4 to 64 ragged solves).
+    int form = -1;
+    bool per_class = false;          // form of the current work list
+    static constexpr int PER_CLASS_GROUPS = 2;
+    static constexpr int64_t PER_CLASS_MIN = 65536;
     std::vector<Launch> launches;    // the batch kernels of a stage, in launch order
     std::vector<int2> raw_items[BATCH_LISTS];  // the work lists in solve order, and
     std::vector<double> raw_cost[BATCH_LISTS]; // each item's estimated cost
     std::vector<int2> h_items;       // host copy of the work lists and their XCD bounds
     std::vector<int> h_parts;
     StepGraph graph;
+    std::vector<hipStream_t> side;   // streams of the second and further launches
+    std::vector<hipEvent_t> join;    // their ends
+    hipEvent_t fork = nullptr;
     int solo_min = 0;             // 0: every solve in the batch launch
     std::vector<Solver*> solo;    // solves launched with their own kernels
     std::vector<uint64_t> solo_uid;  // their ids: the captured step holds their buffers
@@ -433,6 +442,9 @@ class EngineT : public BatchEngine {
     ~EngineT() override {
         if (st) (void)hipStreamSynchronize(st);
         graph.drop();
+        for (hipStream_t q : side) pool_release_stream(q);
+        for (hipEvent_t e : join) (void)hipEventDestroy(e);
+        if (fork) (void)hipEventDestroy(fork);
         void* b[] = {d_slots, d_items, d_xcd, d_status, d_ctrls};
         for (void* q : b)
             if (q) hipFree(q);
@@ -517,10 +529,35 @@ class EngineT : public BatchEngine {
     // the masks of the form's launches, in launch order (Euler tiles first:
     // the longest items start earliest)
     std::vector<int> form_masks() const {
-        switch (form) {
-            case DG_BATCH_PER_CLASS: return {BM_TILE_EUL, BM_TILE_ADV, BM_LANE_EUL, BM_LANE_ADV};
-            default: return {BM_ALL};
+        if (per_class) return {BM_TILE_EUL, BM_TILE_ADV, BM_LANE_EUL, BM_LANE_ADV};
+        return {BM_ALL};
+    }
+
+    static int class_of(const SlotInfo& si) {
+        if (si.kind >= 2) return si.N == 4 ? BM_TILE_EUL : BM_TILE_ADV;
+        return si.N == 4 ? BM_LANE_EUL : BM_LANE_ADV;
+    }
+    bool runs_solo(const SlotInfo& si) const { return si.boundary || (solo_min > 0 && si.K >= solo_min); }
+
+    // The automatic form.  One kernel per class, side by side, holds more
+    // wavefronts per SIMD and its stages wait for their own class only; one
+    // kernel for all has one chain of launches.  One launch / per class, us per
+    // step, FP32 ragged batches: 22,880 triangles 49.6 / 67.4, 41,470 63.6 /
+    // 67.5, 51,414 69.6 / 70.7, 66,568 80.6 / 75.3, 93,950 117.3 / 98.3, 453,104
+    // 267 / 255, 1,748,140 800 / 657; FP64 24 solves of up to 2,000 triangles
+    // 104.4 / 84.7, 453,104 622 / 466, 1,748,140 2,035 / 1,313.
+    // (A served set crosses the line down only at half of it: a change of form
+    // captures the step again.)
+    bool per_class_form(const std::vector<Solver*>& solvers) const {
+        if (form >= 0) return form == DG_BATCH_PER_CLASS;
+        if (sizeof(R) == 8) return true;
+        int64_t elems = 0;
+        for (Solver* sv : solvers) {
+            SlotInfo si;
+            sv->slot_info(&si);
+            if (!runs_solo(si)) elems += si.K;
         }
+        return elems >= (per_class ? PER_CLASS_MIN / 2 : PER_CLASS_MIN);
     }
 
     // Splits each list into 8 contiguous chunks of equal estimated cost, one
@@ -546,6 +583,7 @@ class EngineT : public BatchEngine {
     }
 
     Status set_slots(const std::vector<Solver*>& solvers) override {
+        per_class = per_class_form(solvers);
         const int ns = (int)solvers.size();
         std::vector<Solver*> new_solo;
         std::vector<SlotDesc<R>> hs(ns);
@@ -579,7 +617,7 @@ class EngineT : public BatchEngine {
             const bool tiles = si.kind >= 2;
             // solves with boundary sides always run their own kernels (the
             // batched bodies carry no boundary code)
-            const bool solo_here = si.boundary || (solo_min > 0 && si.K >= solo_min);
+            const bool solo_here = runs_solo(si);
             if (!solo_here && tiles != (si.p >= 3))
                 return Status::err(DG_ERR_STATE, "batch slots use matrix-core tiles exactly when p >= 3");
             if (!solo_here && tiles && si.hcap > MFMA_MAX_HALO)
@@ -607,13 +645,14 @@ class EngineT : public BatchEngine {
             d.p = si.p;
             d.hcap = si.hcap;
             d.tcap = si.tcap;
-            d.path = tiles ? 2 : 1;
             d.phys = si.phys;
             if (solo_here) {
+                d.cls = BM_SOLO;
                 new_solo.push_back(solvers[s]);  // slot kept for dt and status; no work items
                 continue;
             }
-            const int bit = tiles ? (si.N == 4 ? BM_TILE_EUL : BM_TILE_ADV) : (si.N == 4 ? BM_LANE_EUL : BM_LANE_ADV);
+            const int bit = class_of(si);
+            d.cls = bit;
             const int l = list_of[bit];
             if (tiles) hmax[l] = std::max(hmax[l], si.hcap);
             const int te = tiles ? MFMA_TILE : BATCH_VALU_TILE;
@@ -634,6 +673,21 @@ class EngineT : public BatchEngine {
             if (!sh) return sh;
             nl.push_back(L);
         }
+        if (nl.size() > 1)
+            for (Launch& L : nl) {
+                L.resident = std::min(L.resident, PER_CLASS_GROUPS * cus / 8 * 8);
+                L.grid = std::min(L.grid, L.resident);
+            }
+        for (size_t b = side.size() + 1; b < nl.size(); b++) {
+            hipStream_t q = nullptr;
+            Status sq = pool_stream(&q);
+            if (!sq) return sq;
+            side.push_back(q);
+            hipEvent_t e = nullptr;
+            HIPST(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+            join.push_back(e);
+        }
+        if (nl.size() > 1 && !fork) HIPST(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
         if (nl != launches) {
             launches = nl;
             drop_graph();
@@ -662,36 +716,61 @@ class EngineT : public BatchEngine {
         return Status::ok();
     }
 
-    Status launch_stage(int kind) {
-        for (const Launch& L : launches) {
-            const void* fn = batch_stage_fn<R>(kind, L.mask);
+    // the stages' launches of one step of launch L's solves on stream q
+    Status launch_step(const Launch& L, int classes, hipStream_t q) {
+        hipLaunchKernelGGL((k_batch_dt<R>), dim3(dt_grid), dim3(256), 0, q, d_slots, d_xcd + BATCH_NSLOT_AT, classes);
+        HIPST(hipGetLastError());
+        for (int k : {ST_RK4_1, ST_RK4_2, ST_RK4_3, ST_RK4_4}) {
+            const void* fn = batch_stage_fn<R>(k, L.mask);
             if (!fn) return Status::err(DG_ERR_ARG, "unsupported batch stage");
             const SlotDesc<R>* slots = d_slots;
             const int2* items = d_items;
             const int* parts = d_xcd + 9 * L.list;
             void* args[] = {(void*)&slots, (void*)&items, (void*)&parts};
-            HIPST(hipLaunchKernel(fn, dim3(L.grid), dim3(256), args, L.lds, st));
+            HIPST(hipLaunchKernel(fn, dim3(L.grid), dim3(256), args, L.lds, q));
         }
         return Status::ok();
     }
 
-    Status step_direct() {
-        hipLaunchKernelGGL((k_batch_dt<R>), dim3(dt_grid), dim3(256), 0, st, d_slots, d_xcd + BATCH_NSLOT_AT);
+    // one step of the solves that run their own kernels
+    Status solo_step() {
+        hipLaunchKernelGGL((k_batch_dt<R>), dim3(dt_grid), dim3(256), 0, st, d_slots, d_xcd + BATCH_NSLOT_AT,
+                           (int)BM_SOLO);
         HIPST(hipGetLastError());
         Status s0;
-        for (int k : {ST_RK4_1, ST_RK4_2, ST_RK4_3, ST_RK4_4}) {
-            if (!(s0 = launch_stage(k))) return s0;
+        for (int k : {ST_RK4_1, ST_RK4_2, ST_RK4_3, ST_RK4_4})
             for (Solver* sv : solo)
                 if (!(s0 = sv->stage_on(k, st))) return s0;
+        return s0;
+    }
+
+    // n steps on the engine's stream.  Solves do not depend on each other, so
+    // each launch's solves advance the n steps on a stream of their own
+    // (branches of the captured graph) and meet at the end: one class's tail
+    // and launch gap are filled by the others.  Per-class launches one behind
+    // the other -> side by side: FP64 64 solves of up to 200,000 triangles 1,996
+    // -> 1,338 us per step, 32 of up to 100,000 FP32 292 (one launch) -> 267.
+    Status enqueue_steps(int n) {
+        Status s0;
+        const int nb = (int)launches.size();
+        if (nb > 1) HIPST(hipEventRecord(fork, st));
+        for (int b = 1; b < nb; b++) HIPST(hipStreamWaitEvent(side[b - 1], fork, 0));
+        for (int b = 0; b < nb; b++)
+            for (int i = 0; i < n; i++)
+                if (!(s0 = launch_step(launches[b], launches[b].mask, b ? side[b - 1] : st))) return s0;
+        if (!solo.empty())
+            for (int i = 0; i < n; i++)
+                if (!(s0 = solo_step())) return s0;
+        for (int b = 1; b < nb; b++) {
+            HIPST(hipEventRecord(join[b - 1], side[b - 1]));
+            HIPST(hipStreamWaitEvent(st, join[b - 1], 0));
         }
         return Status::ok();
     }
 
     Status steps(int n, bool use_graph) override {
-        if (use_graph) return graph.run(st, n, [&] { return step_direct(); });
-        Status s0;
-        for (int i = 0; i < n && s0; i++) s0 = step_direct();
-        return s0;
+        if (use_graph) return graph.run(st, n, [&](int k) { return enqueue_steps(k); });
+        return n > 0 ? enqueue_steps(n) : Status::ok();
     }
 
     Status status(std::vector<double>& out) override {

@@ -783,7 +783,7 @@ class SolverT : public Solver {
         if (use_graph) {
             if (graph_scheme != scheme) graph.drop();
             graph_scheme = scheme;
-            return graph.run(stream, n, [&] { return enqueue_stages(scheme, true); });
+            return graph.run(stream, n, [&](int k) { return enqueue_cfl_steps(k, scheme, false); });
         }
         for (int i = 0; i < n && st; i++) st = enqueue_stages(scheme, true);
         return st;

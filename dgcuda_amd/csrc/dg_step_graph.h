@@ -26,7 +26,7 @@ class StepGraph {
         taken = 0;
     }
 
-    // `n` steps on stream `st`; `enqueue` puts one step on it
+    // `n` steps on stream `st`; `enqueue(k)` puts k steps on it
     template <typename F>
     Status run(hipStream_t st, int64_t n, F&& enqueue) {
         while (n > 0) {
@@ -53,8 +53,7 @@ class StepGraph {
     static Status capture(hipStream_t st, int len, hipGraphExec_t& out, F&& enqueue) {
         hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
         if (e != hipSuccess) return hip_status(e, "step capture");
-        Status s;
-        for (int i = 0; i < len && s; i++) s = enqueue();
+        const Status s = enqueue(len);
         hipGraph_t gr = nullptr;
         e = hipStreamEndCapture(st, &gr);
         if (s && e == hipSuccess) e = hipGraphInstantiate(&out, gr, nullptr, nullptr, 0);
