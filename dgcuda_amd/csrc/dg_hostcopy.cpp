@@ -22,6 +22,7 @@ namespace {
 constexpr size_t COPY_BLOCK = size_t(1) << 20;
 constexpr size_t COPY_MIN_PART = size_t(4) << 20;
 constexpr int COPY_MAX_THREADS = 4;
+constexpr size_t COPY_SMALL = size_t(64) << 10;
 constexpr size_t COPY_IDLE_BLOCKS = 2 * COPY_MAX_THREADS;  // kept between calls, of all threads together
 
 // pinned blocks, shared by every thread of the process; at most
@@ -140,7 +141,10 @@ Status copy_parts(char* host, char* dev, size_t bytes, bool to_host, hipStream_t
         if (at < end) err[i] = copy_part(host + at, dev + at, end - at, to_host, s);
     };
     std::vector<std::thread> th;
-    std::vector<int> inline_parts{0};
+    std::vector<int> inline_parts;
+    th.reserve(parts);  // (nothing may throw while a thread runs)
+    inline_parts.reserve(parts);
+    inline_parts.push_back(0);
     for (int i = 1; i < parts; i++) {
         bool started = false;
         if (on[i]) {
@@ -167,6 +171,11 @@ Status copy_parts(char* host, char* dev, size_t bytes, bool to_host, hipStream_t
 
 Status copy_to_host(void* dst, const void* src_dev, size_t bytes, hipStream_t st) {
     return copy_parts((char*)dst, (char*)const_cast<void*>(src_dev), bytes, true, st);
+}
+
+Status upload_small(void* dst_dev, const void* src, size_t bytes, hipStream_t st) {
+    if (bytes > COPY_SMALL) return copy_to_device(dst_dev, src, bytes, st);
+    return hip_status(hipMemcpyAsync(dst_dev, src, bytes, hipMemcpyHostToDevice, st), "copy");
 }
 
 Status copy_to_device(void* dst_dev, const void* src, size_t bytes, hipStream_t st) {

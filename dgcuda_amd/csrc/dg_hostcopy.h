@@ -5,9 +5,13 @@
 
 namespace dgmi {
 
-// Both wait for the copy.  The device side is ready (copy_to_host) or free to
+// The first two wait for the copy.  The device side is ready (copy_to_host) or free to
 // be overwritten (copy_to_device) once the work queued on `st` has finished.
 Status copy_to_host(void* dst, const void* src_dev, size_t bytes, hipStream_t st);
 Status copy_to_device(void* dst_dev, const void* src, size_t bytes, hipStream_t st);
+// copy_to_device; a small array is only queued, as a wait for each of a
+// set-up's arrays costs more than its copy: the caller waits for `st` before
+// it lets the array go
+Status upload_small(void* dst_dev, const void* src, size_t bytes, hipStream_t st);
 
 }  // namespace dgmi

@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <tuple>
 #include <map>
+#include <memory>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -414,41 +415,45 @@ class SolverT : public Solver {
         HIPST(hipMemsetAsync(ub, 0, M * sizeof(R), stream));
         // geometry, padded entries replicate the last element; the 5th
         // element value is the inverse mass 1/J (M = J*I), computed in FP64
-        std::vector<R> he(5 * (size_t)Kp), hf(9 * (size_t)Kp);
-        std::vector<int> hn(3 * (size_t)Kp);
-        std::vector<double> hv(6 * (size_t)Kp), hj(Kp);
+        // (one array after the other into memory that is not cleared first)
+        const size_t kp = (size_t)Kp;
+        const std::unique_ptr<R[]> he(new R[5 * kp]), hf(new R[9 * kp]);
+        const std::unique_ptr<int[]> hn(new int[3 * kp]);
+        const std::unique_ptr<double[]> hv(new double[6 * kp]), hj(new double[kp]);
+        const auto put = [this](auto* dst, const auto& src, auto&& f) {
+            for (int i = 0; i < K; i++) dst[i] = f(src[i]);
+            for (int i = K; i < Kp; i++) dst[i] = dst[K - 1];
+        };
         const auto gr = [this](double x) { return (R)(geom_fp32 ? (double)(float)x : x); };
-        for (int i = 0; i < Kp; i++) {
-            const int e = std::min(i, K - 1);
-            he[i] = gr(g.xr[e]);
-            he[Kp + i] = gr(g.yr[e]);
-            he[2 * (size_t)Kp + i] = gr(g.xs[e]);
-            he[3 * (size_t)Kp + i] = gr(g.ys[e]);
-            he[4 * (size_t)Kp + i] = gr(1.0 / g.J[e]);
-            hj[i] = g.J[e];
-            for (int f = 0; f < 3; f++) {
-                hf[(3 * f + 0) * (size_t)Kp + i] = gr(g.fnx[f][e]);
-                hf[(3 * f + 1) * (size_t)Kp + i] = gr(g.fny[f][e]);
-                hf[(3 * f + 2) * (size_t)Kp + i] = gr(g.flen[f][e]);
-                hn[f * (size_t)Kp + i] = g.nbr[f][e];
-            }
-            for (int v = 0; v < 6; v++) hv[v * (size_t)Kp + i] = g.V[v][e];
+        const auto same = [](auto x) { return x; };
+        put(&he[0], g.xr, gr);
+        put(&he[kp], g.yr, gr);
+        put(&he[2 * kp], g.xs, gr);
+        put(&he[3 * kp], g.ys, gr);
+        put(&he[4 * kp], g.J, [&](double J) { return gr(1.0 / J); });
+        put(&hj[0], g.J, same);
+        for (int f = 0; f < 3; f++) {
+            put(&hf[(3 * f + 0) * kp], g.fnx[f], gr);
+            put(&hf[(3 * f + 1) * kp], g.fny[f], gr);
+            put(&hf[(3 * f + 2) * kp], g.flen[f], gr);
+            put(&hn[f * kp], g.nbr[f], same);
         }
-        if (!(st = copy_to_device(geo_e, he.data(), he.size() * sizeof(R), stream))) return st;
-        if (!(st = copy_to_device(geo_f, hf.data(), hf.size() * sizeof(R), stream))) return st;
-        if (!(st = copy_to_device(nbr, hn.data(), hn.size() * sizeof(int), stream))) return st;
+        for (int v = 0; v < 6; v++) put(&hv[v * kp], g.V[v], same);
+        if (!(st = upload_small(geo_e, he.get(), 5 * kp * sizeof(R), stream))) return st;
+        if (!(st = upload_small(geo_f, hf.get(), 9 * kp * sizeof(R), stream))) return st;
+        if (!(st = upload_small(nbr, hn.get(), 3 * kp * sizeof(int), stream))) return st;
         std::vector<int> hp(Kp);
         for (int i = 0; i < Kp; i++) hp[i] = perm[std::min(i, K - 1)];
         if (!(st = alloc((void**)&perm_d, (size_t)Kp * sizeof(int)))) return st;
-        if (!(st = copy_to_device(perm_d, hp.data(), hp.size() * sizeof(int), stream))) return st;
+        if (!(st = upload_small(perm_d, hp.data(), hp.size() * sizeof(int), stream))) return st;
         for (int f = 0; f < 3; f++) h_nbr[f] = g.nbr[f];
         if (has_boundary) {
             const std::vector<double> hb = boundary_data(g, build_tables(p), ic, pr.quirks, pr.wall_x, pr.wall_y);
             if (!(st = alloc((void**)&bnd, hb.size() * sizeof(double)))) return st;
             if (!(st = copy_to_device(bnd, hb.data(), hb.size() * sizeof(double), stream))) return st;
         }
-        if (!(st = copy_to_device(V, hv.data(), hv.size() * sizeof(double), stream))) return st;
-        if (!(st = copy_to_device(Jd, hj.data(), hj.size() * sizeof(double), stream))) return st;
+        if (!(st = upload_small(V, hv.get(), 6 * kp * sizeof(double), stream))) return st;
+        if (!(st = upload_small(Jd, hj.get(), kp * sizeof(double), stream))) return st;
         hctrl = Ctrl{};
         hctrl.min_r = min_r;
         hctrl.two_p1 = 2. * p + 1.;
@@ -464,12 +469,14 @@ class SolverT : public Solver {
     // between two of its elements the left element's, in (element, face) order.
     Status build_mfma_tiles(int tile_elems) {
         const int ntiles = (K + tile_elems - 1) / tile_elems;
-        std::vector<std::vector<int>> halos(ntiles);
-        std::vector<std::vector<SideTask>> lists(ntiles);
-        size_t hmax = 0, tmax = 0;
+        // the tiles' lists one behind the other, and where each tile's begin
+        std::vector<int> halos, halo_at(ntiles + 1, 0), side_at(ntiles + 1, 0);
+        std::vector<SideTask> tasks_h;
+        halos.reserve((size_t)K);
+        tasks_h.reserve((size_t)K * 2);
+        int hmax = 0, tmax = 0;
         for (int t = 0; t < ntiles; t++) {
             const int b = t * tile_elems, end = std::min(b + tile_elems, K);
-            std::vector<int>& h = halos[t];
             for (int e = b; e < end; e++)
                 for (int f = 0; f < 3; f++) {
                     const int wv = h_nbr[f][e];
@@ -477,7 +484,7 @@ class SolverT : public Solver {
                     if (wv < 0) {
                         // boundary side: the kernel reads the ghost data through
                         // the neighbour word
-                        lists[t].push_back(SideTask{3 * e + f, own | SIDE_BOUNDARY});
+                        tasks_h.push_back(SideTask{3 * e + f, own | SIDE_BOUNDARY});
                         continue;
                     }
                     const int nb = wv & NB_ELEM_MASK, fn = (wv >> 28) & 3, left = (wv >> 30) & 1;
@@ -485,18 +492,21 @@ class SolverT : public Solver {
                     if (inner && !left) continue;  // the left element's record computes it
                     uint32_t slot = nb - b;
                     if (!inner) {
-                        auto it = std::find(h.begin(), h.end(), nb);
-                        slot = tile_elems + (int)(it - h.begin());
-                        if (it == h.end()) h.push_back(nb);
+                        const auto h = halos.begin() + halo_at[t];
+                        const auto it = std::find(h, halos.end(), nb);
+                        slot = tile_elems + (int)(it - h);
+                        if (it == halos.end()) halos.push_back(nb);
                     }
                     const uint32_t nbr_at = slot * MFMA_SLOT_POINTS + fn * NQ1 + NQ1 - 1;
-                    lists[t].push_back(SideTask{3 * e + f, own | (nbr_at << SIDE_OWN_BITS) | (inner ? SIDE_INNER : 0)});
+                    tasks_h.push_back(SideTask{3 * e + f, own | (nbr_at << SIDE_OWN_BITS) | (inner ? SIDE_INNER : 0)});
                 }
-            hmax = std::max(hmax, h.size());
-            tmax = std::max(tmax, lists[t].size());
+            halo_at[t + 1] = (int)halos.size();
+            side_at[t + 1] = (int)tasks_h.size();
+            hmax = std::max(hmax, halo_at[t + 1] - halo_at[t]);
+            tmax = std::max(tmax, side_at[t + 1] - side_at[t]);
         }
-        const int hcap = std::max(16, (int)(hmax + 15) / 16 * 16);
-        const int tcap = (int)(tmax + 3) / 4 * 4;
+        const int hcap = std::max(16, (hmax + 15) / 16 * 16);
+        const int tcap = (tmax + 3) / 4 * 4;
         // LDS per workgroup: traces and side records, plus the 5-slot operand table
         if (hcap > MFMA_MAX_HALO || mfma_lds_bytes(N, hcap, (int)sizeof(R)) + 5 * 64 * 4 * sizeof(R) > 160 * 1024)
             return Status::err(DG_ERR_UNSUPPORTED, "tile halo too large for the matrix-core kernel");
@@ -506,11 +516,11 @@ class SolverT : public Solver {
         std::vector<int> hl((size_t)ntiles * hcap), nt(ntiles);
         std::vector<SideTask> tl((size_t)ntiles * tcap);  // unused records repeat the tile's last
         for (int t = 0; t < ntiles; t++) {
-            for (int i = 0; i < hcap; i++)
-                hl[(size_t)t * hcap + i] = i < (int)halos[t].size() ? halos[t][i] : t * tile_elems;
-            nt[t] = (int)lists[t].size();
+            const int nh = halo_at[t + 1] - halo_at[t], h0 = halo_at[t], s0 = side_at[t];
+            for (int i = 0; i < hcap; i++) hl[(size_t)t * hcap + i] = i < nh ? halos[h0 + i] : t * tile_elems;
+            nt[t] = side_at[t + 1] - s0;
             for (int i = 0; i < tcap; i++)
-                tl[(size_t)t * tcap + i] = nt[t] ? lists[t][std::min(i, nt[t] - 1)] : SideTask{3 * t * tile_elems, 0};
+                tl[(size_t)t * tcap + i] = nt[t] ? tasks_h[s0 + std::min(i, nt[t] - 1)] : SideTask{3 * t * tile_elems, 0};
         }
         HIPST(hipStreamSynchronize(stream));  // queued launches may still read the old lists
         for (void* b : {(void*)ntask, (void*)halo, sides, metric4}) pool_free(b);
@@ -532,9 +542,9 @@ class SolverT : public Solver {
         if (sa) sa = pool_alloc(&tasks.p, bt);
         if (!sa) return sa;
         tile_bytes = (int64_t)(bn + bh + bf + bm);
-        if (!(sa = copy_to_device(ntask, nt.data(), bn, stream))) return sa;
-        if (!(sa = copy_to_device(halo, hl.data(), bh, stream))) return sa;
-        if (!(sa = copy_to_device(tasks.p, tl.data(), bt, stream))) return sa;
+        if (!(sa = upload_small(ntask, nt.data(), bn, stream))) return sa;
+        if (!(sa = upload_small(halo, hl.data(), bh, stream))) return sa;
+        if (!(sa = upload_small(tasks.p, tl.data(), bt, stream))) return sa;
         HIPST(launch_mfma_pack<R>(geo_e, geo_f, nbr, (const SideTask*)tasks.p, (int)tl.size(), K, Kp, sides, metric4,
                                   stream));
         HIPST(hipStreamSynchronize(stream));
@@ -840,6 +850,21 @@ class SolverT : public Solver {
         return st;
     }
 
+    // The solve's device as the current one while the state is converted (a
+    // state may be read or set with another device current).
+    struct OnDevice {
+        int prev = -1;
+        explicit OnDevice(int dev) {
+            if (hipGetDevice(&prev) == hipSuccess && prev != dev)
+                (void)hipSetDevice(dev);
+            else
+                prev = -1;
+        }
+        ~OnDevice() {
+            if (prev >= 0) (void)hipSetDevice(prev);
+        }
+    };
+
     // c_ref[var][mode][elem] (FP64, caller's element order) <-> device, in
     // the current layout (padding elements replicate the last element and
     // padding modes are zero).  The order and the precision change on the
@@ -848,6 +873,7 @@ class SolverT : public Solver {
     // reordered by one host thread: 185), setting it 5 (74); FP64 p = 3 at
     // 131,072 1.9 (32) and 1.1 (21).
     Status upload_ref(const double* c_ref, R* dst) {
+        const OnDevice here(device);
         Staging s;
         Status st = staging(dst, s);
         const size_t lo = (size_t)s.rows.split * K, hi = (size_t)N * NP * K - lo;
@@ -860,6 +886,7 @@ class SolverT : public Solver {
     }
 
     Status download_ref(const R* src, double* c_ref) {
+        const OnDevice here(device);
         Staging s;
         Status st = staging(src, s);
         if (!st) return st;
