@@ -98,7 +98,7 @@ __device__ __forceinline__ int batch_mfma_run(const StageArgs<R>& a, const MfmaA
     gc.load(a, mx, tile, w * 16 + j);
     st.load_data(a.u, a.K, tile, w, g, j, hid);
     MfmaTileState<N, P, R>::load_ids(mx.halo, mx.hcap, n1, w, j, hid);
-    if (w == 0) mfma_a_to_lds<N, P, R>(tabA, lane);  // the previous run ended with a barrier
+    mfma_a_to_lds<P, R>(tabA, w, lane);  // the previous run ended with a barrier
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     while (true) {

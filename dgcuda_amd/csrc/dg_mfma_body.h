@@ -179,50 +179,36 @@ struct TileIo<N, P, double> {
     }
 };
 
-// per-lane A operands of the five products (lane layout: A[i][k] from lane
-// i + 16k, B[k][j] from lane j + 16k, D[4(l/16)+r][l%16] in register r).
-// The mode reductions (vol, tr) run mode 4g+s through product s in lane
-// group g, so the B operand of a lane is the lane's own 4 consecutive modes
-// (the state's 16-byte access) and the state in operand registers is
-// already in the output layout of the projections.
-template <int N, int P, typename R = float>
-struct MfmaA {
-    R vol[4], tr[4], sp[4], gx[4], gy[4];
-    // `z` is zero at run time; a caller that loops over several instantiations
-    // passes a loop-variant zero so the table reads stay inside its loop
-    // instead of being hoisted (and held in registers) for every variant.
-    __device__ __forceinline__ void init(int g, int j, int z = 0) {
-        constexpr int NP = n_modes(P), NQ = n_quad_vol(P), NQ1 = P + 1, NPT = 3 * NQ1;
-        const TabP<R, P>& T = *reinterpret_cast<const TabP<R, P>*>(reinterpret_cast<const R*>(&tab<R, P>()) + z);
-        const int qj = MfmaT<R>::qrow(j);  // the point of A row j
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-            const int m = MfmaT<R>::pos(g, s);
-            vol[s] = (m < NP && qj < NQ) ? T.B[m][qj] : R(0);
-            tr[s] = (m < NP && qj < NPT) ? T.S[qj / NQ1][m][qj % NQ1] : R(0);
-            const int q = MfmaT<R>::qpos(g, s);
-            gx[s] = (j < NP && q < NQ) ? T.Gx[j][q] : R(0);
-            gy[s] = (j < NP && q < NQ) ? T.Gy[j][q] : R(0);
-            sp[s] = (j < NP && q < NPT) ? T.S[q / NQ1][j][q % NQ1] * T.W1[q % NQ1] : R(0);
-        }
-    }
-};
-
-// Slots of the per-lane A operands in a workgroup's LDS table [5][64] of
-// 4 values (the pipelined kernel reads them where used instead of holding
-// 20 registers).
+// The five products' per-lane A operands (lane layout: A[i][k] from lane
+// i + 16k, B[k][j] from lane j + 16k) as an LDS table [5][64] of 4 values:
+// read where used, they would hold 20 registers.  The mode reductions (vol,
+// tr) run mode pos(g, s) through product s in lane group g, so the B operand
+// of a lane is its own modes as it loads them and the state in operand
+// registers is already in the output layout of the projections.  A call fills
+// the operands of product step s; the 4 wavefronts of a batch's workgroup take
+// one each at the start of every run (by one wavefront: 64 ragged solves in
+// FP32 657 -> 636 us per step).
 enum { MFMA_A_VOL = 0, MFMA_A_TR = 1, MFMA_A_SP = 2, MFMA_A_GX = 3, MFMA_A_GY = 4, MFMA_A_SLOTS = 5 };
 
-template <int N, int P, typename R>
-__device__ __forceinline__ void mfma_a_to_lds(typename MfmaT<R>::V* tabA, int lane) {
-    using V = typename MfmaT<R>::V;
-    MfmaA<N, P, R> A;
-    A.init(lane >> 4, lane & 15);
-    tabA[MFMA_A_VOL * 64 + lane] = V{A.vol[0], A.vol[1], A.vol[2], A.vol[3]};
-    tabA[MFMA_A_TR * 64 + lane] = V{A.tr[0], A.tr[1], A.tr[2], A.tr[3]};
-    tabA[MFMA_A_SP * 64 + lane] = V{A.sp[0], A.sp[1], A.sp[2], A.sp[3]};
-    tabA[MFMA_A_GX * 64 + lane] = V{A.gx[0], A.gx[1], A.gx[2], A.gx[3]};
-    tabA[MFMA_A_GY * 64 + lane] = V{A.gy[0], A.gy[1], A.gy[2], A.gy[3]};
+template <int P, typename R>
+__device__ __forceinline__ void mfma_a_to_lds(typename MfmaT<R>::V* tabA, int s, int lane) {
+    constexpr int NP = n_modes(P), NQ = n_quad_vol(P), NQ1 = P + 1, NPT = 3 * NQ1;
+    const TabP<R, P>& T = tab<R, P>();
+    const int g = lane >> 4, j = lane & 15;
+    const int qj = MfmaT<R>::qrow(j);  // the point of A row j
+    const int m = MfmaT<R>::pos(g, s), q = MfmaT<R>::qpos(g, s);
+    R* t = reinterpret_cast<R*>(tabA + lane) + s;
+    constexpr int SLOT = 64 * 4;
+    // (loads unconditional with clamped indices, so that none waits for another)
+    const int mc = min(m, NP - 1), jc = min(j, NP - 1), qc = min(q, NQ - 1), fc = min(q, NPT - 1);
+    const int qjc = min(qj, NQ - 1), fjc = min(qj, NPT - 1);
+    const R vol = T.B[mc][qjc], tr = T.S[fjc / NQ1][mc][fjc % NQ1];
+    const R sp = T.S[fc / NQ1][jc][fc % NQ1] * T.W1[fc % NQ1], gx = T.Gx[jc][qc], gy = T.Gy[jc][qc];
+    t[MFMA_A_VOL * SLOT] = (m < NP && qj < NQ) ? vol : R(0);
+    t[MFMA_A_TR * SLOT] = (m < NP && qj < NPT) ? tr : R(0);
+    t[MFMA_A_SP * SLOT] = (j < NP && q < NPT) ? sp : R(0);
+    t[MFMA_A_GX * SLOT] = (j < NP && q < NQ) ? gx : R(0);
+    t[MFMA_A_GY * SLOT] = (j < NP && q < NQ) ? gy : R(0);
 }
 
 // State operands of one tile held by one wavefront: its own sub-tile, and
