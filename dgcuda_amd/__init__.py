@@ -33,7 +33,7 @@ DG_QUIRK_FLOAT_SQRT, DG_QUIRK_FLOAT_GEOM, DG_QUIRK_FLOAT_POW, DG_QUIRK_REFLECT_M
 DG_GMSH_QUIRKS, DG_GMSH_PERIODIC = 1, 2
 DG_BATCH_ONE_LAUNCH, DG_BATCH_PER_CLASS = 0, 1
 # the launch form a batch takes until one is set, per precision (in FP32 from
-# 65,536 triangles on; below, one launch)
+# 81,920 triangles on; below, one launch)
 BATCH_DEFAULT_LAUNCH_MODE = {DG_FP32: DG_BATCH_PER_CLASS, DG_FP64: DG_BATCH_PER_CLASS}
 STATUS_NAMES = {0: "DG_OK", 1: "DG_ERR_ARG", 2: "DG_ERR_IO", 3: "DG_ERR_PARSE", 4: "DG_ERR_HIP",
                 5: "DG_ERR_UNSUPPORTED", 6: "DG_ERR_NUMERIC", 7: "DG_ERR_BUDGET", 8: "DG_ERR_STATE"}
@@ -519,7 +519,7 @@ class Batch:
         """DG_BATCH_ONE_LAUNCH (one persistent launch per stage) or
         DG_BATCH_PER_CLASS (one per kernel class and stage, side by side);
         from the next run on.  Until set: per class in FP64 and, in FP32, from
-        65,536 triangles on."""
+        81,920 triangles on."""
         _check(lib().dg_batch_set_launch_mode(self._h, mode))
 
     def launch_info(self):

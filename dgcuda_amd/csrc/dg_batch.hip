@@ -43,7 +43,7 @@ struct SlotDesc {
     const void* lface;
     const void* lmetric;
     Ctrl* ctrl;
-    int K, Kp, N, p, hcap, tcap, cls;  // cls: the solve's class (BM_* bit)
+    int K, Kp, N, p, hcap, tcap, solo;  // solo: runs its own kernels
     PhysP phys;
 };
 
@@ -76,6 +76,40 @@ __device__ __forceinline__ int run_tile(const int2* __restrict__ items, int x, i
     return uni(v.x) == slot ? uni(v.y) : fallback;
 }
 
+// A work item's view of its solve's step, as StageStep in a single solve:
+// the first stage's items compute dt themselves and the item of the solve's
+// first tile notes the step, the last stage's ends it (a dt kernel per step
+// before: 24 solves of up to 2,000 triangles 49.8 -> 46.9 us per step, 64 of up
+// to 200,000 in one launch 799 -> 783).
+template <typename R, int KIND>
+struct ItemStep {
+    Ctrl* ctrl;
+    const bool notes;
+    StepSlot slot;
+    __device__ __forceinline__ ItemStep(Ctrl* c, int tile) : ctrl(c), notes(tile == 0), slot{} {
+        if constexpr (first_stage(KIND)) slot = step_slot(ctrl);
+    }
+    // whether the solve has work in this stage (uniform)
+    __device__ __forceinline__ static bool active(Ctrl* c, int tile) {
+        if constexpr (!first_stage(KIND)) return cview(c)->active != 0;
+        if (!step_not_taken(c)) return true;
+        if (tile == 0 && threadIdx.x == 0) step_stop(c);
+        return false;
+    }
+    // every lane of a wavefront calls it
+    __device__ __forceinline__ R dt() const {
+        if constexpr (first_stage(KIND))
+            return (R)step_start(ctrl, slot, notes && threadIdx.x < 64);
+        else
+            return (R)cview(ctrl)->dt;
+    }
+    // end of the last stage's item or run: one thread of the workgroup
+    __device__ __forceinline__ static void commit(Ctrl* c, double mx, int tile) {
+        lam_commit_step(mx, c);
+        if (tile == 0) step_finish(c);
+    }
+};
+
 // One workgroup's run of consecutive items of the same solve (items it,
 // it+G8, ... while they belong to `slot`) through the pipelined tile body of
 // the single-solve kernel (the same arithmetic, so a batched solve equals
@@ -88,8 +122,8 @@ __device__ __forceinline__ int batch_mfma_run(const StageArgs<R>& a, const MfmaA
                                               typename MfmaT<R>::V* fd, R* ts, typename MfmaT<R>::V* tabA,
                                               double& lam) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, j = lane & 15;
-    const R dt = (R)uni(a.ctrl->dt);
     int tile = uni(items[it].y);
+    const ItemStep<R, KIND> step(a.ctrl, tile);
     int n1 = run_tile(items, it + G8, i1, slot, tile);
     MfmaTileState<N, P, R> st;
     int hid[MfmaTileState<N, P, R>::HPW];
@@ -99,6 +133,7 @@ __device__ __forceinline__ int batch_mfma_run(const StageArgs<R>& a, const MfmaA
     st.load_data(a.u, a.K, tile, w, g, j, hid);
     MfmaTileState<N, P, R>::load_ids(mx.halo, mx.hcap, n1, w, j, hid);
     mfma_a_to_lds<P, R>(tabA, w, lane);  // the previous run ended with a barrier
+    const R dt = step.dt();
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     while (true) {
@@ -130,7 +165,7 @@ __device__ __forceinline__ StageArgs<R> slot_args(const SlotDesc<R>* sd) {
     a.ntiles = 0;
     a.xcd_remap = 0;
     a.stream = 0;
-    a.in_step = 0;  // k_batch_dt starts the step
+    a.in_step = 0;  // its items start the step themselves (ItemStep)
     a.bnd = nullptr;  // batched solves have no boundary sides
     a.phys.gamma = uni(sd->phys.gamma);
     a.phys.ax = uni(sd->phys.ax);
@@ -178,8 +213,7 @@ enum : int {
     BM_TILE_EUL = 8,
     BM_LANES = BM_LANE_ADV | BM_LANE_EUL,
     BM_TILES = BM_TILE_ADV | BM_TILE_EUL,
-    BM_ALL = BM_LANES | BM_TILES,
-    BM_SOLO = 16  // class of the solves that run their own kernels
+    BM_ALL = BM_LANES | BM_TILES
 };
 
 // Work lists in `parts` (XCD x = blockIdx % 8), 9 bounds per list:
@@ -209,13 +243,15 @@ __device__ __forceinline__ void batch_lane_items(const SlotDesc<R>* __restrict__
     for (; it < i1; it += G8) {
         const int2 item = items[it];
         const SlotDesc<R>* sd = slots + uni(item.x);
-        if (!uni(uni(sd->ctrl)->active)) continue;
+        const int tile = uni(item.y);
+        if (!ItemStep<R, KIND>::active(uni(sd->ctrl), tile)) continue;
         const StageArgs<R> a = slot_args<R, KIND>(sd);
         const int N = uni(sd->N), p = uni(sd->p);
-        const int e = uni(item.y) * BATCH_VALU_TILE + threadIdx.x;
+        const int e = tile * BATCH_VALU_TILE + threadIdx.x;
         double lam = 0.0;
         const auto go = [] { return true; };  // asked above
-        const auto dt = [&] { return (R)a.ctrl->dt; };
+        const ItemStep<R, KIND> step(a.ctrl, tile);
+        const auto dt = [&] { return step.dt(); };
         if constexpr (EUL) {
             // with the non-temporal hint: 1-2% faster per step than without
             // on ragged batches of 24, 32 and 64 solves
@@ -223,12 +259,12 @@ __device__ __forceinline__ void batch_lane_items(const SlotDesc<R>* __restrict__
             else if (N == 4 && p == 1) lam = lane_process<1, KIND, R, false, true>(a, e, lt1, go, dt);
         }
         if constexpr (ADV) {
-            if (N == 1 && p == 2) lam = valu_process<1, 2, R>(a, e, KIND);
-            else if (N == 1 && p == 1) lam = valu_process<1, 1, R>(a, e, KIND);
+            if (N == 1 && p == 2) lam = valu_process<1, 2, R, false, false>(a, e, KIND, dt);
+            else if (N == 1 && p == 1) lam = valu_process<1, 1, R, false, false>(a, e, KIND, dt);
         }
         if constexpr (LAST) {
             const double m = block_max(lam, sh);
-            if (threadIdx.x == 0) lam_commit_step(m, a.ctrl);
+            if (threadIdx.x == 0) ItemStep<R, KIND>::commit(a.ctrl, m, tile);
             __syncthreads();  // sh is reused by the next item
         }
     }
@@ -243,9 +279,9 @@ __device__ __forceinline__ void batch_tile_items(const SlotDesc<R>* __restrict__
                                                  double* sh) {
     constexpr bool LAST = (KIND == ST_RK4_4 || KIND == ST_RK2_2);
     while (it < i1) {
-        const int slot = uni(items[it].x);
+        const int slot = uni(items[it].x), tile = uni(items[it].y);
         const SlotDesc<R>* sd = slots + slot;
-        if (!uni(uni(sd->ctrl)->active)) {
+        if (!ItemStep<R, KIND>::active(uni(sd->ctrl), tile)) {
             it += G8;
             continue;
         }
@@ -271,7 +307,7 @@ __device__ __forceinline__ void batch_tile_items(const SlotDesc<R>* __restrict__
         it = next;
         if constexpr (LAST) {
             const double m = block_max(lam, sh);
-            if (threadIdx.x == 0) lam_commit_step(m, a.ctrl);
+            if (threadIdx.x == 0) ItemStep<R, KIND>::commit(a.ctrl, m, tile);
             __syncthreads();  // sh is reused by the next run
         }
     }
@@ -356,11 +392,11 @@ const void* batch_stage_fn(int kind, int mask) {
     }
 }
 
-// starts a step of the solves of `classes`
+// starts a step of the solves that run their own kernels
 template <typename R>
-__global__ void k_batch_dt(const SlotDesc<R>* __restrict__ slots, const int* __restrict__ nslots, int classes) {
+__global__ void k_batch_dt(const SlotDesc<R>* __restrict__ slots, const int* __restrict__ nslots) {
     const int s = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);  // one wavefront per slot
-    if (s < *nslots && (slots[s].cls & classes)) dt_update(slots[s].ctrl);
+    if (s < *nslots && slots[s].solo) dt_update(slots[s].ctrl);
 }
 
 // every slot's control block into one array (one host copy)
@@ -425,7 +461,7 @@ class EngineT : public BatchEngine {
     int form = -1;
     bool per_class = false;          // form of the current work list
     static constexpr int PER_CLASS_GROUPS = 2;
-    static constexpr int64_t PER_CLASS_MIN = 65536;
+    static constexpr int64_t PER_CLASS_MIN = 81920;
     std::vector<Launch> launches;    // the batch kernels of a stage, in launch order
     std::vector<int2> raw_items[BATCH_LISTS];  // the work lists in solve order, and
     std::vector<double> raw_cost[BATCH_LISTS]; // each item's estimated cost
@@ -541,11 +577,12 @@ class EngineT : public BatchEngine {
 
     // The automatic form.  One kernel per class, side by side, holds more
     // wavefronts per SIMD and its stages wait for their own class only; one
-    // kernel for all has one chain of launches.  One launch / per class, us per
-    // step, FP32 ragged batches: 22,880 triangles 49.6 / 67.4, 41,470 63.6 /
-    // 67.5, 51,414 69.6 / 70.7, 66,568 80.6 / 75.3, 93,950 117.3 / 98.3, 453,104
-    // 267 / 255, 1,748,140 800 / 657; FP64 24 solves of up to 2,000 triangles
-    // 104.4 / 84.7, 453,104 622 / 466, 1,748,140 2,035 / 1,313.
+    // kernel for all has one chain of launches, and the four chains cost the
+    // host about 70-85 us per step to launch.  One launch / per class, us per
+    // step, FP32 ragged batches: 22,880 triangles 46.9 / 73, 41,470 59.5 / 73,
+    // 51,414 65.6 / 77, 66,568 76 / 84, 88,120 98 / 87, 93,950 110 / 92, 453,104
+    // 267 / 255, 1,748,140 783 / 640; FP64 24 solves of up to 2,000 triangles
+    // 104 / 85, 453,104 622 / 466, 1,748,140 2,035 / 1,313.
     // (A served set crosses the line down only at half of it: a change of form
     // captures the step again.)
     bool per_class_form(const std::vector<Solver*>& solvers) const {
@@ -646,13 +683,12 @@ class EngineT : public BatchEngine {
             d.hcap = si.hcap;
             d.tcap = si.tcap;
             d.phys = si.phys;
+            d.solo = solo_here ? 1 : 0;
             if (solo_here) {
-                d.cls = BM_SOLO;
                 new_solo.push_back(solvers[s]);  // slot kept for dt and status; no work items
                 continue;
             }
             const int bit = class_of(si);
-            d.cls = bit;
             const int l = list_of[bit];
             if (tiles) hmax[l] = std::max(hmax[l], si.hcap);
             const int te = tiles ? MFMA_TILE : BATCH_VALU_TILE;
@@ -717,9 +753,7 @@ class EngineT : public BatchEngine {
     }
 
     // the stages' launches of one step of launch L's solves on stream q
-    Status launch_step(const Launch& L, int classes, hipStream_t q) {
-        hipLaunchKernelGGL((k_batch_dt<R>), dim3(dt_grid), dim3(256), 0, q, d_slots, d_xcd + BATCH_NSLOT_AT, classes);
-        HIPST(hipGetLastError());
+    Status launch_step(const Launch& L, hipStream_t q) {
         for (int k : {ST_RK4_1, ST_RK4_2, ST_RK4_3, ST_RK4_4}) {
             const void* fn = batch_stage_fn<R>(k, L.mask);
             if (!fn) return Status::err(DG_ERR_ARG, "unsupported batch stage");
@@ -734,8 +768,7 @@ class EngineT : public BatchEngine {
 
     // one step of the solves that run their own kernels
     Status solo_step() {
-        hipLaunchKernelGGL((k_batch_dt<R>), dim3(dt_grid), dim3(256), 0, st, d_slots, d_xcd + BATCH_NSLOT_AT,
-                           (int)BM_SOLO);
+        hipLaunchKernelGGL((k_batch_dt<R>), dim3(dt_grid), dim3(256), 0, st, d_slots, d_xcd + BATCH_NSLOT_AT);
         HIPST(hipGetLastError());
         Status s0;
         for (int k : {ST_RK4_1, ST_RK4_2, ST_RK4_3, ST_RK4_4})
@@ -757,7 +790,7 @@ class EngineT : public BatchEngine {
         for (int b = 1; b < nb; b++) HIPST(hipStreamWaitEvent(side[b - 1], fork, 0));
         for (int b = 0; b < nb; b++)
             for (int i = 0; i < n; i++)
-                if (!(s0 = launch_step(launches[b], launches[b].mask, b ? side[b - 1] : st))) return s0;
+                if (!(s0 = launch_step(launches[b], b ? side[b - 1] : st))) return s0;
         if (!solo.empty())
             for (int i = 0; i < n; i++)
                 if (!(s0 = solo_step())) return s0;

@@ -179,7 +179,8 @@ __device__ __forceinline__ double step_size(Ctrl* c, double mx, double* t_next) 
     return dt;
 }
 
-// The step's start as a kernel of its own (batches).  One wavefront.
+// The step's start as a kernel of its own (solves of a batch that run their
+// own kernels).  One wavefront.
 __device__ __forceinline__ void dt_update(Ctrl* ctrl) {
     const bool first = (threadIdx.x & 63) == 0;
     if (step_not_taken(ctrl)) {
@@ -218,14 +219,15 @@ __device__ __forceinline__ StepSlot step_slot(Ctrl* ctrl) {
     const unsigned long long* s = lam_slots(ctrl);
     return StepSlot{{lam_slot(s), lam_slot(s + LAM_SIDE)}};
 }
-__device__ __forceinline__ double step_start(Ctrl* ctrl, const StepSlot& slot) {
+// `notes`: this wavefront notes the step (one of the launch)
+__device__ __forceinline__ double step_start(Ctrl* ctrl, const StepSlot& slot, bool notes) {
     const int side = cview(lam_side(ctrl))->current;
     const double mx = lam_reduce(side ? slot.v[1] : slot.v[0]);
     double t;
     const double dt = step_size(ctrl, mx, &t);
-    if (blockIdx.x == 0 && threadIdx.x < 64) {
+    if (notes) {
         lam_clear(lam_slots(ctrl) + (1 - side) * LAM_SIDE);
-        if (threadIdx.x == 0) {
+        if ((threadIdx.x & 63) == 0) {
             ctrl->dt = dt;
             ctrl->t_next = t;
             ctrl->lam_bits = (unsigned long long)__double_as_longlong(mx);
@@ -466,7 +468,9 @@ struct StageStep {
         return false;
     }
     // the stage's dt (every lane of a wavefront calls it)
-    __device__ __forceinline__ R dt() const { return (R)(start ? step_start(a.ctrl, slot) : cview(a.ctrl)->dt); }
+    __device__ __forceinline__ R dt() const {
+        return (R)(start ? step_start(a.ctrl, slot, blockIdx.x == 0 && threadIdx.x < 64) : cview(a.ctrl)->dt);
+    }
 };
 // keeps loads that come before it before it
 #define DG_LOADS_FIRST() asm volatile("" ::: "memory")

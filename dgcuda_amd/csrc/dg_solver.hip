@@ -3,9 +3,9 @@
 //
 // The reference's time loop (src/2d/conservation/time_integrator.cu:221-434)
 // launches four kernels per stage and copies every element's wave speed to
-// the host each step to pick dt.  Here a step is one small dt kernel plus one
-// fused launch per stage; dt never leaves the device, and the host only
-// synchronises once per chunk of steps to test for t >= t_end.
+// the host each step to pick dt.  Here a step is one fused launch per stage;
+// dt never leaves the device, and the host only synchronises once per chunk
+// of steps to test for t >= t_end.
 #include <algorithm>
 #include <atomic>
 #include <cstdlib>

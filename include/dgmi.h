@@ -356,7 +356,7 @@ int dg_batch_info(const dg_batch* b, int* n_solves, int64_t* total_elems, int64_
  * not depend on it.  Test and tuning aid; no counterpart in the reference. */
 int dg_batch_set_max_groups(dg_batch* b, int max_groups);
 /* How a stage of the batch is launched; takes effect at the next run.  Until
- * it is set the batch chooses: per class in FP64 and, in FP32, from 65,536
+ * it is set the batch chooses: per class in FP64 and, in FP32, from 81,920
  * triangles on.
  * DG_BATCH_ONE_LAUNCH: a single persistent launch per
  * stage carrying every body, at the register budget of the largest;

@@ -27,7 +27,7 @@ def cases(sizes, boundary):
 @pytest.mark.parametrize("prec", [dg.DG_FP32, dg.DG_FP64])
 @pytest.mark.parametrize("sizes,boundary", [
     ((9, 5, 12, 7, 16, 8, 11, 13), True),      # every class, below the line
-    ((90, 70, 60, 64, 100, 33, 80, 47), False),  # above it
+    ((90, 70, 60, 64, 110, 33, 80, 47), False),  # above it
     ((20, 21), False),                         # two classes
     ((17,), False),                            # one class
 ])
