@@ -1,11 +1,10 @@
 // Many independent solves of uneven size and mixed order advanced together:
 // persistent launches per RK stage over device-side work lists of (solve,
-// tile) items, the step (per-solve dt kernel + the stage launches) replayed
+// tile) items, the step (the stage launches) replayed
 // from a hipGraph.  Two launch forms: one kernel per stage carrying every
-// class (the FP32 default), or one launch per stage for each kernel class
-// present (Euler tiles, advection tiles, Euler lane items, advection lane
-// items), each at the occupancy its own bodies allow (the FP64 default: the
-// all-class FP64 kernel holds one wavefront per SIMD).
+// class, or one launch per stage for each kernel class present (Euler tiles,
+// advection tiles, Euler lane items, advection lane items), the classes side
+// by side and each at the occupancy its own bodies allow.
 //
 // Every solve keeps its own buffers, geometry and control block (its own
 // CFL dt, time and end time), so a solve's arithmetic does not depend on
@@ -478,7 +477,10 @@ class EngineT : public BatchEngine {
     ~EngineT() override {
         if (st) (void)hipStreamSynchronize(st);
         graph.drop();
-        for (hipStream_t q : side) pool_release_stream(q);
+        for (hipStream_t q : side) {
+            (void)hipStreamSynchronize(q);
+            pool_release_stream(q);
+        }
         for (hipEvent_t e : join) (void)hipEventDestroy(e);
         if (fork) (void)hipEventDestroy(fork);
         void* b[] = {d_slots, d_items, d_xcd, d_status, d_ctrls};

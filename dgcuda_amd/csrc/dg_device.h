@@ -93,8 +93,8 @@ struct Ctrl {
 // Maximum cell wave speed of the current state: LAM_SLOTS partial maxima
 // behind the control block, each the bit pattern of a non-negative double
 // (ordered like the value) on a line of its own.  A workgroup commits with
-// one atomic max to the slot of its number; the dt kernel reduces the slots
-// and clears them.  One address for all workgroups made the last stage wait
+// one atomic max to the slot of its number; the next step's start reduces the
+// slots.  One address for all workgroups made the last stage wait
 // for its atomics, which the memory takes one after another (about 35 ns
 // each: 4,096 workgroups of the lane kernel, Euler p = 1 at 524,288
 // triangles, a step of 4 stages 167 us; with 64 slots 133 us).
