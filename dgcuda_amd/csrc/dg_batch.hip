@@ -2,9 +2,9 @@
 // persistent launches per RK stage over device-side work lists of (solve,
 // tile) items, the step (the stage launches) replayed
 // from a hipGraph.  Two launch forms: one kernel per stage carrying every
-// class, or one launch per stage for each kernel class present (Euler tiles,
-// advection tiles, Euler lane items, advection lane items), the classes side
-// by side and each at the occupancy its own bodies allow.
+// class (the FP32 default), or one launch per stage for each kernel class
+// present (Euler tiles, advection tiles, Euler lane items, advection lane
+// items), each at the occupancy its own bodies allow (the FP64 default).
 //
 // Every solve keeps its own buffers, geometry and control block (its own
 // CFL dt, time and end time), so a solve's arithmetic does not depend on
@@ -201,7 +201,7 @@ __device__ __forceinline__ StageArgs<R> slot_args(const SlotDesc<R>* sd) {
 //   one launch: BM_ALL, so light (advection) and heavy (Euler) items share
 //     the CUs;
 //   per class: one launch per class, each with the register budget of its
-//     own bodies and on a stream of its own (enqueue_steps).
+//     own bodies.
 // A kernel's register allocation, and with it the wavefronts a SIMD holds,
 // is that of the bodies it carries (FP64: Euler tiles alone 2 wavefronts per
 // SIMD, every body together 1).
@@ -453,23 +453,16 @@ class EngineT : public BatchEngine {
     int cap_slots = 0, cap_items = 0;
     int nslots = 0, nitems = 0, dt_grid = 0, cus = 0;
     int max_groups_req = 0;          // set_max_groups (0: no cap)
-    // set_launch_form (-1: automatic, per_class_form).  Several launches run
-    // side by side, so a CU's registers are shared: capped at two workgroups
-    // per CU each (PER_CLASS_GROUPS), 1-5% faster per step than every workgroup
-    // that fits alone, one per CU 3-10% slower (4 to 64 ragged solves).
-    int form = -1;
-    bool per_class = false;          // form of the current work list
-    static constexpr int PER_CLASS_GROUPS = 2;
-    static constexpr int64_t PER_CLASS_MIN = 81920;
+    // set_launch_form; the default is the form measured faster on the
+    // 64-solve ragged mix in each precision (one launch / per class, us per
+    // step: FP32 939 / 1,083, FP64 2,476 / 2,193; now 783 in FP32's one launch)
+    int form = sizeof(R) == 8 ? DG_BATCH_PER_CLASS : DG_BATCH_ONE_LAUNCH;
     std::vector<Launch> launches;    // the batch kernels of a stage, in launch order
     std::vector<int2> raw_items[BATCH_LISTS];  // the work lists in solve order, and
     std::vector<double> raw_cost[BATCH_LISTS]; // each item's estimated cost
     std::vector<int2> h_items;       // host copy of the work lists and their XCD bounds
     std::vector<int> h_parts;
     StepGraph graph;
-    std::vector<hipStream_t> side;   // streams of the second and further launches
-    std::vector<hipEvent_t> join;    // their ends
-    hipEvent_t fork = nullptr;
     int solo_min = 0;             // 0: every solve in the batch launch
     std::vector<Solver*> solo;    // solves launched with their own kernels
     std::vector<uint64_t> solo_uid;  // their ids: the captured step holds their buffers
@@ -477,12 +470,6 @@ class EngineT : public BatchEngine {
     ~EngineT() override {
         if (st) (void)hipStreamSynchronize(st);
         graph.drop();
-        for (hipStream_t q : side) {
-            (void)hipStreamSynchronize(q);
-            pool_release_stream(q);
-        }
-        for (hipEvent_t e : join) (void)hipEventDestroy(e);
-        if (fork) (void)hipEventDestroy(fork);
         void* b[] = {d_slots, d_items, d_xcd, d_status, d_ctrls};
         for (void* q : b)
             if (q) hipFree(q);
@@ -567,7 +554,7 @@ class EngineT : public BatchEngine {
     // the masks of the form's launches, in launch order (Euler tiles first:
     // the longest items start earliest)
     std::vector<int> form_masks() const {
-        if (per_class) return {BM_TILE_EUL, BM_TILE_ADV, BM_LANE_EUL, BM_LANE_ADV};
+        if (form == DG_BATCH_PER_CLASS) return {BM_TILE_EUL, BM_TILE_ADV, BM_LANE_EUL, BM_LANE_ADV};
         return {BM_ALL};
     }
 
@@ -576,28 +563,6 @@ class EngineT : public BatchEngine {
         return si.N == 4 ? BM_LANE_EUL : BM_LANE_ADV;
     }
     bool runs_solo(const SlotInfo& si) const { return si.boundary || (solo_min > 0 && si.K >= solo_min); }
-
-    // The automatic form.  One kernel per class, side by side, holds more
-    // wavefronts per SIMD and its stages wait for their own class only; one
-    // kernel for all has one chain of launches, and the four chains cost the
-    // host about 70-85 us per step to launch.  One launch / per class, us per
-    // step, FP32 ragged batches: 22,880 triangles 46.9 / 73, 41,470 59.5 / 73,
-    // 51,414 65.6 / 77, 66,568 76 / 84, 88,120 98 / 87, 93,950 110 / 92, 453,104
-    // 267 / 255, 1,748,140 783 / 640; FP64 24 solves of up to 2,000 triangles
-    // 104 / 85, 453,104 622 / 466, 1,748,140 2,035 / 1,313.
-    // (A served set crosses the line down only at half of it: a change of form
-    // captures the step again.)
-    bool per_class_form(const std::vector<Solver*>& solvers) const {
-        if (form >= 0) return form == DG_BATCH_PER_CLASS;
-        if (sizeof(R) == 8) return true;
-        int64_t elems = 0;
-        for (Solver* sv : solvers) {
-            SlotInfo si;
-            sv->slot_info(&si);
-            if (!runs_solo(si)) elems += si.K;
-        }
-        return elems >= (per_class ? PER_CLASS_MIN / 2 : PER_CLASS_MIN);
-    }
 
     // Splits each list into 8 contiguous chunks of equal estimated cost, one
     // per XCD, and uploads the lists with their bounds (stream-ordered;
@@ -622,7 +587,6 @@ class EngineT : public BatchEngine {
     }
 
     Status set_slots(const std::vector<Solver*>& solvers) override {
-        per_class = per_class_form(solvers);
         const int ns = (int)solvers.size();
         std::vector<Solver*> new_solo;
         std::vector<SlotDesc<R>> hs(ns);
@@ -711,21 +675,6 @@ class EngineT : public BatchEngine {
             if (!sh) return sh;
             nl.push_back(L);
         }
-        if (nl.size() > 1)
-            for (Launch& L : nl) {
-                L.resident = std::min(L.resident, PER_CLASS_GROUPS * cus / 8 * 8);
-                L.grid = std::min(L.grid, L.resident);
-            }
-        for (size_t b = side.size() + 1; b < nl.size(); b++) {
-            hipStream_t q = nullptr;
-            Status sq = pool_stream(&q);
-            if (!sq) return sq;
-            side.push_back(q);
-            hipEvent_t e = nullptr;
-            HIPST(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-            join.push_back(e);
-        }
-        if (nl.size() > 1 && !fork) HIPST(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
         if (nl != launches) {
             launches = nl;
             drop_graph();
@@ -754,51 +703,31 @@ class EngineT : public BatchEngine {
         return Status::ok();
     }
 
-    // the stages' launches of one step of launch L's solves on stream q
-    Status launch_step(const Launch& L, hipStream_t q) {
-        for (int k : {ST_RK4_1, ST_RK4_2, ST_RK4_3, ST_RK4_4}) {
-            const void* fn = batch_stage_fn<R>(k, L.mask);
+    Status launch_stage(int kind) {
+        for (const Launch& L : launches) {
+            const void* fn = batch_stage_fn<R>(kind, L.mask);
             if (!fn) return Status::err(DG_ERR_ARG, "unsupported batch stage");
             const SlotDesc<R>* slots = d_slots;
             const int2* items = d_items;
             const int* parts = d_xcd + 9 * L.list;
             void* args[] = {(void*)&slots, (void*)&items, (void*)&parts};
-            HIPST(hipLaunchKernel(fn, dim3(L.grid), dim3(256), args, L.lds, q));
+            HIPST(hipLaunchKernel(fn, dim3(L.grid), dim3(256), args, L.lds, st));
         }
         return Status::ok();
     }
 
-    // one step of the solves that run their own kernels
-    Status solo_step() {
-        hipLaunchKernelGGL((k_batch_dt<R>), dim3(dt_grid), dim3(256), 0, st, d_slots, d_xcd + BATCH_NSLOT_AT);
-        HIPST(hipGetLastError());
-        Status s0;
-        for (int k : {ST_RK4_1, ST_RK4_2, ST_RK4_3, ST_RK4_4})
-            for (Solver* sv : solo)
-                if (!(s0 = sv->stage_on(k, st))) return s0;
-        return s0;
-    }
-
-    // n steps on the engine's stream.  Solves do not depend on each other, so
-    // each launch's solves advance the n steps on a stream of their own
-    // (branches of the captured graph) and meet at the end: one class's tail
-    // and launch gap are filled by the others.  Per-class launches one behind
-    // the other -> side by side: FP64 64 solves of up to 200,000 triangles 1,996
-    // -> 1,338 us per step, 32 of up to 100,000 FP32 292 (one launch) -> 267.
     Status enqueue_steps(int n) {
         Status s0;
-        const int nb = (int)launches.size();
-        if (nb > 1) HIPST(hipEventRecord(fork, st));
-        for (int b = 1; b < nb; b++) HIPST(hipStreamWaitEvent(side[b - 1], fork, 0));
-        for (int b = 0; b < nb; b++)
-            for (int i = 0; i < n; i++)
-                if (!(s0 = launch_step(launches[b], b ? side[b - 1] : st))) return s0;
-        if (!solo.empty())
-            for (int i = 0; i < n; i++)
-                if (!(s0 = solo_step())) return s0;
-        for (int b = 1; b < nb; b++) {
-            HIPST(hipEventRecord(join[b - 1], side[b - 1]));
-            HIPST(hipStreamWaitEvent(st, join[b - 1], 0));
+        for (int i = 0; i < n; i++) {
+            if (!solo.empty()) {
+                hipLaunchKernelGGL((k_batch_dt<R>), dim3(dt_grid), dim3(256), 0, st, d_slots, d_xcd + BATCH_NSLOT_AT);
+                HIPST(hipGetLastError());
+            }
+            for (int k : {ST_RK4_1, ST_RK4_2, ST_RK4_3, ST_RK4_4}) {
+                if (!(s0 = launch_stage(k))) return s0;
+                for (Solver* sv : solo)
+                    if (!(s0 = sv->stage_on(k, st))) return s0;
+            }
         }
         return Status::ok();
     }

@@ -1,6 +1,6 @@
-"""A batch's launch forms: the form it chooses by itself on both sides of its
-size line, one launch, and per class on streams of their own, over captured
-graphs of one and of eight steps and over direct launches.  The kernels do
+"""A batch's launch forms: its default, one launch, and per class, on small
+and large batches, over captured graphs of one and of eight steps and over
+direct launches.  The kernels do
 the same arithmetic per solve in every form, so results are equal bit for
 bit."""
 import numpy as np
@@ -26,8 +26,8 @@ def cases(sizes, boundary):
 
 @pytest.mark.parametrize("prec", [dg.DG_FP32, dg.DG_FP64])
 @pytest.mark.parametrize("sizes,boundary", [
-    ((9, 5, 12, 7, 16, 8, 11, 13), True),      # every class, below the line
-    ((90, 70, 60, 64, 110, 33, 80, 47), False),  # above it
+    ((9, 5, 12, 7, 16, 8, 11, 13), True),      # every class, small
+    ((90, 70, 60, 64, 110, 33, 80, 47), False),  # large
     ((20, 21), False),                         # two classes
     ((17,), False),                            # one class
 ])
