@@ -19,7 +19,7 @@ class BatchEngine {
     // kernels inside the captured step, after the batch launch.
     virtual void set_solo_threshold(int min_elems) = 0;
     // DG_BATCH_ONE_LAUNCH or DG_BATCH_PER_CLASS (dgmi.h): which persistent
-    // launches a stage runs.
+    // launches a stage runs; until set, the faster by size.
     // Takes effect at the next set_slots.
     virtual void set_launch_form(int form) = 0;
     // enqueues n steps (per-solve dt + 4 stages) for every resident solve

@@ -2,9 +2,9 @@
 // persistent launches per RK stage over device-side work lists of (solve,
 // tile) items, the step (the stage launches) replayed
 // from a hipGraph.  Two launch forms: one kernel per stage carrying every
-// class (the FP32 default), or one launch per stage for each kernel class
+// class, or one launch per stage for each kernel class
 // present (Euler tiles, advection tiles, Euler lane items, advection lane
-// items), each at the occupancy its own bodies allow (the FP64 default).
+// items), each at the occupancy its own bodies allow (large FP64 batches).
 //
 // Every solve keeps its own buffers, geometry and control block (its own
 // CFL dt, time and end time), so a solve's arithmetic does not depend on
@@ -453,10 +453,14 @@ class EngineT : public BatchEngine {
     int cap_slots = 0, cap_items = 0;
     int nslots = 0, nitems = 0, dt_grid = 0, cus = 0;
     int max_groups_req = 0;          // set_max_groups (0: no cap)
-    // set_launch_form; the default is the form measured faster on the
-    // 64-solve ragged mix in each precision (one launch / per class, us per
-    // step: FP32 939 / 1,083, FP64 2,476 / 2,193; now 783 in FP32's one launch)
-    int form = sizeof(R) == 8 ? DG_BATCH_PER_CLASS : DG_BATCH_ONE_LAUNCH;
+    // set_launch_form (-1: the faster by size).  One launch / per class, us per
+    // step, ragged batches: FP32 24 solves of up to 2,000 triangles 45 / 123, 32
+    // of up to 100,000 255 / 340, 64 of up to 200,000 782 / 801; FP64 22,880
+    // triangles in all 97 / 197, 453,104 607 / 632, 1,748,140 2,074 / 1,592 (the
+    // two lines cross near 520,000).
+    int form = -1;
+    bool per_class = false;  // form of the current work list
+    static constexpr int64_t PER_CLASS_MIN_FP64 = 524288;
     std::vector<Launch> launches;    // the batch kernels of a stage, in launch order
     std::vector<int2> raw_items[BATCH_LISTS];  // the work lists in solve order, and
     std::vector<double> raw_cost[BATCH_LISTS]; // each item's estimated cost
@@ -554,7 +558,7 @@ class EngineT : public BatchEngine {
     // the masks of the form's launches, in launch order (Euler tiles first:
     // the longest items start earliest)
     std::vector<int> form_masks() const {
-        if (form == DG_BATCH_PER_CLASS) return {BM_TILE_EUL, BM_TILE_ADV, BM_LANE_EUL, BM_LANE_ADV};
+        if (per_class) return {BM_TILE_EUL, BM_TILE_ADV, BM_LANE_EUL, BM_LANE_ADV};
         return {BM_ALL};
     }
 
@@ -563,6 +567,18 @@ class EngineT : public BatchEngine {
         return si.N == 4 ? BM_LANE_EUL : BM_LANE_ADV;
     }
     bool runs_solo(const SlotInfo& si) const { return si.boundary || (solo_min > 0 && si.K >= solo_min); }
+
+    bool per_class_form(const std::vector<Solver*>& solvers) const {
+        if (form >= 0) return form == DG_BATCH_PER_CLASS;
+        if (sizeof(R) == 4) return false;
+        int64_t elems = 0;
+        for (Solver* sv : solvers) {
+            SlotInfo si;
+            sv->slot_info(&si);
+            if (!runs_solo(si)) elems += si.K;
+        }
+        return elems >= PER_CLASS_MIN_FP64;
+    }
 
     // Splits each list into 8 contiguous chunks of equal estimated cost, one
     // per XCD, and uploads the lists with their bounds (stream-ordered;
@@ -587,6 +603,7 @@ class EngineT : public BatchEngine {
     }
 
     Status set_slots(const std::vector<Solver*>& solvers) override {
+        per_class = per_class_form(solvers);
         const int ns = (int)solvers.size();
         std::vector<Solver*> new_solo;
         std::vector<SlotDesc<R>> hs(ns);
