@@ -472,6 +472,13 @@ struct StageStep {
         return (R)(start ? step_start(a.ctrl, slot, blockIdx.x == 0 && threadIdx.x < 64) : cview(a.ctrl)->dt);
     }
 };
+// forms x here: the compiler moves sums whose only use lies behind a branch
+// down to it, and with them everything they are made of
+#ifdef __HIP__
+#define DG_FORM(x) asm volatile("" : "+v"(x))
+#else  // a host build of these headers
+#define DG_FORM(x)
+#endif
 // keeps loads that come before it before it
 #define DG_LOADS_FIRST() asm volatile("" ::: "memory")
 

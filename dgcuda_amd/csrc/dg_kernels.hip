@@ -24,8 +24,10 @@ DGMI_TABLE_UPLOADER(upload_tables_kernels)
 
 // BND: the variant for meshes with boundary sides (p <= VALU_BOUNDARY_MAX_P)
 // REF: the right-hand side on the caller's arrays
+// (advection p = 5 FP32 is held to the two wavefronts per SIMD it misses by
+// one register: 320,000 triangles 935 -> 656 us a step; the others spill if held)
 template <int N, int P, typename R, bool BND = false, bool REF = false>
-__global__ void __launch_bounds__(128) k_stage_valu(StageArgs<R> a) {
+__global__ void __launch_bounds__(128, (N == 1 && P == 5 && sizeof(R) == 4 ? 2 : 1)) k_stage_valu(StageArgs<R> a) {
     __shared__ double sh[8];
     if constexpr (REF) {
         const int t = tile_of_block(blockIdx.x, gridDim.x, a.xcd_remap);

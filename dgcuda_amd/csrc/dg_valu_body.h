@@ -81,6 +81,26 @@ __device__ __forceinline__ double valu_process(const StageArgs<R>& a, int e, int
             for (int m = 0; m < NP; m++) nu[v][m] = at(v, m, nb0, ob0);
     }
 
+    // Where the sums are formed before the next face begins (FORM_FACES) and
+    // before the stage's dt is asked for (FORM_LAST): left alone, the compiler
+    // moves them behind the branch in the first stage's dt and holds every
+    // face's values until then.  Us per step so moved -> formed: advection
+    // FP64 p = 2 at 320,000 triangles 184 -> 132, p = 3 at 180,000 813 -> 209,
+    // p = 5 at 320,000 12,260 -> 1,480 (2,275 spilled registers -> 13); Euler
+    // p = 5 at 8,192 FP64 1,918 -> 968, FP32 1,570 -> 407.  Where all values
+    // fit it costs, since a face's loads then wait for the sums of the one before
+    // (advection p = 1 at 2,048 21.3 -> 23.5, FP32 p = 2 27.1 -> 28.7; FP32 p = 3
+    // at 20,000 45 -> 51 with the last forming, and 9.5 -> 12.0 on the caller's
+    // arrays); at p = 5 a face's sums are formed where that leaves fewer spills.
+    constexpr bool F64 = sizeof(R) == 8;
+    constexpr bool FORM_FACES = P == 2 ? F64 : P == 3 ? F64 || !REF : P == 5 ? REF || (N == 4 && F64) : P >= 4;
+    constexpr bool FORM_LAST = P >= 4 || (P >= 2 && F64);
+    // at p = 5 dt is there from the start: its wait does not show, and its
+    // branch splits the arithmetic (advection FP32 at 320,000 triangles 699 -> 656)
+    constexpr bool DT_FIRST = P >= 5 && !REF;
+    R dt;
+    if constexpr (DT_FIRST) dt = stage_dt();
+
     // ---- volume: sum_q F(U_q) . (metric * grad phi_m) ----
     {
         const R xr = gp(a.geo_e)[ee], yr = gp(a.geo_e)[Kp + ee], xs = gp(a.geo_e)[2 * Kp + ee], ys = gp(a.geo_e)[3 * Kp + ee];
@@ -105,9 +125,16 @@ __device__ __forceinline__ double valu_process(const StageArgs<R>& a, int e, int
         }
     }
 
+    const auto form_sums = [&] {
+#pragma unroll
+        for (int v = 0; v < N; v++)
+#pragma unroll
+            for (int m = 0; m < NP; m++) DG_FORM(tot[v][m]);
+    };
     // ---- the three faces, added in face order as eval_rhs adds s1, s2, s3 ----
 #pragma unroll
     for (int f = 0; f < 3; f++) {
+        if constexpr (FORM_FACES) form_sums();
         int w;
         if constexpr (BND) {
             w = gp(a.nbr)[f * Kp + ee];
@@ -191,10 +218,10 @@ __device__ __forceinline__ double valu_process(const StageArgs<R>& a, int e, int
     }
 
     // ---- inverse mass (M = J*I; 1/J precomputed in FP64) and the RK stage update ----
-    R dt;
+    if constexpr (FORM_LAST) form_sums();
     if constexpr (REF)
         dt = (R)a.ref_dt;
-    else
+    else if constexpr (!DT_FIRST)
         dt = stage_dt();
     const R cj = gp(a.geo_e)[4 * Kp + ee] * dt;
     double lam = 0.0;
