@@ -53,6 +53,7 @@ constexpr int BATCH_VALU_TILE = 256;
 // cannot issue them as scalar loads and would keep pointers, sizes and
 // addresses in vector registers.  readfirstlane puts them in SGPRs.
 __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ float uni(float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); }
 __device__ __forceinline__ double uni(double x) {
     const unsigned long long v = __double_as_longlong(x);
     const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v);
@@ -258,8 +259,16 @@ __device__ __forceinline__ void batch_lane_items(const SlotDesc<R>* __restrict__
             else if (N == 4 && p == 1) lam = lane_process<1, KIND, R, false, true>(a, e, lt1, go, dt);
         }
         if constexpr (ADV) {
-            if (N == 1 && p == 2) lam = valu_process<1, 2, R, false, false>(a, e, KIND, dt);
-            else if (N == 1 && p == 1) lam = valu_process<1, 1, R, false, false>(a, e, KIND, dt);
+            if (N == 1) {
+                // dt formed once and in a scalar register: formed at the end of
+                // each body the first stage's kernel spilled 65 (FP32) and 240
+                // registers (FP64: 32 solves of p = 2, 1,181,766 triangles, per
+                // class 1,022 us per step, so formed 557)
+                const R d = uni(step.dt());
+                const auto dt1 = [&] { return d; };
+                if (p == 2) lam = valu_process<1, 2, R, false, false>(a, e, KIND, dt1);
+                else if (p == 1) lam = valu_process<1, 1, R, false, false>(a, e, KIND, dt1);
+            }
         }
         if constexpr (LAST) {
             const double m = block_max(lam, sh);

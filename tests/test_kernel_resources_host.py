@@ -51,3 +51,11 @@ def test_general_lane_kernels(scratch):
         key = (int(m[1]), int(m[2]), m[3])
         assert size <= LANE_BOUNDS.get(key, 0), (name, size)
     assert seen >= 40
+
+
+def test_batch_stage_kernels(scratch):
+    """Every launch form's kernel: at most a few values, kept over a run of
+    items; the bodies' own values stay in registers."""
+    sizes = {n: s for n, s in scratch.items() if "13k_batch_stageI" in n}
+    assert len(sizes) == 40  # precisions x stages x masks
+    assert max(sizes.values()) <= 128, {n: s for n, s in sizes.items() if s > 128}
