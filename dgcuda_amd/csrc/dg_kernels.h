@@ -163,9 +163,6 @@ hipError_t launch_lambda(const R* u, const StateIx& ix, int K, double b0, const 
 struct RefRows {
     double *lo, *hi;
     int split;
-    __device__ double* row(int r, int K) const {
-        return r < split ? lo + (size_t)r * K : hi + (size_t)(r - split) * K;
-    }
 };
 // reference layout (FP64, caller's order) <-> state array in layout ix
 template <typename R>
