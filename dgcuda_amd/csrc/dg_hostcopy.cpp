@@ -19,7 +19,7 @@ namespace dgmi {
 
 namespace {
 
-constexpr size_t COPY_BLOCK = size_t(1) << 20;
+constexpr size_t COPY_BLOCK = PINNED_BLOCK_BYTES;
 constexpr size_t COPY_MIN_PART = size_t(4) << 20;
 constexpr int COPY_MAX_THREADS = 4;
 constexpr size_t COPY_SMALL = size_t(64) << 10;
@@ -168,6 +168,9 @@ Status copy_parts(char* host, char* dev, size_t bytes, bool to_host, hipStream_t
 }
 
 }  // namespace
+
+Status PinnedBlock::take() { return hip_status(take_block(&p), "pinned block"); }
+PinnedBlock::~PinnedBlock() { give_block(p); }
 
 Status copy_to_host(void* dst, const void* src_dev, size_t bytes, hipStream_t st) {
     return copy_parts((char*)dst, (char*)const_cast<void*>(src_dev), bytes, true, st);

@@ -397,11 +397,17 @@ __global__ void __launch_bounds__(256) k_ref_to_state(const double* __restrict__
     if (t >= ix.N * ix.Kp) return;
     const int v = t / ix.Kp, i = t - v * ix.Kp;
     const size_t src = (size_t)perm[i];
-#pragma unroll 4
-    for (int m = 0; m < ix.NP; m++) {
-        const int r = v * ix.NP + m;
-        const double* row = r < split ? lo + (size_t)r * K : hi + (size_t)(r - split) * K;
-        dst[ix.at(v, m, i)] = (R)row[src];
+    // eight at a time: the rows may lie in host memory, about 2 us away
+    for (int m0 = 0; m0 < ix.NP; m0 += 8) {
+        double x[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int r = v * ix.NP + min(m0 + j, ix.NP - 1);
+            x[j] = (r < split ? lo + (size_t)r * K : hi + (size_t)(r - split) * K)[src];
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            if (m0 + j < ix.NP) dst[ix.at(v, m0 + j, i)] = (R)x[j];
     }
     // every slot of the layout is written: padding modes hold zeros
     for (int m = ix.NP; m < ix.slots(); m++) dst[ix.at(v, m, i)] = R(0);
