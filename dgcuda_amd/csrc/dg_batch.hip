@@ -729,7 +729,7 @@ class EngineT : public BatchEngine {
         return Status::ok();
     }
 
-    Status launch_stage(int kind) {
+    Status launch_stage(int kind, hipStream_t on) {
         for (const Launch& L : launches) {
             const void* fn = batch_stage_fn<R>(kind, L.mask);
             if (!fn) return Status::err(DG_ERR_ARG, "unsupported batch stage");
@@ -737,30 +737,31 @@ class EngineT : public BatchEngine {
             const int2* items = d_items;
             const int* parts = d_xcd + 9 * L.list;
             void* args[] = {(void*)&slots, (void*)&items, (void*)&parts};
-            HIPST(hipLaunchKernel(fn, dim3(L.grid), dim3(256), args, L.lds, st));
+            HIPST(hipLaunchKernel(fn, dim3(L.grid), dim3(256), args, L.lds, on));
         }
         return Status::ok();
     }
 
-    Status enqueue_steps(int n) {
+    Status enqueue_steps(int n, hipStream_t on) {
         Status s0;
         for (int i = 0; i < n; i++) {
             if (!solo.empty()) {
-                hipLaunchKernelGGL((k_batch_dt<R>), dim3(dt_grid), dim3(256), 0, st, d_slots, d_xcd + BATCH_NSLOT_AT);
+                hipLaunchKernelGGL((k_batch_dt<R>), dim3(dt_grid), dim3(256), 0, on, d_slots,
+                                   d_xcd + BATCH_NSLOT_AT);
                 HIPST(hipGetLastError());
             }
             for (int k : {ST_RK4_1, ST_RK4_2, ST_RK4_3, ST_RK4_4}) {
-                if (!(s0 = launch_stage(k))) return s0;
+                if (!(s0 = launch_stage(k, on))) return s0;
                 for (Solver* sv : solo)
-                    if (!(s0 = sv->stage_on(k, st))) return s0;
+                    if (!(s0 = sv->stage_on(k, on))) return s0;
             }
         }
         return Status::ok();
     }
 
     Status steps(int n, bool use_graph) override {
-        if (use_graph) return graph.run(st, n, [&](int k) { return enqueue_steps(k); });
-        return n > 0 ? enqueue_steps(n) : Status::ok();
+        if (use_graph) return graph.run(st, n, [&](int k, hipStream_t on) { return enqueue_steps(k, on); });
+        return n > 0 ? enqueue_steps(n, st) : Status::ok();
     }
 
     Status status(std::vector<double>& out) override {

@@ -776,27 +776,28 @@ class SolverT : public Solver {
 
     // The stages of one step.  in_step: the first computes the step's dt and
     // the last ends it (step_start, step_finish), else both are done already.
-    Status enqueue_stages(int scheme, bool in_step) {
+    Status enqueue_stages(int scheme, bool in_step, hipStream_t on = nullptr) {
         Status st;
         if (scheme == DG_RK2) {
-            if (!(st = stage(ST_RK2_1, c, c, ua, nullptr, in_step))) return st;
-            return stage(ST_RK2_2, ua, c, c, nullptr, in_step);
+            if (!(st = stage(ST_RK2_1, c, c, ua, on, in_step))) return st;
+            return stage(ST_RK2_2, ua, c, c, on, in_step);
         }
-        if (!(st = stage(ST_RK4_1, c, c, ua, nullptr, in_step))) return st;
-        if (!(st = stage(ST_RK4_2, ua, c, ub))) return st;
-        if (!(st = stage(ST_RK4_3, ub, c, ua))) return st;
-        return stage(ST_RK4_4, ua, c, c, nullptr, in_step);
+        if (!(st = stage(ST_RK4_1, c, c, ua, on, in_step))) return st;
+        if (!(st = stage(ST_RK4_2, ua, c, ub, on))) return st;
+        if (!(st = stage(ST_RK4_3, ub, c, ua, on))) return st;
+        return stage(ST_RK4_4, ua, c, c, on, in_step);
     }
 
     Status enqueue_cfl_steps(int n, int scheme, bool use_graph) {
-        Status st;
-        if (use_graph) {
-            if (graph_scheme != scheme) graph.drop();
-            graph_scheme = scheme;
-            return graph.run(stream, n, [&](int k) { return enqueue_cfl_steps(k, scheme, false); });
-        }
-        for (int i = 0; i < n && st; i++) st = enqueue_stages(scheme, true);
-        return st;
+        const auto enqueue = [&](int k, hipStream_t on) {
+            Status st;
+            for (int i = 0; i < k && st; i++) st = enqueue_stages(scheme, true, on);
+            return st;
+        };
+        if (!use_graph) return enqueue(n, stream);
+        if (graph_scheme != scheme) graph.drop();
+        graph_scheme = scheme;
+        return graph.run(stream, n, enqueue);
     }
 
     Status begin_run(double t_end, bool has_end, double cfl, hipStream_t on = nullptr) {

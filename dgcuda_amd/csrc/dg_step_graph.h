@@ -26,7 +26,7 @@ class StepGraph {
         taken = 0;
     }
 
-    // `n` steps on stream `st`; `enqueue(k)` puts k steps on it
+    // `n` steps on stream `st`; `enqueue(k, on)` puts k steps on stream `on`
     template <typename F>
     Status run(hipStream_t st, int64_t n, F&& enqueue) {
         while (n > 0) {
@@ -34,7 +34,7 @@ class StepGraph {
             hipGraphExec_t& g = long_graph ? many : one;
             const int len = long_graph ? MANY : 1;
             if (!g) {
-                Status s = capture(st, len, g, enqueue);
+                Status s = capture(len, g, enqueue);
                 if (!s) return s;
             }
             hipError_t e = hipGraphLaunch(g, st);
@@ -49,13 +49,22 @@ class StepGraph {
     hipGraphExec_t one = nullptr, many = nullptr;
     int64_t taken = 0;
 
+    // On a stream of its own: the solve's stream may be in use meanwhile (a
+    // thread reading the state during a run; the long graph is captured in
+    // the middle of one), and a wait for a stream that is being captured fails.
     template <typename F>
-    static Status capture(hipStream_t st, int len, hipGraphExec_t& out, F&& enqueue) {
-        hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
+    static Status capture(int len, hipGraphExec_t& out, F&& enqueue) {
+        struct OwnStream {
+            hipStream_t st = nullptr;
+            ~OwnStream() { pool_release_stream(st); }
+        } own;
+        Status s = pool_stream(&own.st);
+        if (!s) return s;
+        hipError_t e = hipStreamBeginCapture(own.st, hipStreamCaptureModeThreadLocal);
         if (e != hipSuccess) return hip_status(e, "step capture");
-        const Status s = enqueue(len);
+        s = enqueue(len, own.st);
         hipGraph_t gr = nullptr;
-        e = hipStreamEndCapture(st, &gr);
+        e = hipStreamEndCapture(own.st, &gr);
         if (s && e == hipSuccess) e = hipGraphInstantiate(&out, gr, nullptr, nullptr, 0);
         if (gr) (void)hipGraphDestroy(gr);
         if (!s) return s;
