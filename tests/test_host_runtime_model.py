@@ -1,6 +1,7 @@
 """Host code between the caller and the runtime, compiled against a model of
 the runtime's host side (tests/host_check/runtime) and run under sanitizers:
-the replay of captured steps (dg_step_graph.h).  CPU only."""
+the replay of captured steps (dg_step_graph.h) and the copies through pinned
+blocks (dg_hostcopy.cpp).  CPU only."""
 import os
 import subprocess
 
@@ -25,3 +26,9 @@ def run(tmp_path, name, sources, flags, *args):
 @pytest.mark.parametrize("sanitizer", ["address,undefined", "thread"])
 def test_step_graph(tmp_path, sanitizer):
     assert "step graphs ok" in run(tmp_path, "step_graph_check", [], ["-fsanitize=" + sanitizer])
+
+
+@pytest.mark.parametrize("flags,args", [(["-fsanitize=address,undefined"], ()), (["-fsanitize=thread"], ("brief",)),
+                                        (["-DNO_THREADS"], ())])
+def test_host_copies(tmp_path, flags, args):
+    assert "host copies ok" in run(tmp_path, "hostcopy_check", ["dg_hostcopy.cpp"], flags, *args)
