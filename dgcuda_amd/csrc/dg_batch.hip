@@ -17,6 +17,7 @@
 // workgroups of an XCD take the items of its chunk round-robin.
 #include <algorithm>
 #include <cstring>
+#include <mutex>
 #include <numeric>
 
 #include "dg_batch.h"
@@ -877,6 +878,11 @@ class BatchImpl : public Batch {
     std::vector<double> t_end;
     BatchEngine* eng = nullptr;
     bool dirty = true;
+    // Held while steps are put on the engine's stream and while a state is
+    // read, which waits for them and then uses the solve's scratch arrays on
+    // its own stream.
+    std::mutex mu;
+    static constexpr int RUN_CHUNK = 64;  // steps put on the stream at a time
 
     ~BatchImpl() override {
         delete eng;
@@ -908,6 +914,11 @@ class BatchImpl : public Batch {
         return Status::ok();
     }
 
+    Status enqueue(int n, bool use_graph) {
+        const std::lock_guard<std::mutex> lk(mu);
+        return eng->steps(n, use_graph);
+    }
+
     // every control block back in one copy (t, steps and the wave speed the
     // next run starts from)
     Status finish_all() {
@@ -933,7 +944,8 @@ class BatchImpl : public Batch {
         if (!(cfl > 0) || nsteps < 0) return Status::err(DG_ERR_ARG, "invalid arguments");
         Status st = begin_all(false, cfl);
         if (!st) return st;
-        if (!(st = eng->steps(nsteps, use_graph))) return st;
+        for (int n = nsteps; n > 0; n -= RUN_CHUNK)
+            if (!(st = enqueue(std::min(n, RUN_CHUNK), use_graph))) return st;
         return finish_all();
     }
 
@@ -946,13 +958,13 @@ class BatchImpl : public Batch {
         int64_t issued = 0;
         int chunk = 8;
         while (true) {
-            if (!(st = eng->steps(chunk, use_graph))) return st;
+            if (!(st = enqueue(chunk, use_graph))) return st;
             issued += chunk;
             if (!(st = eng->status(h))) return st;
             bool all = true;
             for (int s = 0; s < ns; s++) all = all && (h[3 * s] != 0.0 || !(h[3 * s + 2] < t_end[s]));
             if (all) break;
-            chunk = std::min(chunk * 2, 64);
+            chunk = std::min(chunk * 2, RUN_CHUNK);
         }
         if (steps) *steps = issued;
         return finish_all();
@@ -960,6 +972,7 @@ class BatchImpl : public Batch {
 
     Status get_state(int slot, double* c_ref) override {
         if (slot < 0 || slot >= (int)solvers.size()) return Status::err(DG_ERR_ARG, "slot out of range");
+        const std::lock_guard<std::mutex> lk(mu);
         Status st = eng->sync();
         if (!st) return st;
         return solvers[slot]->get_state(c_ref);

@@ -320,6 +320,10 @@ class SolverT : public Solver {
     StateIx six{};
     bool state_set = false;  // c holds a state (projected, set or stepped)
     double b0 = 0;  // phi_0 at the first volume point (cell mean = c_0 * b0)
+    // Held while steps are put on the stream and while a state is read or set,
+    // whose conversions use acc, ua and ub: a thread may read the state while
+    // another runs steps, and finds it after a whole number of them.
+    std::mutex mu;
     bool geom_fp32 = false;  // FP64 solve with the geometry rounded through FP32 (DG_GEOM_FP32)
 
     ~SolverT() override {
@@ -788,16 +792,26 @@ class SolverT : public Solver {
         return stage(ST_RK4_4, ua, c, c, on, in_step);
     }
 
+    static constexpr int RUN_CHUNK = 64;  // steps put on the stream at a time
     Status enqueue_cfl_steps(int n, int scheme, bool use_graph) {
         const auto enqueue = [&](int k, hipStream_t on) {
             Status st;
             for (int i = 0; i < k && st; i++) st = enqueue_stages(scheme, true, on);
             return st;
         };
-        if (!use_graph) return enqueue(n, stream);
-        if (graph_scheme != scheme) graph.drop();
-        graph_scheme = scheme;
-        return graph.run(stream, n, enqueue);
+        Status st;
+        for (; n > 0 && st; n -= RUN_CHUNK) {
+            const std::lock_guard<std::mutex> lk(mu);
+            const int k = std::min(n, RUN_CHUNK);
+            if (!use_graph) {
+                st = enqueue(k, stream);
+                continue;
+            }
+            if (graph_scheme != scheme) graph.drop();
+            graph_scheme = scheme;
+            st = graph.run(stream, k, enqueue);
+        }
+        return st;
     }
 
     Status begin_run(double t_end, bool has_end, double cfl, hipStream_t on = nullptr) {
@@ -927,6 +941,7 @@ class SolverT : public Solver {
     }
 
     Status set_state(const double* c_ref) override {
+        const std::lock_guard<std::mutex> lk(mu);
         Status st = upload_ref(c_ref, c);
         state_set = (bool)st;
         t = 0;
@@ -935,9 +950,13 @@ class SolverT : public Solver {
         return st;
     }
 
-    Status get_state(double* c_ref) override { return download_ref(c, c_ref); }
+    Status get_state(double* c_ref) override {
+        const std::lock_guard<std::mutex> lk(mu);
+        return download_ref(c, c_ref);
+    }
 
     Status rhs(const double* u_ref, double* k_ref, double dt) override {
+        const std::lock_guard<std::mutex> lk(mu);
         Status st = upload_ref(u_ref, ub);
         if (!st) return st;
         HIPST(launch_set_dt(ctrl, dt, 0, stream));
@@ -986,6 +1005,7 @@ class SolverT : public Solver {
 
     Status rk_step(double dt, int scheme) override {
         if (scheme != DG_RK4 && scheme != DG_RK2) return Status::err(DG_ERR_ARG, "scheme must be DG_RK4 or DG_RK2");
+        const std::lock_guard<std::mutex> lk(mu);
         HIPST(launch_set_dt(ctrl, dt, 1, stream));
         Status st = enqueue_stages(scheme, false);
         if (!st) return st;
@@ -1114,6 +1134,7 @@ class SolverT : public Solver {
     Status time_stage_kernels(int nsteps, double cfl, double* out) override {
         Status st = begin_run(0.0, false, cfl);
         if (!st) return st;
+        const std::lock_guard<std::mutex> lk(mu);
         const int nst = 4 * nsteps;
         std::vector<hipEvent_t> ev(2 * nst + 2);
         for (auto& e : ev) HIPST(hipEventCreate(&e));
@@ -1206,6 +1227,7 @@ class SolverT : public Solver {
     hipStream_t get_stream() const override { return stream; }
 
     Status set_kernel(int kind) override {
+        const std::lock_guard<std::mutex> lk(mu);
         Status st = choose_shape(kind);
         if (!st) return st;
         return push_ctrl();
@@ -1214,6 +1236,7 @@ class SolverT : public Solver {
 
     Status set_max_groups(int n) override {
         if (n < 0 || (n > 0 && n < 8)) return Status::err(DG_ERR_ARG, "max_groups must be 0 or at least 8");
+        const std::lock_guard<std::mutex> lk(mu);
         max_groups = n;
         if (shape.kind != 2) return Status::ok();  // taken up when kind 2 is chosen
         const int req = kernel_req;
