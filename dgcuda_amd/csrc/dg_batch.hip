@@ -463,14 +463,11 @@ class EngineT : public BatchEngine {
     int cap_slots = 0, cap_items = 0;
     int nslots = 0, nitems = 0, dt_grid = 0, cus = 0;
     int max_groups_req = 0;          // set_max_groups (0: no cap)
-    // set_launch_form (-1: the faster by size).  One launch / per class, us per
-    // step, ragged batches: FP32 24 solves of up to 2,000 triangles 45 / 123, 32
-    // of up to 100,000 255 / 340, 64 of up to 200,000 782 / 801; FP64 22,880
-    // triangles in all 97 / 197, 453,104 607 / 632, 1,748,140 2,074 / 1,592 (the
-    // two lines cross near 520,000).
+    // set_launch_form (-1: the faster: FP64 by take_per_class; FP32 in one
+    // launch, us per step against per class: 24 solves of up to 2,000 triangles
+    // 45 / 123, 32 of up to 100,000 255 / 340, 64 of up to 200,000 782 / 801)
     int form = -1;
     bool per_class = false;  // form of the current work list
-    static constexpr int64_t PER_CLASS_MIN_FP64 = 524288;
     std::vector<Launch> launches;    // the batch kernels of a stage, in launch order
     std::vector<int2> raw_items[BATCH_LISTS];  // the work lists in solve order, and
     std::vector<double> raw_cost[BATCH_LISTS]; // each item's estimated cost
@@ -582,12 +579,16 @@ class EngineT : public BatchEngine {
         if (form >= 0) return form == DG_BATCH_PER_CLASS;
         if (sizeof(R) == 4) return false;
         int64_t elems = 0;
+        int present = 0;
         for (Solver* sv : solvers) {
             SlotInfo si;
             sv->slot_info(&si);
-            if (!runs_solo(si)) elems += si.K;
+            if (runs_solo(si)) continue;
+            elems += si.K;
+            present |= class_of(si);
         }
-        return elems >= PER_CLASS_MIN_FP64;
+        return take_per_class(__builtin_popcount(present & BM_LANES), __builtin_popcount(present & BM_TILES), elems,
+                              !launches.empty(), per_class);
     }
 
     // Splits each list into 8 contiguous chunks of equal estimated cost, one

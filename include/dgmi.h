@@ -356,14 +356,17 @@ int dg_batch_info(const dg_batch* b, int* n_solves, int64_t* total_elems, int64_
  * not depend on it.  Test and tuning aid; no counterpart in the reference. */
 int dg_batch_set_max_groups(dg_batch* b, int max_groups);
 /* How a stage of the batch is launched; takes effect at the next run.
- * DG_BATCH_ONE_LAUNCH (the default of FP32
- * and of FP64 below 524,288 triangles): a single persistent launch per
+ * DG_BATCH_ONE_LAUNCH: a single persistent launch per
  * stage carrying every body, at the register budget of the largest;
- * workgroups mix light and heavy items.  DG_BATCH_PER_CLASS (the default of
- * larger FP64 batches): one persistent launch per kernel class present (Euler tiles,
- * advection tiles, Euler lane items, advection lane items), each compiled
+ * workgroups mix light and heavy items.  DG_BATCH_PER_CLASS: one persistent
+ * launch per kernel class present (Euler tiles, advection tiles, Euler lane
+ * items, advection lane items), each compiled
  * with its own bodies only and so holding the wavefronts per SIMD those
  * bodies allow (the FP64 one-launch kernel holds one wavefront per SIMD).
+ * Until one is set: FP32 in one launch; FP64 per class where one class is
+ * present, from 65,536 triangles on where two are and one of them is of
+ * tiles, else from 524,288 on (a batch that has run keeps its form within an
+ * eighth of these).
  * Results are the same bit for bit.  No counterpart in the reference (its
  * solves run one at a time). */
 enum { DG_BATCH_ONE_LAUNCH = 0, DG_BATCH_PER_CLASS = 1 };
