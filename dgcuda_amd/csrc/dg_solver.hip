@@ -978,13 +978,18 @@ class SolverT : public Solver {
         if (cur != device) return Status::err(DG_ERR_STATE, "the solver's device is not the current device");
         char* base = static_cast<char*>(noalloc_scratch(device));
         if (!base) return Status::err(DG_ERR_STATE, "the device's scratch is not set up");
-        // (the limit counts 16 mode slots in the FP64 tile layout, as stated in the interface)
-        const size_t slots = six.tiled == LAYOUT_TILE64 ? 16 : six.slots();
+        // The limit counts the state arrays' mode slots, 16 in the FP64 tile
+        // layout, as stated in the interface.  Up to p = 2 the automatic
+        // choice takes tiles or lanes by their time: it counts the lane
+        // layout's slots whichever it took, so that the choice does not decide
+        // which solves are refused.
+        const size_t slots = kernel_req == 0 && p <= 2 ? NP : six.tiled == LAYOUT_TILE64 ? 16 : six.slots();
         const size_t one = ((size_t)N * slots * Kp * sizeof(R) + 255) / 256 * 256;
         if (2 * one > NOALLOC_SCRATCH_BYTES)
             return Status::err(DG_ERR_BUDGET, "this solve needs " + std::to_string(2 * one) +
                                                   " bytes of scratch; the allocation-free entry point has " +
                                                   std::to_string(NOALLOC_SCRATCH_BYTES));
+        const size_t real = ((size_t)six.elems() * sizeof(R) + 255) / 256 * 256;
         hipStream_t sx = on ? on : stream;
         // one launch on the caller's arrays; the scratch only where they
         // overlap (the kernel reads neighbours while others write) or the
@@ -992,8 +997,12 @@ class SolverT : public Solver {
         const size_t n = (size_t)N * NP * K;
         const bool apart = u_dev + n <= k_dev || k_dev + n <= u_dev;
         if (apart && ref_rhs_supported(N, p, shape.kind)) return stage_ref(u_dev, k_dev, dt, sx);
+        if (2 * real > NOALLOC_SCRATCH_BYTES)
+            return Status::err(DG_ERR_BUDGET, "overlapping arrays of this solve need " + std::to_string(2 * real) +
+                                                  " bytes of scratch; the allocation-free entry point has " +
+                                                  std::to_string(NOALLOC_SCRATCH_BYTES));
         R* in = reinterpret_cast<R*>(base);
-        R* out = reinterpret_cast<R*>(base + one);
+        R* out = reinterpret_cast<R*>(base + real);
         HIPST(launch_ref_to_state<R>(RefRows{const_cast<double*>(u_dev), nullptr, N * NP}, in, perm_d, six, K, sx));
         HIPST(launch_set_dt(ctrl, dt, 0, sx));
         lam_valid = false;  // set_dt cleared the accumulated wave speed

@@ -254,7 +254,8 @@ int dg_rhs(dg_solver* s, const double* u_ref, double* k_ref, double t, double dt
  * p = 4, 5 on the lane kernel, the state goes through a fixed 64 MiB scratch
  * array per device (two arrays of the solve's state layout: up to about
  * 65,000 triangles for FP64 Euler at p = 4, 131,000 for FP32); a solve too
- * large for the scratch returns DG_ERR_BUDGET before any work in every case.
+ * large for the scratch returns DG_ERR_BUDGET before any work in every case
+ * (up to p = 2 an automatically chosen kernel counts n_p slots per variable).
  * No allocation and no wait: the work is enqueued on `stream` (a
  * hipStream_t; NULL = the solver's own stream) and the caller synchronises.
  * Calls that use the scratch share it with every other on the device, so
