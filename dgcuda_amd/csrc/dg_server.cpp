@@ -28,33 +28,9 @@
 
 #include "dg_batch.h"
 #include "dg_server.h"
+#include "dg_solve_bytes.h"
 
 namespace dgmi {
-
-// A request's size against the budget at submit, as stated in the interface:
-// the FP64 tile layout counted with 16 mode slots.
-static int64_t estimate_bytes(int K, int N, int p, int precision) {
-    const int64_t Kp = (K + 63) / 64 * 64;
-    const int64_t s = precision == DG_FP64 ? 8 : 4;
-    // p <= 4 reserves the matrix-core tile layout
-    const bool tl = p >= 1 && p <= 4;
-    const int64_t np = !tl ? n_modes(p) : precision == DG_FP32 ? 4 * tile_groups(n_modes(p)) : 16;
-    const int64_t ntiles = (K + 63) / 64;
-    // matrix-core tiles (p >= 3 in a batch): packed geometry, 16 values per element
-    const int64_t packed = p >= 3 ? 16 * s : 0;
-    return Kp * (4 * N * np * s + 14 * s + 3 * 4 + 6 * 8 + 8 + 8 + 3 * 2 + packed) + ntiles * 64 * 4 + 4096;
-}
-
-// Device bytes a resident solve holds (the solver's allocations): the state
-// arrays with the slots they have, and the packed geometry of the Euler lane
-// kernel (p <= 2 in a batch) where a tile's is not there.
-static int64_t held_bytes(int K, int N, int p, int precision) {
-    const int64_t Kp = (K + 63) / 64 * 64;
-    int64_t b = estimate_bytes(K, N, p, precision);
-    if (precision == DG_FP64) b -= Kp * 4 * N * (16 - tile64_slots(n_modes(p))) * 8;
-    if (N == 4 && p <= 2) b += Kp * 16 * (precision == DG_FP64 ? 8 : 4);
-    return b;
-}
 
 class ServerImpl : public Server {
    public:
@@ -125,7 +101,7 @@ class ServerImpl : public Server {
             return Status::err(DG_ERR_ARG, "invalid request");
         Status st = check_problem(req.prob, req.p, cfg.precision);
         if (!st) return st;
-        const int64_t need = estimate_bytes(2 * req.nx * req.ny, req.prob.physics, req.p, cfg.precision);
+        const int64_t need = estimate_bytes(2 * req.nx * req.ny, req.prob.physics, req.p, cfg.precision == DG_FP64);
         if (need > cfg.hbm_budget) return Status::err(DG_ERR_BUDGET, "request exceeds the HBM budget on its own");
         std::lock_guard<std::mutex> lk(mu);
         if (!fatal.empty()) return Status::err(DG_ERR_STATE, "server stopped: " + fatal);
@@ -196,9 +172,10 @@ class ServerImpl : public Server {
                 continue;
             }
             const int K = 2 * front.req.nx * front.req.ny;
-            // (never more than the budget: a request accepted at submit fits alone)
+            // (never more than the budget: a request accepted at submit runs,
+            // alone if it holds more than was estimated)
             const int64_t need =
-                std::min(cfg.hbm_budget, held_bytes(K, front.req.prob.physics, front.req.p, cfg.precision));
+                std::min(cfg.hbm_budget, held_bytes(K, front.req.prob.physics, front.req.p, cfg.precision == DG_FP64));
             if (slots_held >= cfg.max_slots || bytes_held + need > cfg.hbm_budget) {
                 cv.wait(lk);
                 continue;

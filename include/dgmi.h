@@ -384,7 +384,11 @@ int dg_batch_launch_info(const dg_batch* b, int* out4);
 typedef struct {
     int precision;          /* DG_FP32 or DG_FP64 */
     int max_slots;          /* solves resident at once */
-    int64_t hbm_budget;     /* bytes of device memory the resident solves may hold */
+    int64_t hbm_budget;     /* bytes of device memory the resident solves may hold.  A request is
+                               refused when its estimate alone exceeds it; FP32 Euler at p <= 2
+                               holds 64 bytes a triangle and every solve a few KB more than estimated,
+                               and one that fits by its estimate only runs by itself, over the
+                               budget by that much */
     int steps_per_round;    /* batch steps between admissions / completions */
     double cfl;
     int use_graph;
