@@ -48,6 +48,21 @@ void pool_free(void* p);
 Status pool_stream(hipStream_t* s);
 void pool_release_stream(hipStream_t s);
 
+// Device `dev` as the current one for a scope (a caller may have another one
+// current).
+struct OnDevice {
+    int prev = -1;
+    explicit OnDevice(int dev) {
+        if (hipGetDevice(&prev) == hipSuccess && prev != dev)
+            (void)hipSetDevice(dev);
+        else
+            prev = -1;
+    }
+    ~OnDevice() {
+        if (prev >= 0) (void)hipSetDevice(prev);
+    }
+};
+
 PhysP make_phys(const dg_problem_desc& d);
 IcP make_ic(const dg_problem_desc& d, double Lx, double Ly);
 Status check_problem(const dg_problem_desc& d, int p, int precision);

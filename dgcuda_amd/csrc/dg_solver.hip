@@ -580,7 +580,7 @@ class SolverT : public Solver {
             Status st = build_mfma_tiles(s.tile_elems);
             if (!st) return st;
             if (kind == 2) {
-                // persistent: as many workgroups as fit on the device at once
+                // persistent: as many workgroups as fit on the device at once (stage 2)
                 const int res = mfma_resident_groups(N, p, mx.hcap, (int)sizeof(R), has_boundary);
                 if (res >= 8) s.grid = std::min(s.grid, res / 8 * 8);
                 if (max_groups >= 8) s.grid = std::min(s.grid, max_groups / 8 * 8);
@@ -864,21 +864,6 @@ class SolverT : public Solver {
         if (st) s.rows = RefRows{(double*)s.own, nullptr, rows};
         return st;
     }
-
-    // The solve's device as the current one while the state is converted (a
-    // state may be read or set with another device current).
-    struct OnDevice {
-        int prev = -1;
-        explicit OnDevice(int dev) {
-            if (hipGetDevice(&prev) == hipSuccess && prev != dev)
-                (void)hipSetDevice(dev);
-            else
-                prev = -1;
-        }
-        ~OnDevice() {
-            if (prev >= 0) (void)hipSetDevice(prev);
-        }
-    };
 
     // A host array that fits one pinned block is read or written there by the
     // conversion kernel itself, in one launch and one wait.  Through a copy and

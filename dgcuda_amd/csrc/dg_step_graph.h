@@ -34,7 +34,7 @@ class StepGraph {
             hipGraphExec_t& g = long_graph ? many : one;
             const int len = long_graph ? MANY : 1;
             if (!g) {
-                Status s = capture(len, g, enqueue);
+                Status s = capture(st, len, g, enqueue);
                 if (!s) return s;
             }
             hipError_t e = hipGraphLaunch(g, st);
@@ -49,18 +49,23 @@ class StepGraph {
     hipGraphExec_t one = nullptr, many = nullptr;
     int64_t taken = 0;
 
-    // On a stream of its own: the solve's stream may be in use meanwhile (a
-    // thread reading the state during a run; the long graph is captured in
-    // the middle of one), and a wait for a stream that is being captured fails.
+    // On a stream of its own, of the device of `run`: the solve's stream may be
+    // in use meanwhile (a thread reading the state during a run; the long graph
+    // is captured in the middle of one), and a wait for a stream that is being
+    // captured fails.
     template <typename F>
-    static Status capture(int len, hipGraphExec_t& out, F&& enqueue) {
+    static Status capture(hipStream_t run, int len, hipGraphExec_t& out, F&& enqueue) {
+        hipDevice_t dev = 0;
+        hipError_t e = hipStreamGetDevice(run, &dev);
+        if (e != hipSuccess) return hip_status(e, "step capture");
+        const OnDevice here(dev);
         struct OwnStream {
             hipStream_t st = nullptr;
             ~OwnStream() { pool_release_stream(st); }
         } own;
         Status s = pool_stream(&own.st);
         if (!s) return s;
-        hipError_t e = hipStreamBeginCapture(own.st, hipStreamCaptureModeThreadLocal);
+        e = hipStreamBeginCapture(own.st, hipStreamCaptureModeThreadLocal);
         if (e != hipSuccess) return hip_status(e, "step capture");
         s = enqueue(len, own.st);
         hipGraph_t gr = nullptr;

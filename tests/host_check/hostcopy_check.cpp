@@ -79,7 +79,7 @@ int main(int argc, char**) {
         });
     for (std::thread& t : th) t.join();
     CHECK(model::host_blocks <= IDLE_BLOCKS && model::events == 0);
-    CHECK(stream_pool().idle.size() == stream_pool().all.size());
+    CHECK(stream_pool().idle() == stream_pool().all.size());
     if (!brief)
         for (size_t n : {8 * (size_t)63, 2 * MB + 8, 8 * MB + 8}) {
             int failed = 0;
@@ -90,7 +90,7 @@ int main(int argc, char**) {
                 const bool reached = model::calls > at;
                 model::fail_at = -1;
                 CHECK(model::host_blocks <= IDLE_BLOCKS && model::events == 0);
-                CHECK(stream_pool().idle.size() == stream_pool().all.size());
+                CHECK(stream_pool().idle() == stream_pool().all.size());
                 CHECK(trip(n, 9, true));  // whole again
                 if (!reached) break;
             }

@@ -7,7 +7,8 @@ namespace dgmi {
 struct StreamPool {
     std::mutex mu;
     std::vector<std::unique_ptr<model::Stream>> all;
-    std::vector<hipStream_t> idle;
+    std::vector<hipStream_t> idle_of[2];  // by device
+    size_t idle() const { return idle_of[0].size() + idle_of[1].size(); }
 };
 inline StreamPool& stream_pool() {
     static StreamPool p;
@@ -20,19 +21,21 @@ Status pool_stream(hipStream_t* s) {
     if (model::fails()) return Status::err(DG_ERR_HIP, "stream");
     StreamPool& P = stream_pool();
     std::lock_guard<std::mutex> lk(P.mu);
-    if (P.idle.empty()) {
+    auto& idle = P.idle_of[model::device];
+    if (idle.empty()) {
         P.all.emplace_back(new model::Stream());
-        P.idle.push_back(P.all.back().get());
+        P.all.back()->device = model::device;
+        idle.push_back(P.all.back().get());
     }
-    *s = P.idle.back();
-    P.idle.pop_back();
+    *s = idle.back();
+    idle.pop_back();
     return Status::ok();
 }
 void pool_release_stream(hipStream_t s) {
     if (!s) return;
     StreamPool& P = stream_pool();
     std::lock_guard<std::mutex> lk(P.mu);
-    P.idle.push_back(s);
+    P.idle_of[model::device].push_back(s);
 }
 
 }  // namespace dgmi

@@ -30,6 +30,7 @@ struct Stream {
     bool busy = false, stop = false;
     std::atomic<bool> capturing{false};
     int captured = 0;  // steps put on it while it is captured
+    int device = 0;
     std::thread th;
     Stream() : th([this] { loop(); }) {}
     ~Stream() {
@@ -82,8 +83,21 @@ inline bool fails() { return calls.fetch_add(1) == fail_at.load(); }
 typedef std::shared_ptr<model::Event>* hipEvent_t;
 inline model::Stream* S(hipStream_t s) { return static_cast<model::Stream*>(s); }
 
-inline hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
-inline hipError_t hipSetDevice(int) { return model::fails() ? hipErrorInvalidValue : hipSuccess; }
+typedef int hipDevice_t;
+namespace model {
+inline thread_local int device = 0;
+}
+inline hipError_t hipGetDevice(int* d) { *d = model::device; return hipSuccess; }
+inline hipError_t hipSetDevice(int d) {
+    if (model::fails()) return hipErrorInvalidValue;
+    model::device = d;
+    return hipSuccess;
+}
+inline hipError_t hipStreamGetDevice(hipStream_t st, hipDevice_t* d) {
+    if (model::fails()) return hipErrorInvalidValue;
+    *d = S(st)->device;
+    return hipSuccess;
+}
 inline hipError_t hipHostMalloc(void** p, size_t n, int) {
     if (model::fails()) return hipErrorOutOfMemory;
     *p = std::malloc(n);

@@ -21,7 +21,7 @@ int main() {
         }
     });
     const auto enqueue = [&](int k, hipStream_t on) {
-        CHECK(S(on)->capturing);
+        CHECK(S(on)->capturing && S(on)->device == S(run)->device);
         S(on)->captured += k;
         return Status::ok();
     };
@@ -57,11 +57,19 @@ int main() {
         CHECK(!g.run(run, 4, [](int, hipStream_t) { return Status::err(DG_ERR_ARG, "no"); }));
         CHECK(model::graphs == 0 && model::execs == 0);
     }
+    {
+        StepGraph g;  // with another device current
+        model::device = 1;
+        CHECK(g.run(run, 40, enqueue) && model::device == 1);
+        model::device = 0;
+    }
     over = true;
     waiter.join();
     CHECK(bad_waits == 0);
     pool_release_stream(run);
-    CHECK(stream_pool().idle.size() == stream_pool().all.size());
+    CHECK(stream_pool().idle() == stream_pool().all.size());
+    for (int d = 0; d < 2; d++)
+        for (hipStream_t st : stream_pool().idle_of[d]) CHECK(S(st)->device == d);
     std::printf("step graphs ok\n");
     return 0;
 }
