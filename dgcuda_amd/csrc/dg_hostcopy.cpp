@@ -23,7 +23,7 @@ constexpr size_t COPY_BLOCK = PINNED_BLOCK_BYTES;
 constexpr size_t COPY_MIN_PART = size_t(4) << 20;
 constexpr int COPY_MAX_THREADS = 4;
 constexpr size_t COPY_SMALL = size_t(64) << 10;
-constexpr size_t COPY_IDLE_BLOCKS = 2 * COPY_MAX_THREADS;  // kept between calls, of all threads together
+constexpr size_t COPY_IDLE_BLOCKS = 16;  // kept between calls, of all threads together (a server's set-up threads audit at a time)
 
 // pinned blocks, shared by every thread of the process; at most
 // COPY_IDLE_BLOCKS stay between calls, the others are freed

@@ -23,7 +23,7 @@ using namespace dgmi;
 namespace {
 
 constexpr size_t MB = size_t(1) << 20;
-constexpr int IDLE_BLOCKS = 8;
+constexpr int IDLE_BLOCKS = 16;
 
 std::vector<char> bytes_of(size_t n, unsigned seed) {
     std::vector<char> v(n);
@@ -67,7 +67,7 @@ int main(int argc, char**) {
         });
     for (std::thread& t : th) t.join();
     th.clear();
-    for (unsigned i = 0; i < 12; i++)  // more blocks out at a time than stay idle
+    for (unsigned i = 0; i < 24; i++)  // more blocks out at a time than stay idle
         th.emplace_back([&, i] {
             for (int k = 0; k < 20; k++) {
                 PinnedBlock b;
