@@ -323,11 +323,12 @@ __device__ __forceinline__ void batch_tile_items(const SlotDesc<R>* __restrict__
 }
 
 // Workgroups per CU each kernel's registers are held to, by mask.  One
-// launch: FP32 2 (3 spills 76-220 B per lane and measured no faster); FP64
-// 1, which lets the compiler keep its spills in the accumulation registers
-// (AGPRs) of the single wavefront per SIMD (2 spill about 1 KB per lane to
-// memory).  The others: the settings measured fastest on the ragged
-// 64-solve batch among 2-6.
+// launch: FP32 2 (157-181 VGPRs; held to 3 stages 2 and 4 spill 8 and 6
+// registers: not timed since the bodies took 213-252 VGPRs, when 3 spilled
+// 76-220 B a lane and was no faster); FP64 1, whose single wavefront per SIMD
+// has the accumulation registers (AGPRs) besides (62-80 of them used).  The
+// others: the settings measured fastest on the ragged 64-solve batch among
+// 2-6.
 template <typename R, int MASK>
 constexpr int batch_min_groups() {
     const bool f32 = sizeof(R) == 4;
@@ -463,9 +464,9 @@ class EngineT : public BatchEngine {
     int cap_slots = 0, cap_items = 0;
     int nslots = 0, nitems = 0, dt_grid = 0, cus = 0;
     int max_groups_req = 0;          // set_max_groups (0: no cap)
-    // set_launch_form (-1: the faster: FP64 by take_per_class; FP32 in one
-    // launch, us per step against per class: 24 solves of up to 2,000 triangles
-    // 45 / 123, 32 of up to 100,000 255 / 340, 64 of up to 200,000 782 / 801)
+    // set_launch_form (-1: FP64 by take_per_class; FP32 in one launch, us per
+    // step against per class: 24 solves of up to 2,000 triangles 45 / 113, 32 of
+    // up to 100,000 255 / 318; 64 of up to 200,000 778 / 749, the other way)
     int form = -1;
     bool per_class = false;  // form of the current work list
     std::vector<Launch> launches;    // the batch kernels of a stage, in launch order

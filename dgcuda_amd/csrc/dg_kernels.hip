@@ -50,7 +50,9 @@ __global__ void __launch_bounds__(128, (N == 1 && P == 5 && sizeof(R) == 4 ? 2 :
 // Euler, p <= 3: the lane body on the vector layout, one instance per stage
 // kind (the RK operands' loads and the update are fixed at compile time)
 // Wavefronts per SIMD the registers are held to: the most that fit without
-// spills (FP32 p = 1, 2: 5 and 4; FP64 p = 1, 2: 2).
+// spills in the loops (FP32 p = 1, 2: 5 and 4; FP64 p = 1, 2: 2).  FP32 p = 2
+// spills 3 registers in the first stage, 17-26 with boundary sides, and 16 on
+// the caller's arrays.
 template <int P, typename R>
 constexpr int lane_minw() {
     if (sizeof(R) == 4) return P <= 1 ? 5 : P == 2 ? 4 : 2;

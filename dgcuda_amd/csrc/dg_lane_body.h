@@ -8,14 +8,15 @@
 // element's four variables per access (FP32 one 16-byte access, FP64 two),
 // the geometry comes in packed records, the neighbours' modes are requested
 // ahead of the arithmetic that covers them, and the neighbour's table rows
-// are read from LDS instead of selected: 22 and 37 loads, 910 and 1,755
-// vector instructions instead of 1,163 and 2,608.  The sums of a face are
+// are read from LDS instead of selected: 19.5-20.5 and 34-36 loads by stage,
+// 889-1,100 and 2,067-2,339 vector instructions (counters, the step's dt and
+// wave speeds included) instead of 1,163 and 2,608.  The sums of a face are
 // pinned before the next begins (LANE_KEEP); moved down by the compiler they
 // kept every face's values live (FP32 p = 2 168 registers and spills, pinned
 // 128; FP64 p = 2 512, pinned 250).
-// Per stage of a step, mode-major -> this layout: FP32 p = 1 at 500,000
-// triangles 32.3 -> 22.7 us (111 MB, 4.7 TB/s), p = 2 at 524,288 64.9 -> 40.0
-// (187 MB, 4.7 TB/s) and at 32,768 17.0 -> 9.9; FP64 p = 2 at 131,072
+// Per stage of a step, mode-major -> this layout: FP32 p = 1 at 524,288
+// triangles 40.2 -> 24.1 us (111 MB, 4.6 TB/s), p = 2 71.6 -> 46.1 (187 MB,
+// 4.1 TB/s; by kernel trace) and at 32,768 17.0 -> 9.9; FP64 p = 2 at 131,072
 // 55.2 -> 27.2, at 32,768 24.1 -> 14.3.
 //
 // A face is evaluated in the element's own orientation (point j of the face

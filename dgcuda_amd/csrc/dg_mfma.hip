@@ -192,7 +192,11 @@ template hipError_t launch_mfma_pack<float>(const float*, const float*, const in
 template hipError_t launch_mfma_pack<double>(const double*, const double*, const int*, const SideTask*, int, int, int,
                                              void*, void*, hipStream_t);
 
-// workgroups of the matrix-core kernel that fit on the device at once
+// Workgroups of the matrix-core kernel that fit on the device at once, by its
+// second RK4 stage, whose registers are the most of a step's.  The others take
+// the same grid: stages 1 and 3 in FP32 could hold four workgroups per CU
+// instead of three, and the instance on the caller's arrays holds two, so a
+// third of its persistent workgroups start when others have ended.
 template <typename R, bool BND>
 static const void* stage2_kernel(int N, int p) {
     if (N == 1 && p == 4) return reinterpret_cast<const void*>(&k_stage_mfma<1, 4, ST_RK4_2, R, BND>);
