@@ -974,7 +974,6 @@ class SolverT : public Solver {
             return Status::err(DG_ERR_BUDGET, "this solve needs " + std::to_string(2 * one) +
                                                   " bytes of scratch; the allocation-free entry point has " +
                                                   std::to_string(NOALLOC_SCRATCH_BYTES));
-        const size_t real = ((size_t)six.elems() * sizeof(R) + 255) / 256 * 256;
         hipStream_t sx = on ? on : stream;
         // one launch on the caller's arrays; the scratch only where they
         // overlap (the kernel reads neighbours while others write) or the
@@ -982,6 +981,7 @@ class SolverT : public Solver {
         const size_t n = (size_t)N * NP * K;
         const bool apart = u_dev + n <= k_dev || k_dev + n <= u_dev;
         if (apart && ref_rhs_supported(N, p, shape.kind)) return stage_ref(u_dev, k_dev, dt, sx);
+        const size_t real = ((size_t)six.elems() * sizeof(R) + 255) / 256 * 256;
         if (2 * real > NOALLOC_SCRATCH_BYTES)
             return Status::err(DG_ERR_BUDGET, "overlapping arrays of this solve need " + std::to_string(2 * real) +
                                                   " bytes of scratch; the allocation-free entry point has " +
