@@ -238,7 +238,9 @@ void dg_solver_destroy(dg_solver* s);
 int dg_solver_info(const dg_solver* s, int* sizes, double* min_r);
 /* L2 projection of the problem's initial condition (init_conditions); resets t and steps */
 int dg_project_ic(dg_solver* s);
-/* state I/O in the reference layout, FP64 host buffers of N*n_p*num_elem; set resets t and steps */
+/* state I/O in the reference layout, FP64 host buffers of N*n_p*num_elem; set resets t and steps.
+ * dg_get_state may be called while another thread runs steps of the same solve (or of its
+ * batch, dg_batch_get_state): it returns the state after a whole number of steps. */
 int dg_set_state(dg_solver* s, const double* c_ref);
 int dg_get_state(dg_solver* s, double* c_ref);
 /* k = dt * M^-1 R(u) exactly as eval_surface + eval_volume + eval_rhs compute it
